@@ -37,6 +37,11 @@ struct Family {
     // level tables: for M = 2 .. 2^LT, w_M^q (q < M/2) at offset M/2 - 1,
     // in Montgomery form (w 2^32 mod p); lvi holds the inverse roots' powers
     u32 *lv, *lvi;
+    // matrix-core transforms (ntt_mx.h; null when K < 4): the byte matrices,
+    // and for M = 32 .. 2^LT the twiddles w_M^(k v) (k < 16, v < S = M / 16)
+    // at M + k S + v, with their inverses
+    void *mx_mat;
+    u32 *mx_tf, *mx_ti;
 };
 
 // Four-step outer twiddles w_n^e for one transform size n = 2^k
@@ -165,6 +170,10 @@ hipError_t launch_mul_lds(int logn, const u32 *F, const u32 *G, u32 *H, const Mu
 hipError_t launch_mul_lds_one(int logn, const u32 *F, const u32 *G, u32 *H,
                               const MulDesc *d_descs, int ndesc, const MulDesc &one,
                               const Family *fam, hipStream_t s);
+
+// product d at d times the strides sd.f / sd.g / sd.h, lengths sd.lf / lg / lh
+hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, const MulDesc &sd,
+                                  int count, const Family *fam, hipStream_t s);
 
 // In-place natural-order forward DFT of m rows of 2^k words (k <= 13),
 // outputs multiplied by the residue `scale` (1: none).

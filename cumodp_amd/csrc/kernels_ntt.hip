@@ -3,8 +3,6 @@
 // Replaces the reference's one-stage-per-launch radix-2 Stockham passes
 // (src/stockham.cu:75-397, src/list_stockham.cu:108-576, src/fft_aux.cu:70-322)
 // with:
-//   * k_mul_lds   -- a whole multiply (forward F and G, pointwise product,
-//                    inverse, scaling) inside one workgroup for 2^k <= 2^13;
 //   * k_col_fwd / k_row_mul / k_col_inv -- a three-kernel four-step multiply
 //                    for larger sizes: column transforms of both operands with
 //                    the zero-padding gather fused; row pass with the outer
@@ -25,113 +23,6 @@ namespace cm {
 CM_DEV int xcd_remap(int b, int nb) {
     if (nb & 7) return b;
     return (b & 7) * (nb >> 3) + (b >> 3);
-}
-
-// ---------------------------------------------------------------------------
-// whole multiply in one workgroup (C products per workgroup)
-// ---------------------------------------------------------------------------
-// DESC: descriptors from `descs` (or the by-value `one` when descs is null);
-// otherwise product d reads F + d * one.f, G + d * one.g (one.lf / one.lg
-// words) and writes H + d * one.h (one.lh words).  H may alias F.
-// Held to 128 VGPRs so that the 2^12- and 2^13-point tiles keep as many
-// workgroups per CU as their LDS allows.
-template <int LOGL, int C, bool DESC, class MD>
-__global__ __launch_bounds__((Tile<LOGL, C, false>::T))
-__attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_lds(
-    const u32 *F, const u32 *__restrict__ G, u32 *H, const MulDesc *__restrict__ descs,
-    int ndesc, MulDesc one, const u32 *__restrict__ lv, const u32 *__restrict__ lvi, MD md,
-    u32 sc) {
-    using TL = Tile<LOGL, C, false>;
-    __shared__ u32 lds[2 * TL::LDS_WORDS];
-    u32 *A = lds, *B = lds + TL::LDS_WORDS;
-    const int L = TL::L;
-
-    if constexpr (Round<TL, 0>::R == 4 && Round<TL, 0>::GPT == 1 && TL::NR >= 2) {
-        // thread t's product is c = t >> (LOGL-4); it loads its group of the
-        // first forward and the last inverse round (elements gi + r 2^(LOGL-4)),
-        // which run on the registers
-        constexpr int S = LOGL - 4;
-        constexpr int PER = TL::WORDS / TL::T;
-        const int c = threadIdx.x >> S, gi = threadIdx.x & ((1 << S) - 1);
-        const int d = blockIdx.x * C + c;
-        MulDesc my{};
-        if (d < ndesc) {
-            if (DESC) {
-                my = descs ? descs[d] : one;
-            } else {
-                // product d at d times the strides one.f / one.g / one.h
-                my = one;
-                my.f = (int64_t)d * one.f; my.g = (int64_t)d * one.g; my.h = (int64_t)d * one.h;
-            }
-        }
-        u32 fa[PER], ga[PER];
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int i = gi + (r << S);
-            fa[r] = i < my.lf ? F[my.f + i] : 0u;
-            ga[r] = i < my.lg ? G[my.g + i] : 0u;
-        }
-        cm_row_multiply<TL>(A, B, fa, ga, lv, lvi, md, sc);
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int i = gi + (r << S);
-            if (i < my.lh) H[my.h + i] = cm_canon(fa[r], md);
-        }
-        // words beyond the transform size (lh > L) are zero
-        for (int i = L + gi; i < my.lh; i += 1 << S) H[my.h + i] = 0u;
-        return;
-    } else {
-
-        int64_t off_f[C], off_g[C], off_h[C];
-        int lf[C], lg[C], lh[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int d = blockIdx.x * C + c;
-            if (DESC) {
-                if (d < ndesc) {
-                    const MulDesc dd = descs ? descs[d] : one;
-                    off_f[c] = dd.f; off_g[c] = dd.g; off_h[c] = dd.h;
-                    lf[c] = dd.lf; lg[c] = dd.lg; lh[c] = dd.lh;
-                } else {
-                    off_f[c] = off_g[c] = off_h[c] = 0;
-                    lf[c] = lg[c] = lh[c] = 0;
-                }
-            } else {
-                // product d at d times the strides one.f / one.g / one.h, with
-                // the lengths one.lf / one.lg / one.lh
-                off_f[c] = (int64_t)d * one.f; off_g[c] = (int64_t)d * one.g;
-                off_h[c] = (int64_t)d * one.h;
-                lf[c] = d < ndesc ? one.lf : 0; lg[c] = d < ndesc ? one.lg : 0;
-                lh[c] = d < ndesc ? one.lh : 0;
-            }
-        }
-        // all loads of a thread are issued before the first LDS store
-        constexpr int PER = TL::WORDS / TL::T;
-        u32 fa[PER], ga[PER];
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int idx = threadIdx.x + r * TL::T, c = idx >> LOGL, i = idx & (L - 1);
-            fa[r] = i < lf[c] ? F[off_f[c] + i] : 0u;
-            ga[r] = i < lg[c] ? G[off_g[c] + i] : 0u;
-        }
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int idx = threadIdx.x + r * TL::T, c = idx >> LOGL, i = idx & (L - 1);
-            A[TL::addr(c, i)] = fa[r];
-            B[TL::addr(c, i)] = ga[r];
-        }
-        __syncthreads();
-        cm_tile_multiply<TL>(A, B, lv, lvi, md, sc);
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int idx = threadIdx.x + r * TL::T, c = idx >> LOGL, i = idx & (L - 1);
-            if (i < lh[c]) H[off_h[c] + i] = cm_canon(A[TL::addr(c, i)], md);
-        }
-        // words beyond the transform size (lh > L) are zero
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            for (int i = L + threadIdx.x; i < lh[c]; i += TL::T) H[off_h[c] + i] = 0u;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -618,45 +509,6 @@ u32 mul_scale(int logn, u32 p) {
 template <int LOGL>
 static constexpr int rows_per_wg() { return LOGL >= 10 ? 1 : (1 << (LOGL >= 10 ? 0 : 10 - LOGL)); }
 
-// Multiplies inside one workgroup keep their values in [0, 2p) between
-// butterflies when p < 2^30 (ModLazy) and store canonical residues.
-template <int LOGL, bool DESC>
-static hipError_t mul_lds_t(const u32 *F, const u32 *G, u32 *H, const MulDesc *descs, int ndesc,
-                            const MulDesc &one, const Family *fam, hipStream_t s) {
-    constexpr int C = rows_per_wg<LOGL>();
-    using TL = Tile<LOGL, C, false>;
-    const int nb = (ndesc + C - 1) / C;
-    ProfScope ps(kProfMulLds, s);
-    if (fam->p < (1u << 30))
-        hipLaunchKernelGGL((k_mul_lds<LOGL, C, DESC, ModLazy>), dim3(nb), dim3(TL::T), 0, s, F, G,
-                           H, descs, ndesc, one, fam->lv, fam->lvi, ModLazy{fam->p, fam->np},
-                           mul_scale(LOGL, fam->p));
-    else
-        hipLaunchKernelGGL((k_mul_lds<LOGL, C, DESC, Mod>), dim3(nb), dim3(TL::T), 0, s, F, G, H,
-                           descs, ndesc, one, fam->lv, fam->lvi, mod_of(fam),
-                           mul_scale(LOGL, fam->p));
-    return hipGetLastError();
-}
-
-hipError_t launch_mul_lds(int logn, const u32 *F, const u32 *G, u32 *H, const MulDesc *d_descs,
-                          int ndesc, const Family *fam, hipStream_t s) {
-    MulDesc none{};
-    return launch_mul_lds_one(logn, F, G, H, d_descs, ndesc, none, fam, s);
-}
-
-hipError_t launch_mul_lds_one(int logn, const u32 *F, const u32 *G, u32 *H,
-                              const MulDesc *d_descs, int ndesc, const MulDesc &one,
-                              const Family *fam, hipStream_t s) {
-    if (ndesc <= 0) return hipSuccess;
-    switch (logn) {
-#define CM_CASE(K) case K: return mul_lds_t<K, true>(F, G, H, d_descs, ndesc, one, fam, s);
-        CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8) CM_CASE(9) CM_CASE(10)
-        CM_CASE(11) CM_CASE(12) CM_CASE(13) CM_CASE(14)
-#undef CM_CASE
-    }
-    return hipErrorInvalidValue;
-}
-
 template <int LOGL>
 static hipError_t ntt_lds_t(u32 *X, int64_t m, const u32 *lv, u32 sc, const Family *fam,
                             hipStream_t s) {
@@ -922,19 +774,6 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
     return mul_four_step_t(o->k1, o->k2, io, o, fam, mod_of(fam), s);
 }
 
-template <int LOGL>
-static hipError_t rows_mul_t(u32 *F, u32 *G, int rows, const Family *fam, hipStream_t s) {
-    const int L = 1 << LOGL;
-    const MulDesc rows_desc{L, L, L, L, L, L, LOGL};
-    return mul_lds_t<LOGL, false>(F, G, F, nullptr, rows, rows_desc, fam, s);
-}
-
-template <int LOGL>
-static hipError_t mul_strided_t(const u32 *F, const u32 *G, u32 *H, const MulDesc &sd, int count,
-                                const Family *fam, hipStream_t s) {
-    return mul_lds_t<LOGL, false>(F, G, H, nullptr, count, sd, fam, s);
-}
-
 hipError_t launch_mul_strided(int logn, const u32 *F, int64_t fs, int lf, const u32 *G,
                               int64_t gs, int lg, u32 *H, int64_t hs, int lh, int count,
                               const Family *fam, hipStream_t s) {
@@ -946,13 +785,7 @@ hipError_t launch_mul_strided(int logn, const u32 *F, int64_t fs, int lf, const 
         return launch_plain_strided(F, fs, lf, G, gs, lg, H, hs, lh, count, fam->p, s);
     if (logn <= kMaxLdsLog) {
         const MulDesc sd{fs, gs, hs, lf, lg, lh, logn};
-        switch (logn) {
-#define CM_CASE(K) case K: return mul_strided_t<K>(F, G, H, sd, count, fam, s);
-            CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8) CM_CASE(9) CM_CASE(10)
-            CM_CASE(11) CM_CASE(12) CM_CASE(13)
-#undef CM_CASE
-        }
-        return hipErrorInvalidValue;
+        return launch_mul_lds_strided(logn, F, G, H, sd, count, fam, s);
     }
     // four-step straight from the strided operands into the strided output,
     // in chunks whose two slabs stay within 1 GiB each
@@ -972,11 +805,10 @@ hipError_t launch_mul_strided(int logn, const u32 *F, int64_t fs, int lf, const 
 
 hipError_t launch_rows_mul(int e, u32 *F, u32 *G, int rows, const Family *fam, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    switch (e) {
-#define CM_CASE(K) case K: return rows_mul_t<K>(F, G, rows, fam, s);
-        CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8) CM_CASE(9) CM_CASE(10)
-        CM_CASE(11) CM_CASE(12) CM_CASE(13)
-#undef CM_CASE
+    if (e <= kMaxLdsLog) {
+        const int L = 1 << e;
+        const MulDesc sd{L, L, L, L, L, L, e};
+        return launch_mul_lds_strided(e, F, G, F, sd, rows, fam, s);
     }
     const int64_t n = (int64_t)1 << e;
     FourStepIO io{F, G, n, n, n, F, G, F, n, n, rows};

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "ntt_mx.h"
 
 namespace cm {
 
@@ -50,6 +51,78 @@ std::vector<u32> power_table(u32 r, size_t cnt, u32 p) {
     return t;
 }
 
+// One byte matrix of ntt_mx.h: output k of 16 adjacent elements is
+// scale * sum_d w^((d mod m)(k mod m)) x_d over the d in k's block of m = 2^t
+// (t = 0: m = 16), w of order m, times 2^32.  Byte b of the constants is the
+// signed digit of 256^b; the initial values of out_0 supply the part of the
+// product that the bytes' offset of 128 leaves out.
+void mx_matrix(int8_t *out, u32 w, int t, u32 scale, u32 p) {
+    const int m = t ? 1 << t : 16;
+    u32 *init = (u32 *)(out + 4 * 64 * 16);
+    const u32 f = cm_host_mul(scale, cm_host_r1(p), p);
+    u32 sum[16];
+    for (int k = 0; k < 16; ++k) {
+        u64 acc = 0;
+        for (int d = 0; d < 16; ++d) {
+            const u32 e = d / m == k / m ? cm_host_mul(cm_host_pow(w, (u64)(d % m) * (k % m), p), f, p) : 0u;
+            acc += e;
+            for (int a = 0; a < 4; ++a) {
+                const u32 y = cm_host_mul(e, (u32)(((u64)1 << (8 * a)) % p), p);
+                int64_t v = y > p / 2 ? (int64_t)y - p : (int64_t)y;
+                for (int b = 0; b < 4; ++b) {
+                    const int8_t digit = (int8_t)(v & 255);
+                    v = (v - digit) / 256;
+                    // lane (output k, group d / 4), byte 4 (d mod 4) + a
+                    out[(b * 64 + (d / 4) * 16 + k) * 16 + 4 * (d % 4) + a] = digit;
+                }
+            }
+        }
+        sum[k] = (u32)(acc % p);
+    }
+    auto at_least = [&](u64 c) { return (u32)(c + (kMxBias > c ? (kMxBias - c + p - 1) / p * p : 0)); };
+    for (int lane = 0; lane < 64; ++lane)
+        for (int r = 0; r < 4; ++r) {
+            const int k = 4 * (lane >> 4) + r;
+            init[lane * 4 + r] = at_least(cm_host_mul(0x80808080u % p, sum[k], p));
+            init[(64 + lane) * 4 + r] = at_least(0);
+        }
+}
+
+// matrices and twiddles of the matrix-core transforms
+bool make_mx(Family *f) {
+    const u32 p = f->p;
+    std::vector<u32> mats((size_t)kMxMats * kMxMatWords * 4, 0u);
+    auto mat = [&](int which) { return (int8_t *)(mats.data() + (size_t)which * kMxMatWords * 4); };
+    for (int t = 0; t < 4; ++t) {
+        const int lg = t ? t : 4;
+        const u32 w = cm_host_pow(f->wN, (u64)1 << (f->K - lg), p), wi = cm_host_inv(w, p);
+        const u32 sc = cm_host_inv((u32)(1 << lg) % p, p);
+        mx_matrix(mat(kMxFwd + t), w, t, 1u, p);
+        mx_matrix(mat(kMxInvFirst + t), wi, t, cm_host_mul(sc, cm_host_r1(p), p), p);
+        if (t == 0) mx_matrix(mat(kMxInv), wi, 0, sc, p);
+    }
+    f->mx_mat = upload(mats);
+    for (int dir = 0; dir < 2; ++dir) {
+        std::vector<u32> tab((size_t)2 << f->LT, 0u);
+        for (int j = 5; j <= f->LT; ++j) {
+            const size_t M = (size_t)1 << j, S = M / 16;
+            u32 w = cm_host_pow(f->wN, (u64)1 << (f->K - j), p);
+            if (dir) w = cm_host_inv(w, p);
+            u32 wk = 1;   // w^k
+            for (size_t k = 0; k < 16; ++k) {
+                u64 x = cm_host_mont(1, p);
+                for (size_t v = 0; v < S; ++v) {
+                    tab[M + k * S + v] = (u32)x;
+                    x = x * wk % p;
+                }
+                wk = cm_host_mul(wk, w, p);
+            }
+        }
+        (dir ? f->mx_ti : f->mx_tf) = upload(tab);
+    }
+    return f->mx_mat && f->mx_tf && f->mx_ti;
+}
+
 Family *make_family(u32 p, u32 wN, int K) {
     Family *f = new Family();
     f->p = p;
@@ -70,7 +143,9 @@ Family *make_family(u32 p, u32 wN, int K) {
     if (lv.empty()) { lv.push_back(cm_host_mont(1, p)); lvi.push_back(cm_host_mont(1, p)); }
     f->lv = upload(lv);
     f->lvi = upload(lvi);
-    if (!f->lv || !f->lvi) {
+    f->mx_mat = nullptr;
+    f->mx_tf = f->mx_ti = nullptr;
+    if (!f->lv || !f->lvi || (K >= 4 && !make_mx(f))) {
         delete f;
         return nullptr;
     }
