@@ -68,9 +68,10 @@ const Outer *outer_for(const Family *f, int k);   // for the current split of k
 const Family *family_default_cached(u32 p);
 const Outer *outer_cached(const Family *f, int k);
 
-// four-step split of a transform of size 2^k (k > kMaxLdsLog): rows 2^k2
-// long (k2 in 12..14), columns 2^k1 long (k1 <= 13).  The default is
-// overridden per size by cumodp_tune_set_split or CUMODP_SPLIT_<k>=<k2>.
+// four-step split of a transform of size 2^k (k > kMaxLdsLog): columns of 2^k1
+// words (4 <= k1 <= 12), rows of 2^k2.  nominal_split: the row length 12, 13 or
+// 14 that cumodp_tune_set_split or CUMODP_SPLIT_<k>=<k2> names.
+int nominal_split(int k);
 void four_step_split(int k, int &k1, int &k2);
 bool set_four_step_split(int k, int k2);
 

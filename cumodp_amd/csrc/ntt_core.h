@@ -387,16 +387,6 @@ CM_DEV void cm_dit_rounds(u32 *const (&lds)[NV], const u32 *lvi, MD md) {
     }
 }
 
-// Full forward transform of every vector of one tile whose upper halves are
-// zero (and were not stored to LDS).
-template <class TL, class MD>
-CM_DEV void cm_tile_dif_topzero(u32 *lds, const u32 *lv, MD md) {
-    u32 *const t[1] = {lds};
-    Round<TL, 0>::template dif<1, true>(t, lv, md);
-    __syncthreads();
-    cm_dif_rounds<TL, 1, TL::NR, 1>(t, lv, md);
-}
-
 // Full forward transform of every vector of one tile (bit-reversed result).
 template <class TL, class MD>
 CM_DEV void cm_tile_dif(u32 *lds, const u32 *lv, MD md) {
@@ -408,138 +398,6 @@ template <class TL, class MD>
 CM_DEV void cm_tile_dit(u32 *lds, const u32 *lvi, MD md) {
     u32 *const t[1] = {lds};
     cm_dit_rounds<TL, TL::NR - 1, 0, 1>(t, lvi, md);
-}
-
-// Column tiles (COLS) whose first and last rounds talk to global memory
-// directly: element (row, c) of the tile is X[row n2 + c], X at the tile's
-// first column.  Each thread's round-group is one column, so a wave reads or
-// writes C-column row segments; the row-dependent part of an address is
-// uniform (m 2^DLOG n2), which keeps the per-lane offset in one 32-bit
-// register.  No LDS staging pass and no barrier precede the first round or
-// follow the last.
-
-// Word `off` of a row whose base is uniform, addressed as base + 4 off with a
-// 32-bit byte offset.  off < 2^30 (tiles of transforms up to 2^26 words).
-CM_DEV u32 cm_ld_row(const u32 *base, u32 off) {
-    return *(const u32 *)((const char *)base + (off << 2));
-}
-CM_DEV void cm_st_row(u32 *base, u32 off, u32 v) { *(u32 *)((char *)base + (off << 2)) = v; }
-
-// Raw buffer view of a tile: the tile base in a scalar resource, each access
-// = per-lane byte offset (vector register) + uniform row byte offset (scalar
-// register), so no vector instruction computes an address.  No range limit
-// (every access stays inside the arrays the caller passed); word 3 is the
-// raw-buffer format of the gfx9 family.
-CM_DEV __amdgpu_buffer_rsrc_t cm_tile_rsrc(const u32 *base) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
-}
-CM_DEV u32 cm_buf_ld(__amdgpu_buffer_rsrc_t r, u32 off_bytes, u32 row_bytes) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off_bytes, (int)row_bytes, 0);
-}
-CM_DEV void cm_buf_st(__amdgpu_buffer_rsrc_t r, u32 off_bytes, u32 row_bytes, u32 v) {
-    __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)off_bytes, (int)row_bytes, 0);
-}
-
-// Forward round 0 from global memory into LDS.  CHECK: elements at or beyond
-// lim (relative to X) read as zero.  TOPZERO: rows >= L/2 are zero and not
-// read.
-template <class TL, bool TOPZERO, bool CHECK, class MD>
-CM_DEV void cm_col_dif_first(u32 *lds, const u32 *X, int64_t n2, int64_t lim, const u32 *lv,
-                             MD md) {
-    using RD = Round<TL, 0>;
-    constexpr int R = RD::R, M = TOPZERO ? (1 << (R - 1)) : (1 << R);
-#pragma unroll
-    for (int q = 0; q < RD::GPT; ++q) {
-        typename RD::G g(threadIdx.x + q * TL::T);
-        const u32 off = (u32)g.i0 * (u32)n2 + (u32)g.c;
-        u32 v[1][1 << R];
-        if constexpr (CHECK) {
-#pragma unroll
-            for (int m = 0; m < M; ++m) {
-                const int64_t rowoff = (int64_t)(m << RD::DLOG) * n2;
-                v[0][m] = rowoff + off < lim ? cm_ld_row(X + rowoff, off) : 0u;
-            }
-        } else {
-            const auto rx = cm_tile_rsrc(X);
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-                v[0][m] = cm_buf_ld(rx, off << 2, (u32)((m << RD::DLOG) * n2) << 2);
-        }
-        cm_dif_stages<TL::LOGL, R, RD::S0, RD::DLOG, 1, TOPZERO>(v, g.gi_lo, lv, md);
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m) lds[g.a(m)] = v[0][m];
-    }
-}
-
-// Last forward round from LDS straight to global memory (all rows).
-template <class TL, class MD>
-CM_DEV void cm_col_dif_last(const u32 *lds, u32 *Y, int64_t n2, const u32 *lv, MD md) {
-    using RD = Round<TL, TL::NR - 1>;
-    constexpr int R = RD::R;
-    const auto ry = cm_tile_rsrc(Y);
-#pragma unroll
-    for (int q = 0; q < RD::GPT; ++q) {
-        typename RD::G g(threadIdx.x + q * TL::T);
-        const u32 off = (u32)g.i0 * (u32)n2 + (u32)g.c;
-        u32 v[1][1 << R];
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m) v[0][m] = lds[g.a(m)];
-        cm_dif_stages<TL::LOGL, R, RD::S0, RD::DLOG, 1>(v, g.gi_lo, lv, md);
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m)
-            cm_buf_st(ry, off << 2, (u32)((m << RD::DLOG) * n2) << 2, v[0][m]);
-    }
-}
-
-// First inverse round (round NR-1) from global memory into LDS (all rows).
-template <class TL, class MD>
-CM_DEV void cm_col_dit_first(u32 *lds, const u32 *X, int64_t n2, const u32 *lvi, MD md) {
-    using RD = Round<TL, TL::NR - 1>;
-    constexpr int R = RD::R;
-    const auto rx = cm_tile_rsrc(X);
-#pragma unroll
-    for (int q = 0; q < RD::GPT; ++q) {
-        typename RD::G g(threadIdx.x + q * TL::T);
-        const u32 off = (u32)g.i0 * (u32)n2 + (u32)g.c;
-        u32 v[1][1 << R];
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m)
-            v[0][m] = cm_buf_ld(rx, off << 2, (u32)((m << RD::DLOG) * n2) << 2);
-        cm_dit_stages<TL::LOGL, R, RD::S0, RD::DLOG, 1>(v, g.gi_lo, lvi, md);
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m) lds[g.a(m)] = v[0][m];
-    }
-}
-
-// Last inverse round (round 0) from LDS straight to global memory, canonical
-// residues out.  CHECK: elements at or beyond lim (relative to Y) are not
-// stored.
-template <class TL, bool CHECK, class MD>
-CM_DEV void cm_col_dit_last(const u32 *lds, u32 *Y, int64_t n2, int64_t lim, const u32 *lvi,
-                            MD md) {
-    using RD = Round<TL, 0>;
-    constexpr int R = RD::R;
-#pragma unroll
-    for (int q = 0; q < RD::GPT; ++q) {
-        typename RD::G g(threadIdx.x + q * TL::T);
-        const u32 off = (u32)g.i0 * (u32)n2 + (u32)g.c;
-        u32 v[1][1 << R];
-#pragma unroll
-        for (int m = 0; m < (1 << R); ++m) v[0][m] = lds[g.a(m)];
-        cm_dit_stages<TL::LOGL, R, RD::S0, RD::DLOG, 1>(v, g.gi_lo, lvi, md);
-        if constexpr (CHECK) {
-#pragma unroll
-            for (int m = 0; m < (1 << R); ++m) {
-                const int64_t rowoff = (int64_t)(m << RD::DLOG) * n2;
-                if (rowoff + off < lim) cm_st_row(Y + rowoff, off, cm_canon(v[0][m], md));
-            }
-        } else {
-            const auto ry = cm_tile_rsrc(Y);
-#pragma unroll
-            for (int m = 0; m < (1 << R); ++m)
-                cm_buf_st(ry, off << 2, (u32)((m << RD::DLOG) * n2) << 2, cm_canon(v[0][m], md));
-        }
-    }
 }
 
 // Multiply of two tiles A (first operand, becomes the product) and B:

@@ -28,6 +28,7 @@ std::mutex g_plan_mutex;
 std::map<std::tuple<u32, u32, int>, Family *> g_families;
 std::map<std::tuple<const Family *, int, int>, Outer *> g_outer;
 int g_split[kMaxLog + 1];   // chosen k2 per k (0: default)
+int default_split(int k) { return k >= 25 ? 14 : (k >= 21 ? 13 : 12); }
 std::map<u32, const Family *> g_default;
 
 u32 *upload(const std::vector<u32> &h) {
@@ -79,12 +80,14 @@ void mx_matrix(int8_t *out, u32 w, int t, u32 scale, u32 p) {
         }
         sum[k] = (u32)(acc % p);
     }
-    auto at_least = [&](u64 c) { return (u32)(c + (kMxBias > c ? (kMxBias - c + p - 1) / p * p : 0)); };
+    // out_0's initial value: the offset's share less the 2^32 kMxHigh that the
+    // kernels add, a residue at or above kMxBias
+    const u32 high = cm_host_mul(kMxHigh % p, cm_host_r1(p), p);
     for (int lane = 0; lane < 64; ++lane)
         for (int r = 0; r < 4; ++r) {
-            const int k = 4 * (lane >> 4) + r;
-            init[lane * 4 + r] = at_least(cm_host_mul(0x80808080u % p, sum[k], p));
-            init[(64 + lane) * 4 + r] = at_least(0);
+            const u32 sum_k = sum[4 * (lane >> 4) + r];
+            const u32 c = cm_sub(cm_host_mul(0x80808080u % p, sum_k, p), high, p);
+            init[lane * 4 + r] = c + (c < kMxBias ? (kMxBias - c + p - 1) / p * p : 0u);
         }
 }
 
@@ -99,7 +102,10 @@ bool make_mx(Family *f) {
         const u32 sc = cm_host_inv((u32)(1 << lg) % p, p);
         mx_matrix(mat(kMxFwd + t), w, t, 1u, p);
         mx_matrix(mat(kMxInvFirst + t), wi, t, cm_host_mul(sc, cm_host_r1(p), p), p);
-        if (t == 0) mx_matrix(mat(kMxInv), wi, 0, sc, p);
+        mx_matrix(mat(kMxInv + t), wi, t, sc, p);
+        if (t == 0)
+            mx_matrix(mat(kMxInvPair), wi, 0,
+                      cm_host_mul(cm_host_inv(32 % p, p), cm_host_r1(p), p), p);
     }
     f->mx_mat = upload(mats);
     for (int dir = 0; dir < 2; ++dir) {
@@ -188,7 +194,9 @@ const Family *family_default_cached(u32 p) {
     return it != g_default.end() ? it->second : nullptr;
 }
 
-void four_step_split(int k, int &k1, int &k2) {
+// The row length 2^k2 that cumodp_tune_set_split or the environment names;
+// 12 (k <= 20), 13 (k <= 24) or 14 when nothing does.
+int nominal_split(int k) {
     int c = (k >= 0 && k <= kMaxLog) ? g_split[k] : 0;
     if (!c) {
         char name[32];
@@ -196,12 +204,19 @@ void four_step_split(int k, int &k1, int &k2) {
         const char *e = getenv(name);
         if (e) c = atoi(e);
     }
-    // measured defaults on MI355X (cumodp_amd.autotune, back-to-back 2^k
-    // multiplies): 2^12-word rows up to 2^20, 2^13 for 2^21..2^24, 2^14 above
-    if (c < 12 || c > 14 || k - c < 1 || k - c > kMaxLdsLog)
-        c = k >= 25 ? 14 : (k >= 21 ? 13 : 12);
-    k2 = c;
-    k1 = k - k2;
+    if (c < 12 || c > 14 || k - c < 1 || k - c > kMaxLdsLog) c = default_split(k);
+    return c;
+}
+
+// The nominal value stands for the library's own choice: columns short enough
+// that both passes fill the chip (measured over every split of 2^14 .. 2^24).
+// Columns have 2^4 .. 2^12 words.
+void four_step_split(int k, int &k1, int &k2) {
+    static const int own[kMaxLog - kMaxLdsLog] = {6, 6, 6, 7, 8, 8, 8, 8, 10, 10, 11, 11, 12};
+    const int c = nominal_split(k);
+    k1 = c == default_split(k) ? own[k - kMaxLdsLog - 1] : k - c;
+    k1 = k1 < 4 ? 4 : (k1 > 12 ? 12 : k1);
+    k2 = k - k1;
 }
 
 bool set_four_step_split(int k, int k2) {
@@ -233,17 +248,14 @@ const Outer *outer_for(const Family *f, int k) {
     o->hi_f = upload(power_table(cm_host_pow(wn, nlo, p), nhi, p));
     o->lo_i = upload(power_table(wni, nlo, p));
     o->hi_i = upload(power_table(cm_host_pow(wni, nlo, p), nhi, p));
-    // row-pass tables; the inverse rb table also carries 2^32 / n, the scale
-    // the row pass leaves out of its pointwise product (one Montgomery
-    // product gives F G / 2^32, the inverse transform a factor n)
+    // row-pass tables
     const size_t n1 = (size_t)1 << k1, T = ((size_t)1 << k2) / 16;
-    const u32 unscale = cm_host_mul(cm_host_r1(p), cm_host_inv(cm_host_pow(2, k, p), p), p);
     for (int dir = 0; dir < 2; ++dir) {
         const u32 w = dir ? wni : wn;
         std::vector<u32> rb(n1 * T), rc(n1 * 16);
         for (size_t r = 0; r < n1; ++r) {
             const u32 wr = cm_host_pow(w, r, p);                 // w^k1
-            u64 x = cm_host_mont(dir ? unscale : 1u, p);
+            u64 x = cm_host_mont(1, p);
             for (size_t t = 0; t < T; ++t) {
                 rb[r * T + t] = (u32)x;
                 x = x * wr % p;

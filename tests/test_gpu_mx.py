@@ -55,3 +55,48 @@ def test_output_over_an_operand(cm, orc):
             a, b = (other, d) if over else (d, other)
             cm.fftmul_uni_dev(n - 2, d, n // 2 - 1, a, n // 2 - 1, b, P1)
             assert (d.download()[:n - 1] == want).all(), (e, over)
+
+
+@pytest.mark.parametrize("p,top", [(P1, 22), (P2, 21), (TOP, 17), (65537, 16)])
+def test_four_step_products(cm, orc, p, top):
+    """Ragged operands at odd word offsets, in the small and the large form
+    (2^20 words and up), and a truncated output."""
+    rng = np.random.default_rng(p + 1)
+    for e in range(14, top + 1):
+        n = 1 << e
+        for s, off in ((n, 0), (n // 2 + 1, 1), (n - 3, 3)):
+            lf = (s + 1) * 5 // 8
+            lg = s + 1 - lf
+            F = rng.integers(0, p, lf + off, dtype=np.int32)
+            G = rng.integers(0, p, lg + off, dtype=np.int32)
+            want = orc.ntt_polymul(F[off:], G[off:], p)
+            dF, dG = cm.DeviceArray.from_host(F), cm.DeviceArray.from_host(G)
+            for nout in (s, s // 2 + 5):
+                dH = cm.DeviceArray.from_host(np.full(s + off + 8, -1, np.int32))
+                cm.fftmul_uni_dev(nout - 1, dH.ptr + 4 * off, lf - 1, dF.ptr + 4 * off, lg - 1,
+                                  dG.ptr + 4 * off, p)
+                got = dH.download()
+                assert (got[off:off + nout] == want[:nout]).all(), (p, e, s, nout)
+                assert (got[:off] == -1).all() and (got[off + nout:] == -1).all(), (p, e, s, nout)
+
+
+@pytest.mark.parametrize("logn", [14, 15, 17, 19, 21, 22])
+def test_every_split_and_tile(cm, orc, logn):
+    """Row lengths named by the tuner (columns down to 16 words) and both
+    column tiles give the same words."""
+    L = cm.lib()
+    rng = np.random.default_rng(logn)
+    n = 1 << logn
+    F, G = rng.integers(0, P2, n // 2, dtype=np.int32), rng.integers(0, P2, n // 2, dtype=np.int32)
+    want = orc.ntt_polymul(F, G, P2)
+    keep = L.cumodp_tune_get_split(logn)
+    try:
+        for k2 in (12, 13, 14):
+            if L.cumodp_tune_set_split(logn, k2):
+                continue
+            for tile in (8192, 16384):
+                assert L.cumodp_tune_set_col_tile(tile) == 0
+                assert (_mul(cm, F, G, P2) == want).all(), (logn, k2, tile)
+    finally:
+        assert L.cumodp_tune_set_split(logn, keep) == 0
+        assert L.cumodp_tune_set_col_tile(16384) == 0
