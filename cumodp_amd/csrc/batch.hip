@@ -20,6 +20,7 @@
 #include "accum.h"
 #include "internal.h"
 #include "ntt_core.h"
+#include "ntt_mx.h"
 
 namespace cm {
 
@@ -162,6 +163,8 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 //     2^15-point product, recombined by a short kernel after the launch;
 //   * plain: 4096 consecutive outputs of one schoolbook product (16 waves of
 //     256 outputs, each wave on its own, the arithmetic of k_plain_mul).
+// The 4096 uneven pairs (degrees 32 .. 16384) take 226 us per call with the
+// tile products on the matrix cores, 256 us as radix-2 butterflies.
 // Largest tasks first keeps the tail short; the counter starts at zero in
 // every call's uploaded descriptor blob.  (A loop over tasks in fewer
 // workgroups was measured slower: inlined into the loop, the task bodies'
@@ -169,7 +172,6 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 // line they take their uniform pointers in vector registers.)
 constexpr int kPT = 1024;                    // threads of the persistent workgroup
 constexpr int kPW = 16384;                   // words per product tile
-constexpr int kPLW = kPW + (kPW >> 4);       // LDS words of one operand tile (padded layouts)
 constexpr int kPlainTaskOut = 4096;          // outputs of a plain task (16 waves x 256)
 constexpr int kPlainJT = 512;                // B coefficients per pass of a plain task
 
@@ -189,62 +191,87 @@ struct ListTask {
 //   B = H mod x^n + 1, the negacyclic product of F_lo - F_hi and G_lo - G_hi,
 //       taken as the cyclic product of the operands twisted by psi^i (psi a
 //       primitive 2^15-th root, psi^n = -1) and untwisted by psi^-i.
-// With the pointwise constant of a 2^15-point product both come out halved,
-// so H_i = A_i/2 + psi^-i B'_i/2 and H_(n+i) = A_i/2 - psi^-i B'_i/2.  psi^i
-// and psi^-i are entries of the 2^15 level tables.
-// The halves are separate tasks: the cyclic one leaves A/2 in H_0 ..
-// H_(n-1) (inside the output: the product has more than n coefficients), the
-// negacyclic one psi^-i B'/2 in the product's slot of the scratch S, and
-// k_big_combine adds and subtracts them after the launch.  (Both halves in
-// one workgroup spill: the operand loads of the second are scheduled beside
-// the registers of the first.)  Thread t holds elements i = t + 1024 r.
-template <bool NEGA, class MD>
+// Then 2 H_i = A_i + psi^-i B'_i and 2 H_(n+i) = A_i - psi^-i B'_i.  psi^i and
+// psi^-i are entries of the 2^15 level tables.
+// The halves are separate tasks: the cyclic one leaves A in H_0 .. H_(n-1)
+// (inside the output: the product has more than n coefficients), the
+// negacyclic one psi^-i B' in the product's slot of the scratch S, and
+// k_big_combine adds, subtracts and halves them after the launch.
+template <bool NEGA>
 CM_DEV void task_big_half(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp,
-                          u32 *S, int slot, const u32 *lv, const u32 *lvi, MD md, u32 sc15) {
-    using TL = Tile<14, 1, false, kPT>;
-    constexpr int n = 1 << 14;
+                          u32 *S, int slot, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
+    constexpr int LOGN = 14, n = 1 << LOGN, V = 4, LT = LOGN - 4;
+    using Map = MxMap<LT, V>;
     const MulDesc d = *dp;
-    const u32 p = md.p;
-    const int t = threadIdx.x;
-    u32 fa[16], ga[16];
+    const int i0 = Map::base();
+    MxMat m;
+    u32 x[2][V][4], tw[V][4];
+    mx_forward_begin<LOGN, 0, V>(m, tw, cx);
+    // F_lo +- F_hi (the sum of two residues fits a word; p is added to the
+    // difference), the negacyclic operands times psi^i
+    auto operand = [&](u32 (&y)[V][4], const u32 *q, int len) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int i = t + (r << 10);
-        const u32 f0 = i < d.lf ? F[d.f + i] : 0u, f1 = n + i < d.lf ? F[d.f + n + i] : 0u;
-        const u32 g0 = i < d.lg ? G[d.g + i] : 0u, g1 = n + i < d.lg ? G[d.g + n + i] : 0u;
-        if constexpr (NEGA) {
-            const u32 psi = lv[n - 1 + i];
-            fa[r] = cm_mulw(cm_sub(f0, f1, p), psi, md);
-            ga[r] = cm_mulw(cm_sub(g0, g1, p), psi, md);
-        } else {
-            fa[r] = cm_add(f0, f1, p);
-            ga[r] = cm_add(g0, g1, p);
+        for (int r = 0; r < 4; ++r) {
+            const int i = i0 + Map::off(0, r);
+            MxQuad lo, hi;
+            if (i + 4 <= len) {
+                lo = *(const MxQuad *)(q + i);
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) lo.v[s] = i + s < len ? q[i + s] : 0u;
+            }
+            if (n + i + 4 <= len) {
+                hi = *(const MxQuad *)(q + n + i);
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) hi.v[s] = n + i + s < len ? q[n + i + s] : 0u;
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) y[s][r] = NEGA ? lo.v[s] - hi.v[s] + cx.p : lo.v[s] + hi.v[s];
         }
-    }
-    cm_row_multiply<TL>(lds, lds + n, fa, ga, lv, lvi, md, sc15);
-    u32 *Sp = S + (int64_t)slot * n;
+        if constexpr (NEGA) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int i = t + (r << 10);
-        if constexpr (NEGA) Sp[i] = cm_mulw(fa[r], lvi[n - 1 + i], md);
-        else H[d.h + i] = fa[r];
+            for (int r = 0; r < 4; ++r) {
+                const MxQuad w = *(const MxQuad *)(lv + n - 1 + i0 + Map::off(0, r));
+#pragma unroll
+                for (int s = 0; s < 4; ++s) y[s][r] = cm_mont_lazy(y[s][r], w.v[s], cx.p, cx.np);
+            }
+        }
+    };
+    operand(x[0], F + d.f, d.lf);
+    operand(x[1], G + d.g, d.lg);
+    mx_tile_multiply<LOGN, V>(x, lds, lds + mx_lds_words(n), cx, m, tw);
+    u32 *out = NEGA ? S + (int64_t)slot * n : H + d.h;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int i = i0 + Map::off(0, r);
+        MxQuad v;
+        if constexpr (NEGA) {
+            const MxQuad w = *(const MxQuad *)(lvi + n - 1 + i);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v.v[s] = cm_mont_lazy(x[0][s][r], w.v[s], cx.p, cx.np);
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v.v[s] = x[0][s][r];
+        }
+        *(MxQuad *)(out + i) = v;
     }
 }
 
-// H_i = A_i/2 + S_i, H_(n+i) = A_i/2 - S_i for the 2^15-point products
-// (descriptors descs[0 .. count), slot j at S + j n), canonical out.  A/2
-// and S are in [0, c), c = p or 2p.
-template <class MD>
+// H_i = (A_i + S_i) / 2, H_(n+i) = (A_i - S_i) / 2 for the 2^15-point products
+// (descriptors descs[0 .. count), slot j at S + j n), canonical out.  A is a
+// matrix step's word (below p + 4200), S a Montgomery product's (below 2p).
 __global__ void k_big_combine(u32 *__restrict__ H, const MulDesc *__restrict__ descs,
-                              const u32 *__restrict__ S, MD md) {
+                              const u32 *__restrict__ S, MxCtx cx) {
     constexpr int n = 1 << 14;
     const MulDesc d = descs[blockIdx.y];
-    const u32 c = cm_bound(md);
     const u32 *Sp = S + (int64_t)blockIdx.y * n;
+    const u32 p = cx.p;
+    auto half = [&](u32 v) { return (v + (v & 1 ? p : 0u)) >> 1; };
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const u32 a = H[d.h + i], u = Sp[i];
-        H[d.h + i] = cm_canon(cm_reduce2p(a + u, c), md);
-        if (n + i < d.lh) H[d.h + n + i] = cm_canon(cm_sub(a, u, c), md);
+        const u32 a = mx_canon(H[d.h + i], cx), u = cm_reduce2p(Sp[i], p);
+        H[d.h + i] = half(cm_add(a, u, p));
+        if (n + i < d.lh) H[d.h + n + i] = half(cm_sub(a, u, p));
     }
 }
 
@@ -329,50 +356,71 @@ CM_DEV void task_plain(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDe
 }
 
 // One tile of products of 2^K points (16384 >> K of them).
-template <int K, class MD>
-CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H,
-                                       const MulDesc *d, int cnt, const u32 *lv, const u32 *lvi,
-                                       MD md, u32 sc) {
-    mul_tile<K, kPW, kPT>(lds, lds + kPLW, F, G, H, d, cnt, lv, lvi, md, sc);
+template <int K>
+CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *d, int cnt,
+                      const MxCtx &cx) {
+    constexpr int V = 4;
+    using Map = MxMap<MxPlan<K>::words(0), V>;
+    const int row0 = Map::base() >> K;
+    auto desc = [&](int s) {
+        const int c = row0 + (Map::off(s, 0) >> K);
+        return c < cnt ? d[c] : MulDesc{};
+    };
+    MxMat m;
+    u32 x[2][V][4], tw[V][4];
+    mx_forward_begin<K, 0, V>(m, tw, cx);
+    mx_load_rows<K, V>(x[0], [&](int s, const u32 *&q, int &len) {
+        const MulDesc e = desc(s);
+        q = F + e.f;
+        len = e.lf;
+    });
+    mx_load_rows<K, V>(x[1], [&](int s, const u32 *&q, int &len) {
+        const MulDesc e = desc(s);
+        q = G + e.g;
+        len = e.lg;
+    });
+    mx_tile_multiply<K, V>(x, lds, lds + mx_lds_words(kPW), cx, m, tw);
+    mx_store_rows<K, V>(
+        x[0],
+        [&](int s, u32 *&q, int &len) {
+            const MulDesc e = desc(s);
+            q = H + e.h;
+            len = e.lh;
+        },
+        cx);
 }
 
-template <class MD>
 __global__ __launch_bounds__(kPT) void k_list_persistent(
     const u32 *__restrict__ F, const u32 *__restrict__ G, u32 *__restrict__ H,
     const MulDesc *__restrict__ descs, const ListTask *__restrict__ tasks, int ntasks,
-    int *__restrict__ counter, const u32 *__restrict__ scales, u32 *__restrict__ big_s,
-    const u32 *__restrict__ lv, const u32 *__restrict__ lvi, MD md, PlainMod pm) {
-    __shared__ __align__(16) u32 lds[2 * kPLW];
+    int *__restrict__ counter, u32 *__restrict__ big_s, const u32 *__restrict__ lv,
+    const u32 *__restrict__ lvi, MxCtx cx, PlainMod pm) {
+    __shared__ __align__(16) u32 lds[2 * mx_lds_words(kPW)];
     __shared__ int s_next;
     if (threadIdx.x == 0) s_next = atomicAdd(counter, 1);
     __syncthreads();
     // uniform: the task and its descriptor load through the scalar unit
     const int ti = __builtin_amdgcn_readfirstlane(s_next);
     if (ti >= ntasks) return;   // one workgroup per task: never taken
-    {
-        const ListTask t = tasks[ti];
-        if (t.kind == kTaskPlain) {
-            task_plain(lds, F, G, H, descs + t.first, t.count, pm);
-        } else if (t.kind == kTaskBigCyc) {
-            task_big_half<false>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, md,
-                                 scales[15]);
-        } else if (t.kind == kTaskBigNeg) {
-            task_big_half<true>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, md,
-                                scales[15]);
-        } else {
-            const MulDesc *d = descs + t.first;
-            const u32 sc = scales[t.logn];
-#define CM_PMIX(K)                                                          \
-    case K:                                                                 \
-        task_tile<K>(lds, F, G, H, d, t.count, lv, lvi, md, sc);            \
+    const ListTask t = tasks[ti];
+    if (t.kind == kTaskPlain) {
+        task_plain(lds, F, G, H, descs + t.first, t.count, pm);
+    } else if (t.kind == kTaskBigCyc) {
+        task_big_half<false>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, cx);
+    } else if (t.kind == kTaskBigNeg) {
+        task_big_half<true>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, cx);
+    } else {
+        const MulDesc *d = descs + t.first;
+#define CM_PMIX(K)                                       \
+    case K:                                              \
+        task_tile<K>(lds, F, G, H, d, t.count, cx);      \
         break;
-            switch (t.logn) {
-                CM_PMIX(4) CM_PMIX(5) CM_PMIX(6) CM_PMIX(7) CM_PMIX(8) CM_PMIX(9) CM_PMIX(10)
-                CM_PMIX(11) CM_PMIX(12) CM_PMIX(13) CM_PMIX(14)
-            default: break;
-            }
-#undef CM_PMIX
+        switch (t.logn) {
+            CM_PMIX(4) CM_PMIX(5) CM_PMIX(6) CM_PMIX(7) CM_PMIX(8) CM_PMIX(9) CM_PMIX(10)
+            CM_PMIX(11) CM_PMIX(12) CM_PMIX(13) CM_PMIX(14)
+        default: break;
         }
+#undef CM_PMIX
     }
 }
 
@@ -685,19 +733,16 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     const int64_t ntasks = nplain_tasks + ntile + 2 * nbig;
     if (ntasks > INT32_MAX) return hipErrorInvalidValue;
 
-    // blob: the task counter (16 bytes), the pointwise scales of sizes 2^0 ..
-    // 2^15 (64 bytes), the sorted descriptors, the tasks; written straight
-    // into the pinned staging buffer
-    const size_t scale_off = 16, desc_off = 80;
+    // blob: the task counter (16 bytes), the sorted descriptors, the tasks;
+    // written straight into the pinned staging buffer
+    const size_t desc_off = 16;
     const size_t task_off = desc_off + sizeof(MulDesc) * (size_t)count;
     const size_t bytes = task_off + sizeof(ListTask) * (size_t)ntasks;
-    const Scales scl = scale_table(fam);
     std::vector<MulDesc> tail;   // host copy of the four-step classes' descriptors
     char *dblob = (char *)workspace(7, bytes, s);
     if (!dblob) return hipErrorOutOfMemory;
     hipError_t e = stage_upload_fill(bytes, dblob, s, [&](char *blob) {
         memset(blob, 0, desc_off);   // the task counter starts at 0
-        memcpy(blob + scale_off, scl.v, sizeof(scl.v));
         MulDesc *sorted = (MulDesc *)(blob + desc_off);
         ListTask *tasks = (ListTask *)(blob + task_off);
         int64_t pos[33];
@@ -751,10 +796,9 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     });
     if (e != hipSuccess) return e;
     int *d_counter = (int *)dblob;
-    const u32 *d_scales = (const u32 *)(dblob + scale_off);
     const MulDesc *d_descs = (const MulDesc *)(dblob + desc_off);
     const ListTask *d_tasks = (const ListTask *)(dblob + task_off);
-    u32 *big_s = nullptr;   // psi^-i B'/2 of each 2^15-point product, 2^14 words each
+    u32 *big_s = nullptr;   // psi^-i B' of each 2^15-point product, 2^14 words each
     if (nbig > 0) {
         big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig << 14), s);
         if (!big_s) return hipErrorOutOfMemory;
@@ -762,27 +806,16 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     if (ntasks > 0) {
         ProfScope ps(kProfListPersistent, s);
         const dim3 grid((unsigned)ntasks);
-        const PlainMod pm = plain_mod(fam->p);
-        if (fam->p < (1u << 30))
-            hipLaunchKernelGGL(k_list_persistent<ModLazy>, grid, dim3(kPT), 0, s, F, G, H, d_descs,
-                               d_tasks, (int)ntasks, d_counter, d_scales, big_s, fam->lv,
-                               fam->lvi, ModLazy{fam->p, fam->np}, pm);
-        else
-            hipLaunchKernelGGL(k_list_persistent<Mod>, grid, dim3(kPT), 0, s, F, G, H, d_descs,
-                               d_tasks, (int)ntasks, d_counter, d_scales, big_s, fam->lv,
-                               fam->lvi, Mod{fam->p, fam->np}, pm);
+        hipLaunchKernelGGL(k_list_persistent, grid, dim3(kPT), 0, s, F, G, H, d_descs, d_tasks,
+                           (int)ntasks, d_counter, big_s, fam->lv, fam->lvi, mx_ctx(fam),
+                           plain_mod(fam->p));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (nbig > 0) {
         ProfScope ps(kProfListPersistent, s);
-        const dim3 grid(16, (unsigned)nbig);
-        if (fam->p < (1u << 30))
-            hipLaunchKernelGGL(k_big_combine<ModLazy>, grid, dim3(1024), 0, s, H,
-                               d_descs + off[kBigLog], big_s, ModLazy{fam->p, fam->np});
-        else
-            hipLaunchKernelGGL(k_big_combine<Mod>, grid, dim3(1024), 0, s, H,
-                               d_descs + off[kBigLog], big_s, Mod{fam->p, fam->np});
+        hipLaunchKernelGGL(k_big_combine, dim3(16, (unsigned)nbig), dim3(1024), 0, s, H,
+                           d_descs + off[kBigLog], big_s, mx_ctx(fam));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

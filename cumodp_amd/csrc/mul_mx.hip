@@ -81,11 +81,6 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
 // fit a workgroup).
 constexpr int64_t kMxSpreadWords = (int64_t)1 << 19;
 
-static MxCtx ctx_of(const Family *fam) {
-    return MxCtx{(const mx_v4i *)fam->mx_mat, fam->mx_tf, fam->mx_ti, fam->p, fam->np,
-                 cm_host_r1(fam->p), 1u << 16};
-}
-
 template <int LOGL, int V, bool DESC>
 static hipError_t mul_mx_v(const u32 *F, const u32 *G, u32 *H, const MulDesc *descs, int ndesc,
                            const MulDesc &one, const Family *fam, hipStream_t s) {
@@ -93,7 +88,7 @@ static hipError_t mul_mx_v(const u32 *F, const u32 *G, u32 *H, const MulDesc *de
     constexpr int C = 1 << (LOGW - LOGL);
     ProfScope ps(kProfMulLds, s);
     hipLaunchKernelGGL((k_mul_mx<LOGL, LOGW, V, DESC>), dim3((ndesc + C - 1) / C),
-                       dim3((1 << LOGW) / (4 * V)), 0, s, F, G, H, descs, ndesc, one, ctx_of(fam));
+                       dim3((1 << LOGW) / (4 * V)), 0, s, F, G, H, descs, ndesc, one, mx_ctx(fam));
     return hipGetLastError();
 }
 
@@ -418,7 +413,7 @@ int col_tile_words() { return g_col_words; }
 
 static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCols &s1, int cnt0,
                               int cnt1, int k2, bool small, const Family *fam, hipStream_t s) {
-    const MxCtx cx = ctx_of(fam);
+    const MxCtx cx = mx_ctx(fam);
 #define CM_COL(LC, V) return cols_t<K, LC, V>(inverse, s0, s1, cnt0, cnt1, k2, cx, s)
 #define CM_COLS(KK, LS, VS, LB)                       \
     case KK: {                                        \
@@ -459,7 +454,7 @@ static hipError_t rows_t(const FourStepIO &io, const Outer *o, const Family *fam
     const int64_t words = (int64_t)io.cnt << o->k;
     hipLaunchKernelGGL((k_row_mx<LOGL, V>), dim3((unsigned)(words >> LOGW)),
                        dim3((1 << LOGW) / (4 * V)), 0, s, io.f_ws, io.g_ws, o->k1, o->rb_f,
-                       o->rc_f, o->rb_i, o->rc_i, ctx_of(fam));
+                       o->rc_f, o->rb_i, o->rc_i, mx_ctx(fam));
     return hipGetLastError();
 }
 

@@ -39,6 +39,7 @@
 // is its exact mirror, so products never permute data.
 #pragma once
 
+#include "internal.h"
 #include "modarith.h"
 
 #define CM_DEV __device__ __forceinline__
@@ -73,6 +74,11 @@ struct MxCtx {
     const u32 *tf, *ti;
     u32 p, np, r1, c16;
 };
+
+static inline MxCtx mx_ctx(const Family *fam) {
+    return MxCtx{(const mx_v4i *)fam->mx_mat, fam->mx_tf, fam->mx_ti, fam->p, fam->np,
+                 cm_host_r1(fam->p), 1u << 16};
+}
 
 struct MxMat {
     mx_v4i a0, a1, a2, a3, clo;
