@@ -246,6 +246,16 @@ int list_persistent();
 // (G overwritten when 2^e > 2^13).
 hipError_t launch_rows_mul(int e, u32 *F, u32 *G, int rows, const Family *fam, hipStream_t s);
 
+// f[r] <- f[r] * g[r] mod x^(2^e) - 1 for the rows of several segments, each of
+// one length and modulus (rows_batch.hip); only the first flen / glen words of
+// a row of f / g are read, g is overwritten.
+struct RowSeg {
+    u32 *f, *g;
+    int rows, e, flen, glen;
+    const Family *fam;
+};
+hipError_t launch_rows_batch(std::vector<RowSeg> segs, hipStream_t s);
+
 // two-convolution integer multiply on device buffers (twoconv.hip); *err is
 // set when no (K, M, primes) satisfies the CRT bound
 hipError_t launch_two_convolution(const u64 *a, int64_t na, int wa, const u64 *b, int64_t nb,

@@ -1,0 +1,206 @@
+// mul_mx.h -- the passes of the matrix-core four-step multiply (ntt_mx.h) as
+// device functions: columns of a 2^k1 x 2^k2 array and its rows.
+#pragma once
+
+#include "ntt_mx.h"
+
+namespace cm {
+
+// Workgroups are dispatched round-robin over the 8 XCDs; give each XCD a
+// contiguous range of logical blocks so that neighbouring column tiles (which
+// share 128-byte lines) meet in the same L2.
+CM_DEV int mx_xcd(int b, int nb) { return nb & 7 ? b : (b & 7) * (nb >> 3) + (b >> 3); }
+
+// Outer twiddle tables of one size (struct Outer of internal.h).
+struct MxOuter {
+    const u32 *rb_f, *rc_f, *rb_i, *rc_i;
+};
+
+static inline MxOuter mx_outer_of(const Outer *o) {
+    return MxOuter{o->rb_f, o->rc_f, o->rb_i, o->rc_i};
+}
+
+template <int LOGL, int LOGC>
+constexpr int mx_col_lds() {
+    return MxPlan<LOGL, LOGC>::NR > 1 ? mx_lds_words(1 << (LOGL + LOGC)) : 4;
+}
+
+// The forward pass of 2^24 points (2^11 rows, 8 columns per tile) takes 82 us
+// and the inverse 39 us, where the same addresses copied without a transform
+// take 36 and 26 us: one workgroup of 16 waves fits a CU (86 registers), so a
+// tile's loads, rounds and stores follow each other.  16 columns of 2^10 rows
+// (64-byte segments) take 71 and 34 us but leave rows of 2^14.
+//
+// Forward transforms of 2^LOGC columns: rows straight from global memory into
+// the first round (words at or beyond lim, relative to X, are zero), the last
+// round's rows straight to Y (digit-reversed rows, words below p + 4200).
+// X and Y point at the tile's first column; rows are 2^logn2 words apart.
+template <int LOGL, int LOGC, int V>
+CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const MxCtx &cx) {
+    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
+                  "a wave's 256 V words lie inside the tile");
+    using P = MxPlan<LOGL, LOGC>;
+    constexpr int C = 1 << LOGC;
+    MxMat m;
+    u32 x[1][V][4], tw[V][4];
+    mx_forward_begin<LOGL, LOGC, V>(m, tw, cx);
+    {
+        const int b = MxMap<P::words(0), V>::base();
+        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+        const u32 row = 1u << (logn2 + P::logs(0));   // words between the elements of a digit
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = (int)(off + r * row);
+            if (V == 4 && e + V <= lim) {
+                const MxQuad v = *(const MxQuad *)(X + e);
+#pragma unroll
+                for (int s = 0; s < V; ++s) x[0][s][r] = v.v[s];
+            } else {
+#pragma unroll
+                for (int s = 0; s < V; ++s) x[0][s][r] = e + s < lim ? X[e + s] : 0u;
+            }
+        }
+    }
+    u32 *const t[1] = {lds};
+    mx_forward<LOGL, LOGC, V, 0, 1>(x, t, cx, m, tw);
+    const int b = MxMap<LOGC, V>::base();
+    u32 *q = Y + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
+#pragma unroll
+    for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
+        if constexpr (V == 4) {
+            *(uint4 *)q = make_uint4(x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]);
+        } else {
+#pragma unroll
+            for (int s = 0; s < V; ++s) q[s] = x[0][s][r];
+        }
+    }
+}
+
+// The mirror: digit-reversed rows in, natural rows out (canonical, words at or
+// beyond lim not stored).
+template <int LOGL, int LOGC, int V>
+CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int lim, int logn2, const MxCtx &cx) {
+    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
+                  "a wave's 256 V words lie inside the tile");
+    using P = MxPlan<LOGL, LOGC>;
+    constexpr int C = 1 << LOGC;
+    u32 x[V][4], tw[V][4];
+    MxMat m = mx_load_mat(cx, kMxInv + P::T);
+    {
+        const int b = MxMap<LOGC, V>::base();
+        const u32 *q = X + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
+#pragma unroll
+        for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
+            if constexpr (V == 4) {
+                const uint4 v = *(const uint4 *)q;
+                x[0][r] = v.x; x[1][r] = v.y; x[2][r] = v.z; x[3][r] = v.w;
+            } else {
+#pragma unroll
+                for (int s = 0; s < V; ++s) x[s][r] = q[s];
+            }
+        }
+    }
+    mx_inverse<LOGL, LOGC, V, P::NR - 1>(x, lds, cx, m, tw);
+    const int b = MxMap<P::words(0), V>::base();
+    const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+    const u32 row = 1u << (logn2 + P::logs(0));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int e = (int)(off + r * row);
+#pragma unroll
+        for (int s = 0; s < V; ++s) x[s][r] = mx_canon(x[s][r], cx);
+        if constexpr (V == 4) {
+            if (e + V <= lim) {
+                *(MxQuad *)(Y + e) = MxQuad{{x[0][r], x[1][r], x[2][r], x[3][r]}};
+                continue;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < V; ++s)
+            if (e + s < lim) Y[e + s] = x[s][r];
+    }
+}
+
+// Words of a row tile: at least the 256 V words of a wave.
+template <int LOGL, int V>
+constexpr int mx_row_logw() { return LOGL > 8 + mx_log2(V) ? LOGL : 8 + mx_log2(V); }
+
+// Outer twiddles of a lane's words in the row of frequency f: w_n^(f i) =
+// rb[f T + v] rc[16 f + d], i = d T + v, T = 2^LOGL / 16.
+template <int LOGL, int V>
+CM_DEV void mx_outer(u32 (&tw)[V][4], const u32 *rb, const u32 *rc, int f, const MxCtx &cx) {
+    constexpr int LT = LOGL - 4;
+    const int i = MxMap<LT, V>::base() & ((1 << LOGL) - 1), v = i & ((1 << LT) - 1), d = i >> LT;
+    const u32 *pb = rb + ((int64_t)f << LT) + v;
+    const uint4 c = *(const uint4 *)(rc + 16 * f + d);
+    u32 b[V];
+    if constexpr (V == 4) {
+        const uint4 q = *(const uint4 *)pb;
+        b[0] = q.x; b[1] = q.y; b[2] = q.z; b[3] = q.w;
+    } else {
+#pragma unroll
+        for (int s = 0; s < V; ++s) b[s] = pb[s];
+    }
+    const u32 cc[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+    for (int s = 0; s < V; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tw[s][r] = cm_mont_lazy(cc[r], b[s], cx.p, cx.np);
+}
+
+// Bound by vector issue: transforms and twiddles take 2.1 of its 2.3 G lane
+// instructions at 2^24 points; 2^11 rows of 2^13 points take 87 us at four
+// sets per lane (operands one after the other, 116 registers, no spills),
+// 100 us at two, 121 us with both operands in registers at four (168 bytes of
+// scratch), and 115 us as radix-2 butterflies.
+//
+// One tile of rows of F and G (row0: its first row; the row at position
+// r mod 2^k1 holds frequency f = mx_freq(r mod 2^k1)): times the outer
+// twiddles, the multiply in LDS, and the inverse outer twiddles on the way
+// out.  In place on F.
+template <int LOGL, int V>
+CM_DEV void mx_row(u32 *lds, u32 *F, const u32 *G, int row0, int k1, const MxOuter &o,
+                   const MxCtx &cx) {
+    static_assert(LOGL - 4 >= mx_log2(V), "row");
+    using Map = MxMap<LOGL - 4, V>;
+    const int b = Map::base();
+    u32 *Fr = F + b;
+    const u32 *Gr = G + b;
+    const int f = mx_freq((row0 + (b >> LOGL)) & ((1 << k1) - 1), k1);
+    MxMat m;
+    u32 x[2][V][4], tw[V][4], ow[V][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if constexpr (V == 4) {
+            const uint4 u = *(const uint4 *)(Fr + Map::off(0, r));
+            const uint4 w = *(const uint4 *)(Gr + Map::off(0, r));
+            x[0][0][r] = u.x; x[0][1][r] = u.y; x[0][2][r] = u.z; x[0][3][r] = u.w;
+            x[1][0][r] = w.x; x[1][1][r] = w.y; x[1][2][r] = w.z; x[1][3][r] = w.w;
+        } else {
+#pragma unroll
+            for (int s = 0; s < V; ++s) {
+                x[0][s][r] = Fr[Map::off(s, r)];
+                x[1][s][r] = Gr[Map::off(s, r)];
+            }
+        }
+    }
+    mx_outer<LOGL, V>(ow, o.rb_f, o.rc_f, f, cx);
+    mx_mul<V>(x[0], ow, cx);
+    mx_mul<V>(x[1], ow, cx);
+    mx_forward_begin<LOGL, 0, V>(m, tw, cx);
+    mx_tile_multiply<LOGL, V>(x, lds, lds + mx_lds_words(1 << mx_row_logw<LOGL, V>()), cx, m, tw);
+    mx_outer<LOGL, V>(ow, o.rb_i, o.rc_i, f, cx);
+    mx_mul<V>(x[0], ow, cx);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if constexpr (V == 4) {
+            *(uint4 *)(Fr + Map::off(0, r)) =
+                make_uint4(x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]);
+        } else {
+#pragma unroll
+            for (int s = 0; s < V; ++s) Fr[Map::off(s, r)] = x[0][s][r];
+        }
+    }
+}
+
+}  // namespace cm

@@ -2,7 +2,7 @@
 #include <algorithm>
 
 #include "internal.h"
-#include "ntt_mx.h"
+#include "mul_mx.h"
 
 namespace cm {
 
@@ -140,11 +140,6 @@ hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, 
 // ---------------------------------------------------------------------------
 // four-step multiply: an n-word array viewed as 2^k1 rows x 2^k2 columns
 // ---------------------------------------------------------------------------
-// Workgroups are dispatched round-robin over the 8 XCDs; give each XCD a
-// contiguous range of logical blocks so that neighbouring column tiles (which
-// share 128-byte lines) meet in the same L2.
-CM_DEV int mx_xcd(int b, int nb) { return nb & 7 ? b : (b & 7) * (nb >> 3) + (b >> 3); }
-
 // One set of arrays of the column passes: array a reads in[a in_stride + e]
 // for e < in_len (zero beyond) and writes out[a out_stride + e], e < out_len.
 struct MxCols {
@@ -153,228 +148,41 @@ struct MxCols {
     int64_t in_stride, in_len, out_stride, out_len;
 };
 
-// The forward pass of 2^24 points (2^11 rows, 8 columns per tile) takes 82 us
-// and the inverse 39 us, where the same addresses copied without a transform
-// take 36 and 26 us: one workgroup of 16 waves fits a CU (86 registers), so a
-// tile's loads, rounds and stores follow each other.  16 columns of 2^10 rows
-// (64-byte segments) take 71 and 34 us but leave rows of 2^14.
-//
-// Forward column transforms of 2^LOGC columns per workgroup: rows straight
-// from global memory into the first round, the last round's rows straight
-// back (digit-reversed rows, words below p + 4200).  grid.y: arrays, the
-// first cnt0 from set s0, the rest from s1.
+// Forward column transforms of 2^LOGC columns per workgroup (mx_col_fwd).
+// grid.y: arrays, the first cnt0 from set s0, the rest from s1.
 template <int LOGL, int LOGC, int V>
 __global__ __launch_bounds__((1 << (LOGL + LOGC)) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_fwd_mx(MxCols s0, MxCols s1, int cnt0,
                                                              int logn2, MxCtx cx) {
-    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
-                  "a wave's 256 V words lie inside the tile");
-    using P = MxPlan<LOGL, LOGC>;
-    constexpr int W = 1 << (LOGL + LOGC), C = 1 << LOGC;
-    __shared__ __align__(16) u32 lds[P::NR > 1 ? mx_lds_words(W) : 4];
+    __shared__ __align__(16) u32 lds[mx_col_lds<LOGL, LOGC>()];
     const int y = blockIdx.y;
     const MxCols &S = y < cnt0 ? s0 : s1;
     const int64_t a = y < cnt0 ? y : y - cnt0;
-    const int c0 = mx_xcd(blockIdx.x, gridDim.x) * C;
-    const u32 *X = S.in + a * S.in_stride + c0;
-    u32 *Y = S.out + a * S.out_stride + c0;
-    MxMat m;
-    u32 x[1][V][4], tw[V][4];
-    mx_forward_begin<LOGL, LOGC, V>(m, tw, cx);
-    {
-        using Map = MxMap<P::words(0), V>;
-        const int b = Map::base();
-        const int lim = (int)(S.in_len - c0);
-        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
-        const u32 row = 1u << (logn2 + P::logs(0));   // words between the elements of a digit
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = (int)(off + r * row);
-            if (e + V <= lim) {
-                const u32 *q = X + e;
-                if constexpr (V >= 4) {
-#pragma unroll
-                    for (int s = 0; s < V; s += 4) {
-                        const MxQuad v = *(const MxQuad *)(q + s);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) x[0][s + j][r] = v.v[j];
-                    }
-                } else {
-#pragma unroll
-                    for (int s = 0; s < V; ++s) x[0][s][r] = q[s];
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < V; ++s) x[0][s][r] = e + s < lim ? X[e + s] : 0u;
-            }
-        }
-    }
-    u32 *const t[1] = {lds};
-    mx_forward<LOGL, LOGC, V, 0, 1>(x, t, cx, m, tw);
-    {
-        using Map = MxMap<LOGC, V>;
-        const int b = Map::base();
-        u32 *q = Y + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
-#pragma unroll
-        for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
-            if constexpr (V >= 4) {
-#pragma unroll
-                for (int s = 0; s < V; s += 4)
-                    *(uint4 *)(q + s) =
-                        make_uint4(x[0][s][r], x[0][s + 1][r], x[0][s + 2][r], x[0][s + 3][r]);
-            } else {
-#pragma unroll
-                for (int s = 0; s < V; ++s) q[s] = x[0][s][r];
-            }
-        }
-    }
+    const int c0 = mx_xcd(blockIdx.x, gridDim.x) << LOGC;
+    mx_col_fwd<LOGL, LOGC, V>(lds, S.in + a * S.in_stride + c0, (int)(S.in_len - c0),
+                              S.out + a * S.out_stride + c0, logn2, cx);
 }
 
-// Inverse column transforms, the mirror: digit-reversed rows in, natural rows
-// out (canonical, truncated to out_len).
+// Inverse column transforms (mx_col_inv), truncated to out_len.
 template <int LOGL, int LOGC, int V>
 __global__ __launch_bounds__((1 << (LOGL + LOGC)) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_inv_mx(MxCols S, int logn2, MxCtx cx) {
-    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
-                  "a wave's 256 V words lie inside the tile");
-    using P = MxPlan<LOGL, LOGC>;
-    constexpr int W = 1 << (LOGL + LOGC), C = 1 << LOGC;
-    __shared__ __align__(16) u32 lds[P::NR > 1 ? mx_lds_words(W) : 4];
+    __shared__ __align__(16) u32 lds[mx_col_lds<LOGL, LOGC>()];
     const int64_t a = blockIdx.y;
-    const int c0 = mx_xcd(blockIdx.x, gridDim.x) * C;
-    const u32 *X = S.in + a * S.in_stride + c0;
-    u32 *Y = S.out + a * S.out_stride + c0;
-    u32 x[V][4], tw[V][4];
-    MxMat m = mx_load_mat(cx, kMxInv + P::T);
-    {
-        using Map = MxMap<LOGC, V>;
-        const int b = Map::base();
-        const u32 *q = X + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
-#pragma unroll
-        for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
-            if constexpr (V >= 4) {
-#pragma unroll
-                for (int s = 0; s < V; s += 4) {
-                    const uint4 v = *(const uint4 *)(q + s);
-                    x[s][r] = v.x; x[s + 1][r] = v.y; x[s + 2][r] = v.z; x[s + 3][r] = v.w;
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < V; ++s) x[s][r] = q[s];
-            }
-        }
-    }
-    mx_inverse<LOGL, LOGC, V, P::NR - 1>(x, lds, cx, m, tw);
-    {
-        using Map = MxMap<P::words(0), V>;
-        const int b = Map::base();
-        const int lim = (int)(S.out_len - c0);
-        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
-        const u32 row = 1u << (logn2 + P::logs(0));
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = (int)(off + r * row);
-#pragma unroll
-            for (int s = 0; s < V; ++s) x[s][r] = mx_canon(x[s][r], cx);
-            if (V >= 4 && e + V <= lim) {
-#pragma unroll
-                for (int s = 0; s + 3 < V; s += 4)
-                    *(MxQuad *)(Y + e + s) =
-                        MxQuad{{x[s][r], x[s + 1][r], x[s + 2][r], x[s + 3][r]}};
-            } else {
-#pragma unroll
-                for (int s = 0; s < V; ++s)
-                    if (e + s < lim) Y[e + s] = x[s][r];
-            }
-        }
-    }
+    const int c0 = mx_xcd(blockIdx.x, gridDim.x) << LOGC;
+    mx_col_inv<LOGL, LOGC, V>(lds, S.in + a * S.in_stride + c0, S.out + a * S.out_stride + c0,
+                              (int)(S.out_len - c0), logn2, cx);
 }
 
-// Bound by vector issue: 2.1 G of its 2.3 G lane instructions of 2^24 points
-// are transforms and twiddles; 2^11 rows of 2^13 points take 87 us at four
-// sets per lane (operands one after the other, 116 registers, no spills),
-// 100 us at two, 121 us with both operands in registers at four (168 bytes of
-// scratch), and 115 us as radix-2 butterflies.
-// Row pass: row r (array r >> k1, position r mod 2^k1 holding frequency
-// f = mx_freq(r mod 2^k1)) of F and G times the outer twiddles w_n^(f i) =
-// rb[f T + v] rc[16 f + d] (i = d T + v, T = 2^LOGL / 16), the multiply in
-// LDS, and the inverse outer twiddles on the way out.  In place on F.
-template <int LOGL, int V>
-constexpr int mx_row_logw() { return LOGL > 8 + mx_log2(V) ? LOGL : 8 + mx_log2(V); }
-
-template <int LOGL, int V>
-CM_DEV void mx_outer(u32 (&tw)[V][4], const u32 *rb, const u32 *rc, int f, const MxCtx &cx) {
-    constexpr int LT = LOGL - 4;
-    using Map = MxMap<LT, V>;
-    const int i = Map::base() & ((1 << LOGL) - 1), v = i & ((1 << LT) - 1), d = i >> LT;
-    const u32 *pb = rb + ((int64_t)f << LT) + v;
-    const uint4 c = *(const uint4 *)(rc + 16 * f + d);
-    u32 b[V];
-    if constexpr (V == 4) {
-        const uint4 q = *(const uint4 *)pb;
-        b[0] = q.x; b[1] = q.y; b[2] = q.z; b[3] = q.w;
-    } else {
-#pragma unroll
-        for (int s = 0; s < V; ++s) b[s] = pb[s];
-    }
-    const u32 cc[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-    for (int s = 0; s < V; ++s)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) tw[s][r] = cm_mont_lazy(cc[r], b[s], cx.p, cx.np);
-}
-
+// Row pass (mx_row) over all rows of cnt arrays, in place on F.
 template <int LOGL, int V>
 __global__ __launch_bounds__((1 << mx_row_logw<LOGL, V>()) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_row_mx(u32 *F, const u32 *__restrict__ G, int k1,
-                                                         const u32 *__restrict__ rb,
-                                                         const u32 *__restrict__ rc,
-                                                         const u32 *__restrict__ rbi,
-                                                         const u32 *__restrict__ rci, MxCtx cx) {
-    static_assert(LOGL - 4 >= mx_log2(V), "row");
-    constexpr int LOGW = mx_row_logw<LOGL, V>(), W = 1 << LOGW, LW = mx_lds_words(W);
-    __shared__ __align__(16) u32 lds[2 * LW];
-    using Map = MxMap<LOGL - 4, V>;
-    const int b = Map::base();
+                                                         MxOuter o, MxCtx cx) {
+    constexpr int LOGW = mx_row_logw<LOGL, V>();
+    __shared__ __align__(16) u32 lds[2 * mx_lds_words(1 << LOGW)];
     const int64_t t0 = (int64_t)blockIdx.x << LOGW;
-    u32 *Fr = F + t0 + b;
-    const u32 *Gr = G + t0 + b;
-    const int row = (int)(blockIdx.x << (LOGW - LOGL)) + (b >> LOGL);
-    const int f = mx_freq(row & ((1 << k1) - 1), k1);
-    MxMat m;
-    u32 x[2][V][4], tw[V][4], ow[V][4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if constexpr (V == 4) {
-            const uint4 u = *(const uint4 *)(Fr + Map::off(0, r));
-            const uint4 w = *(const uint4 *)(Gr + Map::off(0, r));
-            x[0][0][r] = u.x; x[0][1][r] = u.y; x[0][2][r] = u.z; x[0][3][r] = u.w;
-            x[1][0][r] = w.x; x[1][1][r] = w.y; x[1][2][r] = w.z; x[1][3][r] = w.w;
-        } else {
-#pragma unroll
-            for (int s = 0; s < V; ++s) {
-                x[0][s][r] = Fr[Map::off(s, r)];
-                x[1][s][r] = Gr[Map::off(s, r)];
-            }
-        }
-    }
-    mx_outer<LOGL, V>(ow, rb, rc, f, cx);
-    mx_mul<V>(x[0], ow, cx);
-    mx_mul<V>(x[1], ow, cx);
-    mx_forward_begin<LOGL, 0, V>(m, tw, cx);
-    mx_tile_multiply<LOGL, V>(x, lds, lds + LW, cx, m, tw);
-    mx_outer<LOGL, V>(ow, rbi, rci, f, cx);
-    mx_mul<V>(x[0], ow, cx);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if constexpr (V == 4) {
-            *(uint4 *)(Fr + Map::off(0, r)) =
-                make_uint4(x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]);
-        } else {
-#pragma unroll
-            for (int s = 0; s < V; ++s) Fr[Map::off(s, r)] = x[0][s][r];
-        }
-    }
+    mx_row<LOGL, V>(lds, F + t0, G + t0, (int)(blockIdx.x << (LOGW - LOGL)), k1, o, cx);
 }
 
 template <int LOGL, int LOGC, int V>
@@ -453,8 +261,8 @@ static hipError_t rows_t(const FourStepIO &io, const Outer *o, const Family *fam
     ProfScope ps(kProfRowMul, s);
     const int64_t words = (int64_t)io.cnt << o->k;
     hipLaunchKernelGGL((k_row_mx<LOGL, V>), dim3((unsigned)(words >> LOGW)),
-                       dim3((1 << LOGW) / (4 * V)), 0, s, io.f_ws, io.g_ws, o->k1, o->rb_f,
-                       o->rc_f, o->rb_i, o->rc_i, mx_ctx(fam));
+                       dim3((1 << LOGW) / (4 * V)), 0, s, io.f_ws, io.g_ws, o->k1,
+                       mx_outer_of(o), mx_ctx(fam));
     return hipGetLastError();
 }
 

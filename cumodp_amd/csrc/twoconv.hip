@@ -164,52 +164,78 @@ __global__ void k_tc_split(const u64 *__restrict__ src, const TcDesc *__restrict
     }
 }
 
-// k_tc_split for one-word coefficients fused with the forward x transform,
-// for both operands and every prime in one launch (grid.z = 2 q + which):
-// thread i forms the K = 2^LK2 / 2 limbs of coefficient i of operand
-// `which` (upper K2 - K limbs zero), runs the natural-order length-K2 DFT
-// on them in registers (DIF stages with prime q's x-root level table, zero
-// upper half) and writes out[q][which][(k R + r) Ly + i] = DFT_k for every
-// k < K2.  Positions i >= n are zero rows.
-struct TcFwdX {
-    const u32 *lv[3];   // x root's level tables, per prime
-    u32 p[3], np[3];
-    u32 *out[3][2];     // A and B arrays of each prime
+// One class of products in the fused form (one-word coefficients, 2K <= 8):
+// rows of item r and x-point k at out[q][operand] + (k R + r) 2^ey, and per
+// prime the tables of the x transforms.
+struct TcCls {
+    u32 *out[3][2];
+    const u32 *lvf[3], *lvi[3];   // level tables of the x root and its inverse
+    u32 p[3], np[3], ki[3];       // modulus, -p^-1 mod 2^32, Montgomery form of 1 / 2K
+    int lk2, nprimes, M, ey, R, first;   // first: its first item among the descriptors
+    int len[2];                   // words of a row that are written (longest operand)
 };
 
+// One block of work: positions from start of operand `which` (split) or of
+// the product (CRT) of item `item` (counted within the class).
+struct TcBlock {
+    int cls, item, which, start;
+};
+
+// k_tc_split for one-word coefficients fused with the forward x transform:
+// thread i forms the K limbs of coefficient i (upper K limbs zero) once, runs
+// the natural-order length-2K DFT on them in registers for every prime (DIF
+// stages, zero upper half) and writes the 2K words.  Positions from the item's
+// length to the class's longest are zero rows.
 template <int LK2>
-__global__ void k_tc_split_x(const u64 *__restrict__ A, const u64 *__restrict__ B,
-                             const TcDesc *__restrict__ d, TcDesc one, int M, TcFwdX fx,
-                             int64_t Ly, int R) {
+CM_DEV void tc_split_block(const TcCls &c, const u64 *a, int n, int r, int which, int start,
+                           int span) {
     constexpr int K2 = 1 << LK2, K = K2 / 2;
-    const int r = blockIdx.y, q = blockIdx.z >> 1, which = blockIdx.z & 1;
-    const TcDesc dd = d ? d[r] : one;
-    const u64 *a = which ? B + dd.b_off : A + dd.a_off;
-    const int64_t n = which ? dd.nb : dd.na;
-    u32 *o = fx.out[q][which] + (int64_t)r * Ly;
-    const int64_t js = (int64_t)R * Ly;
-    const u64 mask = (1ull << M) - 1;
-    const Mod md{fx.p[q], fx.np[q]};
-    const u32 *lvx = fx.lv[q];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < Ly;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        u32 v[1][K2];
+    const int64_t js = (int64_t)c.R << c.ey;
+    const u64 mask = (1ull << c.M) - 1;
+    const int end = min(start + span, c.len[which]);
+    for (int i = start + threadIdx.x; i < end; i += blockDim.x) {
+        const u64 x = i < n ? a[i] : 0;
+        const bool neg = (int64_t)x < 0;
+        const u64 mag = neg ? ~x + 1 : x;                // |x| (2^63 for the minimum)
+        u32 limb[K];
 #pragma unroll
-        for (int j = 0; j < K2; ++j) v[0][j] = 0u;
-        if (i < n) {
-            const u64 x = a[i];
-            const bool neg = (int64_t)x < 0;
-            const u64 mag = neg ? ~x + 1 : x;            // |x| (2^63 for the minimum)
+        for (int j = 0; j < K; ++j) {
+            const int sh = j * c.M;
+            limb[j] = sh < 64 ? (u32)((mag >> sh) & mask) : 0u;
+        }
+        for (int q = 0; q < c.nprimes; ++q) {
+            const Mod md{c.p[q], c.np[q]};
+            u32 v[1][K2];
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                const int sh = j * M;
-                const u32 limb = sh < 64 ? (u32)((mag >> sh) & mask) : 0u;
-                v[0][j] = neg ? (limb ? md.p - limb : 0u) : limb;
+                v[0][j] = neg ? (limb[j] ? md.p - limb[j] : 0u) : limb[j];
+                v[0][K + j] = 0u;
             }
-        }
-        cm_dif_stages<LK2, LK2, 0, 0, 1, true>(v, 0, lvx, md);
+            cm_dif_stages<LK2, LK2, 0, 0, 1, true>(v, 0, c.lvf[q], md);
+            u32 *o = c.out[q][which] + ((int64_t)r << c.ey) + i;
 #pragma unroll
-        for (int m = 0; m < K2; ++m) o[(int64_t)cm_brev((u32)m, LK2) * js + i] = v[0][m];
+            for (int m = 0; m < K2; ++m) o[(int64_t)cm_brev((u32)m, LK2) * js] = v[0][m];
+        }
+    }
+}
+
+// blocks: the work of each workgroup (null: class `one`, item 0, operand
+// blockIdx.y, span positions per workgroup); d: descriptors (null: `od`).
+__global__ __launch_bounds__(256) void k_tc_split_x(const u64 *__restrict__ A,
+                                                    const u64 *__restrict__ B,
+                                                    const TcDesc *__restrict__ d, TcDesc od,
+                                                    const TcCls *__restrict__ cls, TcCls one,
+                                                    const TcBlock *__restrict__ blocks, int span) {
+    const TcBlock t = blocks ? blocks[blockIdx.x]
+                             : TcBlock{0, 0, (int)blockIdx.y, (int)blockIdx.x * span};
+    const TcCls &c = cls ? cls[t.cls] : one;
+    const TcDesc dd = d ? d[c.first + t.item] : od;
+    const u64 *a = t.which ? B + dd.b_off : A + dd.a_off;
+    const int n = (int)(t.which ? dd.nb : dd.na);
+    switch (c.lk2) {
+    case 1: tc_split_block<1>(c, a, n, t.item, t.which, t.start, span); break;
+    case 2: tc_split_block<2>(c, a, n, t.item, t.which, t.start, span); break;
+    default: tc_split_block<3>(c, a, n, t.item, t.which, t.start, span); break;
     }
 }
 
@@ -218,28 +244,29 @@ struct TcCrt {
     u32 p0, p1, p2, inv01, inv01q, inv012, inv012q, p0m2, p0m2q;
 };
 
+// The signed CRT value (in (-P/2, P/2]) of the residues r0, r1 (, r2).  Each
+// prime exceeds half of every other, so one conditional subtraction takes a
+// residue of one into the range of another (p0 < p1 needs none).
+template <int NP>
+__device__ __forceinline__ __int128 tc_crt_value(u32 r0, u32 r1, u32 r2, const TcCrt &k) {
+    // Garner: t1 = (r1 - r0) p0^-1 mod p1;  z = r0 + p0 t1 (+ p0 p1 t2)
+    const u32 t1 = cm_shoup(cm_sub(r1, r0, k.p1), k.inv01, k.inv01q, k.p1);
+    const u64 z2 = (u64)k.p0 * t1 + r0, P2 = (u64)k.p0 * k.p1;
+    if (NP == 2) return z2 > P2 / 2 ? (__int128)z2 - (__int128)P2 : (__int128)z2;
+    // t2 = (r2 - (r0 + p0 t1)) (p0 p1)^-1 mod p2
+    const u32 zm = cm_add(cm_reduce2p(r0, k.p2),
+                          cm_shoup(cm_reduce2p(t1, k.p2), k.p0m2, k.p0m2q, k.p2), k.p2);
+    const u32 t2 = cm_shoup(cm_sub(r2, zm, k.p2), k.inv012, k.inv012q, k.p2);
+    const unsigned __int128 z = (unsigned __int128)P2 * t2 + z2, P = (unsigned __int128)P2 * k.p2;
+    return z > P / 2 ? (__int128)z - (__int128)P : (__int128)z;
+}
+
 // Adds z 2^sh to the wc-word two's-complement accumulator o, where z is the
-// signed CRT value (in (-P/2, P/2]) of the residues r0, r1 (, r2).
+// CRT value of the residues r0, r1 (, r2).
 template <int NP>
 __device__ __forceinline__ void tc_crt_add(u64 *o, int wc, int sh, u32 r0, u32 r1, u32 r2,
                                            const TcCrt &k) {
-    // Garner: t1 = (r1 - r0) p0^-1 mod p1;  z = r0 + p0 t1 (+ p0 p1 t2)
-    const u32 d1 = cm_sub(r1, r0 % k.p1, k.p1);
-    const u32 t1 = cm_shoup(d1, k.inv01, k.inv01q, k.p1);
-    unsigned __int128 z = (unsigned __int128)r0 + (unsigned __int128)k.p0 * t1;
-    unsigned __int128 P = (unsigned __int128)k.p0 * k.p1;
-    if (NP == 3) {
-        // t2 = (r2 - (r0 + p0 t1)) (p0 p1)^-1 mod p2
-        const u32 zm =
-            (u32)(((u64)(r0 % k.p2) + cm_shoup(t1 % k.p2, k.p0m2, k.p0m2q, k.p2)) % k.p2);
-        const u32 d2 = cm_sub(r2, zm, k.p2);
-        const u32 t2 = cm_shoup(d2, k.inv012, k.inv012q, k.p2);
-        z += P * t2;
-        P *= k.p2;
-    }
-    // signed value in (-P/2, P/2]
-    __int128 sz = (__int128)z;
-    if (z > P / 2) sz -= (__int128)P;
+    const __int128 sz = tc_crt_value<NP>(r0, r1, r2, k);
     if (sz == 0) return;
     // add sz << sh into the wc-word accumulator
     const int w0 = sh >> 6, b0 = sh & 63;
@@ -296,48 +323,77 @@ __global__ void k_tc_crt(const u32 *__restrict__ C0, const u32 *__restrict__ C1,
     }
 }
 
-// Inverse x transforms of the residues of each prime (natural-order length-K2
-// DFT with the inverse root's level table, times 1/K2) fused with the CRT
-// and recombination: thread y loads C_q[(k R + r) Ly + y] for k < K2 and
-// prime q, transforms them in registers, then adds z_j 2^(M j) for
-// j < K2 - 1 as k_tc_crt does.
-struct TcInvX {
-    const u32 *lv[3];   // inverse x root's level tables, per prime
-    u32 np[3];          // -p^-1 mod 2^32, per prime
-    u32 ki[3];          // Montgomery form of 1 / K2, per prime
-};
-
+// Inverse x transforms of the residues of each prime (natural-order length-2K
+// DFT with the inverse root's level table, times 1/2K) fused with the CRT and
+// recombination of output coefficient y: sum_j z_j 2^(M j), j < 2K - 1, in four
+// words of registers (one-word operands: the sum has at most 2 64 + 32 + 1
+// bits), sign-extended to the wc words of the output.
 template <int NP, int LK2>
-__global__ void k_tc_crt_x(const u32 *__restrict__ C0, const u32 *__restrict__ C1,
-                           const u32 *__restrict__ C2, const TcDesc *__restrict__ d, TcDesc one,
-                           int M, int64_t Ly, int R, u64 *__restrict__ out, TcCrt k, TcInvX ix) {
+CM_DEV void tc_crt_block(const TcCls &c, const TcDesc &dd, u64 *out, int r, int start, int span,
+                         const TcCrt &k) {
     constexpr int K2 = 1 << LK2;
-    const int r = blockIdx.y;
-    const TcDesc dd = d ? d[r] : one;
+    const int64_t js = (int64_t)c.R << c.ey, base = (int64_t)r << c.ey;
     const int64_t ny = dd.na + dd.nb - 1;
+    const int end = (int)(ny < start + span ? ny : start + span);
     const int wc = dd.wc;
-    const int64_t js = (int64_t)R * Ly, base = (int64_t)r * Ly;
-    const u32 ps[3] = {k.p0, k.p1, k.p2};
-    const u32 *Cs[3] = {C0, C1, C2};
-    for (int64_t y = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; y < ny;
-         y += (int64_t)gridDim.x * blockDim.x) {
+    for (int y = start + threadIdx.x; y < end; y += blockDim.x) {
         u32 res[NP][K2];
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
+            const u32 *C = c.out[q][0] + base + y;
             u32 v[1][K2];
 #pragma unroll
-            for (int j = 0; j < K2; ++j) v[0][j] = Cs[q][j * js + base + y];
-            const Mod md{ps[q], ix.np[q]};
-            cm_dif_stages<LK2, LK2, 0, 0, 1>(v, 0, ix.lv[q], md);
+            for (int j = 0; j < K2; ++j) v[0][j] = C[j * js];
+            const Mod md{c.p[q], c.np[q]};
+            cm_dif_stages<LK2, LK2, 0, 0, 1>(v, 0, c.lvi[q], md);
 #pragma unroll
             for (int j = 0; j < K2; ++j)
-                res[q][j] = cm_mul_tw(v[0][cm_brev((u32)j, LK2)], ix.ki[q], md.p, md.np);
+                res[q][j] = cm_mul_tw(v[0][cm_brev((u32)j, LK2)], c.ki[q], md.p, md.np);
         }
-        u64 *o = out + dd.c_off + y * wc;
-        for (int q = 0; q < wc; ++q) o[q] = 0;
+        u64 acc[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < K2 - 1; ++j)
-            tc_crt_add<NP>(o, wc, M * j, res[0][j], res[1][j], NP == 3 ? res[2][j] : 0u, k);
+        for (int j = 0; j < K2 - 1; ++j) {
+            const __int128 z = tc_crt_value<NP>(res[0][j], res[1][j], NP == 3 ? res[2][j] : 0u, k);
+            const int sh = c.M * j, w0 = sh >> 6, b0 = sh & 63;   // uniform
+            const u64 sign = (u64)(int64_t)(z >> 127);
+            const unsigned __int128 lo = (unsigned __int128)z << b0;
+            const u64 part[3] = {(u64)lo, (u64)(lo >> 64),
+                                 b0 ? (u64)((unsigned __int128)z >> 64) >> (64 - b0) | sign << b0
+                                    : sign};
+            u64 carry = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u64 w = q < w0 ? 0 : (q == w0 ? part[0]
+                                                    : (q == w0 + 1 ? part[1]
+                                                                   : (q == w0 + 2 ? part[2] : sign)));
+                const u64 t = acc[q] + w, u = t + carry;
+                carry = (u64)(t < w) | (u64)(u < t);
+                acc[q] = u;
+            }
+        }
+        u64 *o = out + dd.c_off + (int64_t)y * wc;
+        const u64 top = (u64)((int64_t)acc[3] >> 63);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (q < wc) o[q] = acc[q];
+        for (int q = 4; q < wc; ++q) o[q] = top;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_tc_crt_x(const TcDesc *__restrict__ d, TcDesc od,
+                                                  const TcCls *__restrict__ cls, TcCls one,
+                                                  const TcBlock *__restrict__ blocks, int span,
+                                                  u64 *__restrict__ out, TcCrt k) {
+    const TcBlock t = blocks ? blocks[blockIdx.x] : TcBlock{0, 0, 0, (int)blockIdx.x * span};
+    const TcCls &c = cls ? cls[t.cls] : one;
+    const TcDesc dd = d ? d[c.first + t.item] : od;
+    switch (c.nprimes * 4 + c.lk2) {
+    case 9: tc_crt_block<2, 1>(c, dd, out, t.item, t.start, span, k); break;
+    case 10: tc_crt_block<2, 2>(c, dd, out, t.item, t.start, span, k); break;
+    case 11: tc_crt_block<2, 3>(c, dd, out, t.item, t.start, span, k); break;
+    case 13: tc_crt_block<3, 1>(c, dd, out, t.item, t.start, span, k); break;
+    case 14: tc_crt_block<3, 2>(c, dd, out, t.item, t.start, span, k); break;
+    default: tc_crt_block<3, 3>(c, dd, out, t.item, t.start, span, k); break;
     }
 }
 
@@ -360,10 +416,6 @@ static int blocks_for(int64_t n, int t = 256) {
 // ---------------------------------------------------------------------------
 // host driver
 // ---------------------------------------------------------------------------
-struct TcWorkspace {
-    u32 *rows = nullptr;   // per prime: A (2K x Ly) then B (2K x Ly)
-};
-
 int tc_bit_width(const u64 *a, int64_t n, int w) {
     int best = 1;
     std::vector<u64> mag((size_t)w);
@@ -386,50 +438,48 @@ int tc_bit_width(const u64 *a, int64_t n, int w) {
     return best;
 }
 
+static TcCrt tc_crt_consts() {
+    const u32 p0 = kTcPrimes[0], p1 = kTcPrimes[1], p2 = kTcPrimes[2];
+    const u32 inv01 = cm_host_inv(p0 % p1, p1);
+    const u32 p0m2 = p0 % p2;
+    const u32 inv012 = cm_host_inv(cm_host_mul(p0 % p2, p1 % p2, p2), p2);
+    return TcCrt{p0, p1, p2, inv01, cm_host_shoup_q(inv01, p1), inv012,
+                 cm_host_shoup_q(inv012, p2), p0m2, cm_host_shoup_q(p0m2, p2)};
+}
+
+// The families of prime q's x transforms of 2^lk2 points (forward and inverse
+// root).
+static hipError_t tc_x_families(int q, int lk2, const Family *&fam, const Family *&fx,
+                                const Family *&fxi) {
+    const u32 p = kTcPrimes[q];
+    fam = family_default(p);
+    if (!fam) return hipErrorOutOfMemory;
+    const u32 wx = cm_host_pow(fam->wN, (u64)1 << (fam->K - lk2), p);
+    fx = family_for_root(p, wx, lk2);
+    fxi = family_for_root(p, cm_host_inv(wx, p), lk2);
+    return fx && fxi ? hipSuccess : hipErrorOutOfMemory;
+}
+
 // The products of one class (same plan and y size) over R items: per prime,
 // A and B are 2K x R x Ly (limb row j of item r at (j R + r) Ly), so the x
 // transforms are column transforms over R Ly columns and the y products are
-// 2K R rows of Ly words.  d: device descriptors, or null with `one`.  w1:
-// every coefficient of the class is one word; then, for 2K <= 8, the x
-// transforms run inside the split and CRT kernels (k_tc_split_x,
-// k_tc_crt_x) instead of as three column passes per prime.
+// 2K R rows of Ly words.  d: device descriptors, or null with `one`.
 static hipError_t tc_run_class(const TcPlan &pl, const u64 *A, const u64 *B, u64 *C,
-                               const TcDesc *d, const TcDesc &one, int R, int64_t ymax, bool w1,
-                               u32 *ws, hipStream_t s) {
+                               const TcDesc *d, const TcDesc &one, int R, int64_t ymax, u32 *ws,
+                               hipStream_t s) {
     const int K2 = 1 << pl.lk2;
     const int64_t Ly = (int64_t)1 << pl.ey;
     const size_t per = (size_t)2 * K2 * R * Ly;   // A and B rows of one prime
     const int bx = blocks_for(Ly);
-    const bool fused = w1 && pl.lk2 >= 1 && pl.lk2 <= 3;   // 2K = 16 would spill in the CRT
     u32 *Cr[3] = {nullptr, nullptr, nullptr};
-    TcInvX ix{};
-    TcFwdX fw{};
-    const Family *fams[3] = {nullptr, nullptr, nullptr};
     for (int q = 0; q < pl.np; ++q) {
         const u32 p = kTcPrimes[q];
-        const Family *fam = family_default(p);
-        if (!fam) return hipErrorOutOfMemory;
-        fams[q] = fam;
+        const Family *fam, *fx, *fxi;
+        hipError_t e = tc_x_families(q, pl.lk2, fam, fx, fxi);
+        if (e != hipSuccess) return e;
         u32 *Aq = ws + per * q, *Bq = Aq + (size_t)K2 * R * Ly;
         Cr[q] = Aq;
-        // x: length-2K DFT down the columns (cyclic points even, negacyclic odd)
-        const u32 wx = cm_host_pow(fam->wN, (u64)1 << (fam->K - pl.lk2), p);
-        const Family *fx = family_for_root(p, wx, pl.lk2);
-        const Family *fxi = family_for_root(p, cm_host_inv(wx, p), pl.lk2);
-        if (!fx || !fxi) return hipErrorOutOfMemory;
         const u32 ki = cm_host_inv((u32)K2, p);
-        if (fused) {
-            fw.lv[q] = fx->lv;
-            fw.p[q] = p;
-            fw.np[q] = fam->np;
-            fw.out[q][0] = Aq;
-            fw.out[q][1] = Bq;
-            ix.lv[q] = fxi->lv;
-            ix.np[q] = fam->np;
-            ix.ki[q] = cm_host_mont(ki, p);
-            continue;
-        }
-        hipError_t e;
         {
             ProfScope ps(kProfTcSplit, s);
             hipLaunchKernelGGL(k_tc_split, dim3(bx, R), dim3(256), 0, s, A, d, one, 0, pl.K, K2,
@@ -438,6 +488,7 @@ static hipError_t tc_run_class(const TcPlan &pl, const u64 *A, const u64 *B, u64
                                pl.M, p, Bq, Ly, R);
         }
         e = hipGetLastError();
+        // x: length-2K DFT down the columns (cyclic points even, negacyclic odd)
         if (e == hipSuccess) e = launch_col_ntt(pl.lk2, Aq, (int64_t)R * Ly, 1u, fx, s);
         if (e == hipSuccess) e = launch_col_ntt(pl.lk2, Bq, (int64_t)R * Ly, 1u, fx, s);
         // y: 2K R independent cyclic products of length Ly (= linear: ny <= Ly)
@@ -446,59 +497,52 @@ static hipError_t tc_run_class(const TcPlan &pl, const u64 *A, const u64 *B, u64
         if (e == hipSuccess) e = launch_col_ntt(pl.lk2, Aq, (int64_t)R * Ly, ki, fxi, s);
         if (e != hipSuccess) return e;
     }
-    if (fused) {
-        // both operands of every prime split and transformed in one launch,
-        // then the y products prime by prime
-        {
-            ProfScope ps(kProfTcSplit, s);
-            const dim3 g(bx, R, 2 * pl.np);
-            if (pl.lk2 == 1)
-                hipLaunchKernelGGL(k_tc_split_x<1>, g, dim3(256), 0, s, A, B, d, one, pl.M, fw, Ly, R);
-            else if (pl.lk2 == 2)
-                hipLaunchKernelGGL(k_tc_split_x<2>, g, dim3(256), 0, s, A, B, d, one, pl.M, fw, Ly, R);
-            else
-                hipLaunchKernelGGL(k_tc_split_x<3>, g, dim3(256), 0, s, A, B, d, one, pl.M, fw, Ly, R);
-        }
-        hipError_t e = hipGetLastError();
-        for (int q = 0; q < pl.np && e == hipSuccess; ++q)
-            e = launch_rows_mul(pl.ey, fw.out[q][0], fw.out[q][1], K2 * R, fams[q], s);
-        if (e != hipSuccess) return e;
-    }
-    const u32 p0 = kTcPrimes[0], p1 = kTcPrimes[1], p2 = kTcPrimes[2];
-    const u32 inv01 = cm_host_inv(p0 % p1, p1);
-    const u32 p0m2 = p0 % p2;
-    const u32 inv012 = cm_host_inv(cm_host_mul(p0 % p2, p1 % p2, p2), p2);
-    const TcCrt kc{p0, p1, p2, inv01, cm_host_shoup_q(inv01, p1), inv012,
-                   cm_host_shoup_q(inv012, p2), p0m2, cm_host_shoup_q(p0m2, p2)};
     ProfScope ps(kProfTcCrt, s);
     const dim3 g(blocks_for(ymax), R);
+    const TcCrt kc = tc_crt_consts();
     const u32 *C2 = pl.np == 3 ? Cr[2] : Cr[1];
-    if (fused) {
-#define CM_CX(NP, L)                                                                        \
-    hipLaunchKernelGGL((k_tc_crt_x<NP, L>), g, dim3(256), 0, s, Cr[0], Cr[1], C2, d, one, pl.M, \
-                       Ly, R, C, kc, ix)
-        if (pl.np == 2) {
-            switch (pl.lk2) {
-            case 1: CM_CX(2, 1); break;
-            case 2: CM_CX(2, 2); break;
-            default: CM_CX(2, 3); break;
-            }
-        } else {
-            switch (pl.lk2) {
-            case 1: CM_CX(3, 1); break;
-            case 2: CM_CX(3, 2); break;
-            default: CM_CX(3, 3); break;
-            }
-        }
-#undef CM_CX
-    } else if (pl.np == 2) {
+    if (pl.np == 2)
         hipLaunchKernelGGL((k_tc_crt<2>), g, dim3(256), 0, s, Cr[0], Cr[1], C2, d, one, K2, pl.M,
                            Ly, R, C, kc);
-    } else {
+    else
         hipLaunchKernelGGL((k_tc_crt<3>), g, dim3(256), 0, s, Cr[0], Cr[1], C2, d, one, K2, pl.M,
                            Ly, R, C, kc);
-    }
     return hipGetLastError();
+}
+
+// The fused form serves one-word coefficients and 2K <= 8 (2K = 16 would
+// spill in the CRT): x transforms in the split and CRT kernels, the y products
+// of every class and prime as one list of row segments.
+static bool tc_fused(const TcPlan &pl, int wa, int wb) {
+    return wa == 1 && wb == 1 && pl.lk2 >= 1 && pl.lk2 <= 3;
+}
+
+static size_t tc_item_words(const TcPlan &pl) {
+    return ((size_t)2 * pl.np << pl.lk2) << pl.ey;
+}
+
+// Fills one fused class over ws (R items, operands of at most la and lb
+// coefficients) and appends its row segments.
+static hipError_t tc_make_cls(const TcPlan &pl, int R, int la, int lb, int first, u32 *ws,
+                              TcCls &c, std::vector<RowSeg> &segs) {
+    c = TcCls{};
+    c.lk2 = pl.lk2; c.nprimes = pl.np; c.M = pl.M; c.ey = pl.ey; c.R = R; c.first = first;
+    c.len[0] = la; c.len[1] = lb;
+    const size_t half = ((size_t)R << pl.lk2) << pl.ey;   // rows of one operand and prime
+    for (int q = 0; q < pl.np; ++q) {
+        const Family *fam, *fx, *fxi;
+        hipError_t e = tc_x_families(q, pl.lk2, fam, fx, fxi);
+        if (e != hipSuccess) return e;
+        c.out[q][0] = ws + 2 * half * q;
+        c.out[q][1] = c.out[q][0] + half;
+        c.lvf[q] = fx->lv;
+        c.lvi[q] = fxi->lv;
+        c.p[q] = kTcPrimes[q];
+        c.np[q] = fam->np;
+        c.ki[q] = cm_host_mont(cm_host_inv(1u << pl.lk2, kTcPrimes[q]), kTcPrimes[q]);
+        segs.push_back(RowSeg{c.out[q][0], c.out[q][1], R << pl.lk2, pl.ey, la, lb, fam});
+    }
+    return hipSuccess;
 }
 
 // Runs the whole product on device buffers.  bits: largest coefficient bit
@@ -511,16 +555,34 @@ hipError_t launch_two_convolution(const u64 *a, int64_t na, int wa, const u64 *b
         *err = 1;
         return hipSuccess;
     }
-    const size_t per = (size_t)2 * (1 << pl.lk2) * ((size_t)1 << pl.ey);
-    u32 *ws = (u32 *)workspace(10, sizeof(u32) * per * pl.np, s);
+    u32 *ws = (u32 *)workspace(10, sizeof(u32) * tc_item_words(pl), s);
     if (!ws) return hipErrorOutOfMemory;
     TcDesc one{0, 0, 0, na, nb, wa, wb, wc, 0};
-    return tc_run_class(pl, a, b, c, nullptr, one, 1, na + nb - 1, wa == 1 && wb == 1, ws, s);
+    if (!tc_fused(pl, wa, wb))
+        return tc_run_class(pl, a, b, c, nullptr, one, 1, na + nb - 1, ws, s);
+    // one position per thread: a single product is bound by latency
+    constexpr int span = 256;
+    TcCls cls;
+    std::vector<RowSeg> segs;
+    hipError_t e = tc_make_cls(pl, 1, (int)na, (int)nb, 0, ws, cls, segs);
+    if (e != hipSuccess) return e;
+    {
+        ProfScope ps(kProfTcSplit, s);
+        const dim3 g((unsigned)((std::max(na, nb) + span - 1) / span), 2);
+        hipLaunchKernelGGL(k_tc_split_x, g, dim3(256), 0, s, a, b, nullptr, one, nullptr, cls,
+                           nullptr, span);
+    }
+    e = hipGetLastError();
+    if (e == hipSuccess) e = launch_rows_batch(std::move(segs), s);
+    if (e != hipSuccess) return e;
+    ProfScope ps(kProfTcCrt, s);
+    hipLaunchKernelGGL(k_tc_crt_x, dim3((unsigned)((na + nb - 1 + span - 1) / span)), dim3(256), 0,
+                       s, nullptr, one, nullptr, cls, nullptr, span, c, tc_crt_consts());
+    return hipGetLastError();
 }
 
 // Batch of products: items are grouped by class plan (tc_class_plan: one plan
-// per y size and (np, K)) and each class runs as one sequence of batched
-// launches, in chunks whose scratch stays under kTcChunkBytes.
+// per y size and (np, K)), in chunks whose scratch stays under kTcChunkBytes.
 static constexpr size_t kTcChunkBytes = (size_t)1 << 30;
 
 // Class merging of the batched multiply: 0 keeps one class per exact plan;
@@ -537,14 +599,113 @@ bool set_zmul_merge(int m) {
 
 int zmul_merge() { return g_tc_merge; }
 
+namespace {
+struct TcClass {
+    TcPlan pl;
+    bool fused;
+    std::vector<int64_t> idx;
+};
+}  // namespace
+
+// The fused classes of a batch: a split launch, the row products of all of
+// them and a CRT launch per chunk.  Each workgroup takes `span` positions of
+// one operand or product from a table.  (One launch sequence per class and
+// prime, on four streams, took 198 launches and 1.16 ms for 96 requests of
+// degrees 64 .. 65536; two uploads and 13 launches take 0.31 ms.)
+static hipError_t tc_run_fused(const std::vector<const TcClass *> &classes, const TcItem *items,
+                               const u64 *A, const u64 *B, u64 *C, hipStream_t s) {
+    constexpr int span = 1024;
+    size_t ci = 0, at = 0;   // next class, next item of it
+    while (ci < classes.size()) {
+        std::vector<TcCls> cls;
+        std::vector<TcDesc> desc;
+        std::vector<TcBlock> split, crt;
+        std::vector<RowSeg> segs;
+        std::vector<size_t> base;         // scratch offset of each class
+        struct Part {
+            const TcClass *c;
+            size_t i0, i1;
+        };
+        std::vector<Part> parts;
+        size_t words = 0;
+        // parts of classes up to the chunk's scratch (at least one item)
+        while (ci < classes.size()) {
+            const TcClass &c = *classes[ci];
+            const size_t per = tc_item_words(c.pl), room = kTcChunkBytes / sizeof(u32);
+            size_t n = words < room ? (room - words) / per : 0;
+            if (parts.empty() && n == 0) n = 1;
+            n = std::min(n, c.idx.size() - at);
+            if (n == 0) break;
+            parts.push_back(Part{&c, at, at + n});
+            base.push_back(words);
+            words += per * n;
+            at += n;
+            if (at < c.idx.size()) break;
+            ++ci;
+            at = 0;
+        }
+        u32 *ws = (u32 *)workspace(10, sizeof(u32) * words, s);
+        if (!ws) return hipErrorOutOfMemory;
+        for (size_t k = 0; k < parts.size(); ++k) {
+            const Part &q = parts[k];
+            const int first = (int)desc.size(), R = (int)(q.i1 - q.i0);
+            int64_t la = 0, lb = 0;
+            for (size_t i = q.i0; i < q.i1; ++i) {
+                const TcItem &it = items[q.c->idx[i]];
+                desc.push_back(TcDesc{it.a_off, it.b_off, it.c_off, it.na, it.nb, it.wa, it.wb,
+                                      it.wc, 0});
+                la = std::max(la, it.na);
+                lb = std::max(lb, it.nb);
+            }
+            TcCls c;
+            hipError_t e =
+                tc_make_cls(q.c->pl, R, (int)la, (int)lb, first, ws + base[k], c, segs);
+            if (e != hipSuccess) return e;
+            cls.push_back(c);
+            for (int r = 0; r < R; ++r) {
+                for (int w = 0; w < 2; ++w)
+                    for (int x = 0; x < c.len[w]; x += span)
+                        split.push_back(TcBlock{(int)k, r, w, x});
+                const TcDesc &d = desc[(size_t)(first + r)];
+                for (int64_t x = 0; x < d.na + d.nb - 1; x += span)
+                    crt.push_back(TcBlock{(int)k, r, 0, (int)x});
+            }
+        }
+        const size_t b0 = sizeof(TcCls) * cls.size(), b1 = sizeof(TcDesc) * desc.size(),
+                     b2 = sizeof(TcBlock) * split.size(), b3 = sizeof(TcBlock) * crt.size();
+        char *d = (char *)workspace(14, b0 + b1 + b2 + b3, s);
+        if (!d) return hipErrorOutOfMemory;
+        hipError_t e = stage_upload_fill(b0 + b1 + b2 + b3, d, s, [&](char *h) {
+            memcpy(h, cls.data(), b0);
+            memcpy(h + b0, desc.data(), b1);
+            memcpy(h + b0 + b1, split.data(), b2);
+            memcpy(h + b0 + b1 + b2, crt.data(), b3);
+        });
+        if (e != hipSuccess) return e;
+        const TcCls *dc = (const TcCls *)d;
+        const TcDesc *dd = (const TcDesc *)(d + b0);
+        const TcBlock *ds = (const TcBlock *)(d + b0 + b1), *dr = (const TcBlock *)(d + b0 + b1 + b2);
+        {
+            ProfScope ps(kProfTcSplit, s);
+            hipLaunchKernelGGL(k_tc_split_x, dim3((unsigned)split.size()), dim3(256), 0, s, A, B,
+                               dd, TcDesc{}, dc, TcCls{}, ds, span);
+        }
+        e = hipGetLastError();
+        if (e == hipSuccess) e = launch_rows_batch(std::move(segs), s);
+        if (e != hipSuccess) return e;
+        ProfScope ps(kProfTcCrt, s);
+        hipLaunchKernelGGL(k_tc_crt_x, dim3((unsigned)crt.size()), dim3(256), 0, s, dd, TcDesc{},
+                           dc, TcCls{}, dr, span, C, tc_crt_consts());
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 hipError_t launch_two_convolution_list(const TcItem *items, int64_t count, const u64 *A,
                                        const u64 *B, u64 *C, hipStream_t s, int *err) {
     *err = 0;
-    struct Cls {
-        TcPlan pl;
-        std::vector<int64_t> idx;
-    };
-    std::vector<Cls> classes;
+    std::vector<TcClass> classes;
     auto y_size = [](const TcItem &it) {
         int ey = 0;
         while (((int64_t)1 << ey) < it.na + it.nb - 1) ++ey;
@@ -561,32 +722,37 @@ hipError_t launch_two_convolution_list(const TcItem *items, int64_t count, const
         const int ey = y_size(it);
         const int bits = (g_tc_merge && ey < 64) ? widest[ey] : it.bits;
         TcPlan pl;
-        if (!tc_class_plan(bits, ey, pl) || pl.lk2 > kMaxLdsLog) {
+        if (!tc_class_plan(bits, ey, pl) || pl.lk2 > kMaxLdsLog || pl.ey > kMaxLog) {
             *err = 1;
             return hipSuccess;
         }
-        if (pl.ey > kMaxLog) {
-            *err = 1;
-            return hipSuccess;
-        }
-        Cls *c = nullptr;
+        const bool fused = tc_fused(pl, it.wa, it.wb);
+        TcClass *c = nullptr;
         for (auto &x : classes)
-            if (x.pl.np == pl.np && x.pl.K == pl.K && x.pl.M == pl.M && x.pl.ey == pl.ey) c = &x;
+            if (x.fused == fused && x.pl.np == pl.np && x.pl.K == pl.K && x.pl.M == pl.M &&
+                x.pl.ey == pl.ey)
+                c = &x;
         if (!c) {
-            classes.push_back(Cls{pl, {}});
+            classes.push_back(TcClass{pl, fused, {}});
             c = &classes.back();
         }
         c->idx.push_back(i);
     }
-    // descriptors of every class, in class order, uploaded once
-    std::vector<TcDesc> hd((size_t)count);
-    size_t at = 0;
-    for (auto &c : classes)
-        for (int64_t i : c.idx) {
+    std::vector<const TcClass *> fused, plain;
+    for (const TcClass &c : classes) (c.fused ? fused : plain).push_back(&c);
+    if (!fused.empty()) {
+        const hipError_t e = tc_run_fused(fused, items, A, B, C, s);
+        if (e != hipSuccess) return e;
+    }
+    if (plain.empty()) return hipSuccess;
+    // descriptors of the other classes, in class order, uploaded once
+    std::vector<TcDesc> hd;
+    for (const TcClass *c : plain)
+        for (int64_t i : c->idx) {
             const TcItem &it = items[i];
-            hd[at++] = TcDesc{it.a_off, it.b_off, it.c_off, it.na, it.nb, it.wa, it.wb, it.wc, 0};
+            hd.push_back(TcDesc{it.a_off, it.b_off, it.c_off, it.na, it.nb, it.wa, it.wb, it.wc, 0});
         }
-    TcDesc *dd = (TcDesc *)workspace(14, sizeof(TcDesc) * hd.size(), s);
+    TcDesc *dd = (TcDesc *)workspace(22, sizeof(TcDesc) * hd.size(), s);
     if (!dd) return hipErrorOutOfMemory;
     hipError_t e = stage_upload(hd.data(), sizeof(TcDesc) * hd.size(), dd, s);
     if (e != hipSuccess) return e;
@@ -594,7 +760,7 @@ hipError_t launch_two_convolution_list(const TcItem *items, int64_t count, const
     // stream's auxiliary streams (forked after the descriptor upload, joined
     // back at the end), so one class's launch gaps overlap another's work.
     // Each auxiliary stream has its own scratch.
-    const int nclass = (int)classes.size();
+    const int nclass = (int)plain.size();
     AuxStreams *aux = nclass > 1 ? aux_streams(s) : nullptr;
     const int nuse = aux ? std::min(nclass, (int)kAuxStreams) : 0;
     if (aux) {
@@ -605,27 +771,21 @@ hipError_t launch_two_convolution_list(const TcItem *items, int64_t count, const
     }
     size_t first = 0;
     for (int ci = 0; ci < nclass; ++ci) {
-        const auto &c = classes[(size_t)ci];
+        const TcClass &c = *plain[(size_t)ci];
         const hipStream_t cs = aux ? aux->s[ci % nuse] : s;
-        const int K2 = 1 << c.pl.lk2;
-        const int64_t Ly = (int64_t)1 << c.pl.ey;
-        const size_t item_bytes = sizeof(u32) * (size_t)2 * K2 * Ly * c.pl.np;
-        int64_t chunk = (int64_t)(kTcChunkBytes / item_bytes);
-        if (chunk < 1) chunk = 1;
+        const size_t item_bytes = sizeof(u32) * tc_item_words(c.pl);
+        const int64_t chunk = std::max<int64_t>(1, (int64_t)(kTcChunkBytes / item_bytes));
         const int64_t n = (int64_t)c.idx.size();
         for (int64_t k0 = 0; k0 < n; k0 += chunk) {
             const int R = (int)std::min<int64_t>(chunk, n - k0);
             u32 *ws = (u32 *)workspace(10, item_bytes * (size_t)R, cs);
             if (!ws) return hipErrorOutOfMemory;
             int64_t ymax = 1;
-            bool w1 = true;
             for (int r = 0; r < R; ++r) {
                 const TcItem &it = items[c.idx[(size_t)(k0 + r)]];
                 ymax = std::max<int64_t>(ymax, it.na + it.nb - 1);
-                w1 = w1 && it.wa == 1 && it.wb == 1;
             }
-            TcDesc none{};
-            e = tc_run_class(c.pl, A, B, C, dd + first + k0, none, R, ymax, w1, ws, cs);
+            e = tc_run_class(c.pl, A, B, C, dd + first + k0, TcDesc{}, R, ymax, ws, cs);
             if (e != hipSuccess) return e;
         }
         first += (size_t)n;

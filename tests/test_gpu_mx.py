@@ -100,3 +100,52 @@ def test_every_split_and_tile(cm, orc, logn):
     finally:
         assert L.cumodp_tune_set_split(logn, keep) == 0
         assert L.cumodp_tune_set_col_tile(16384) == 0
+
+
+def test_batched_rows_of_every_size(cm, orc):
+    """One batch of integer products whose rows have 2^4 .. 2^16 points in two
+    and three primes (every launch of the row list), with one- and two-word
+    operands, output words beyond the product's, and the most negative
+    coefficients; each product against the exact schoolbook."""
+    rng = np.random.default_rng(77)
+    pieces, items, want, at, out = [], [], [], 0, 0
+    for e in range(1, 17):
+        n = 1 << e
+        for bits in (1, 16, 33, 64):
+            if e >= 14 and bits == 33:
+                continue
+            nb = int(rng.integers(1, min(n, 700)))        # short: the check is schoolbook
+            na = max(1, n - nb + 1 - int(rng.integers(0, 2)))
+            lim = (1 << (bits - 1)) - 1 if bits == 64 else (1 << bits) - 1
+            a = rng.integers(-lim, lim, na, dtype=np.int64, endpoint=True)
+            b = rng.integers(-lim, lim, nb, dtype=np.int64, endpoint=True)
+            a[0], b[-1] = -lim, -lim
+            if bits == 64:
+                a[-1] = b[0] = -(1 << 63)
+            two = bits == 33 and e % 2 == 0               # the other form, in the same call
+            wc = 3 if bits == 64 else 3 + int(rng.integers(0, 3))
+            words = []
+            for v in (a, b):
+                w = v.view(np.uint64).reshape(-1, 1)
+                if two:
+                    w = np.concatenate([w, np.where(v < 0, np.uint64(2**64 - 1), np.uint64(0))
+                                        .reshape(-1, 1)], 1)
+                words.append(np.ascontiguousarray(w).ravel())
+            W = 2 if two else 1
+            items.append((at, at + na * W, out, na, nb, W, W, wc, bits))
+            pieces += words
+            at += (na + nb) * W
+            out += (na + nb - 1) * wc
+            want.append((orc.zmul_i64(a, b), wc))
+    arr = (cm.ZmulItem * len(items))(*[cm.ZmulItem(*t) for t in items])
+    A = cm.DeviceArray.from_host(np.concatenate(pieces), np.uint64)
+    H = cm.DeviceArray.from_host(np.full(out, 0x5A5A5A5A5A5A5A5A, np.uint64), np.uint64)
+    assert cm.lib().cumodp_two_convolution_list_dev(arr, len(items), A.addr(), A.addr(), H.addr(),
+                                                    None) == 0
+    got = H.download()
+    for t, (w, wc) in zip(items, want):
+        r = got[t[2]:t[2] + (t[3] + t[4] - 1) * wc].reshape(-1, wc)
+        assert (r[:, :3] == w).all(), t
+        sign = np.where(w[:, 2] >> np.uint64(63), np.uint64(2**64 - 1), np.uint64(0))
+        for j in range(3, wc):
+            assert (r[:, j] == sign).all(), t
