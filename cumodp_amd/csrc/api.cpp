@@ -182,8 +182,7 @@ cumodp_err ntt_dev_impl(u32 *X, int64_t m, int k, u32 w, u32 p, bool inverse, hi
     if (!fam) return fail(CUMODP_OUT_OF_MEMORY, "twiddle tables");
     hipError_t he;
     if (k <= kMaxLdsLog) {
-        const u32 sc = inverse ? cm_host_inv(cm_host_pow(2, k, p), p) : 1u;
-        he = launch_ntt_lds(k, X, m, inverse, sc, fam, s);
+        he = launch_ntt_lds(k, X, m, inverse, fam, s);
     } else {
         const int64_t n = (int64_t)1 << k;
         if (m > INT_MAX) return fail(CUMODP_FFT_SIZE_TOO_LARGE, "too many rows");

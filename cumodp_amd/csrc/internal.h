@@ -16,7 +16,6 @@ constexpr int kMaxLdsLog = 13;     // largest multiply done inside one workgroup
 constexpr int kMaxRowLog = 14;     // largest four-step row
 constexpr int kMaxLevelLog = 15;   // largest level of the twiddle tables (in-LDS 2^15 products)
 constexpr int kMaxLog = 26;        // largest transform supported (2^13 x 2^13)
-constexpr int kOuterLoBits = 12;   // four-step twiddle split: w^e = lo[e & 4095] * hi[e >> 12]
 constexpr int kNoAllocMaxLog = 22; // largest transform of the non-allocating multiply
 
 // Scratch of the non-allocating multiply (noalloc.hip): a file-scope device
@@ -46,14 +45,11 @@ struct Family {
 
 // Four-step outer twiddles w_n^e for one transform size n = 2^k
 // (n = 2^k1 rows x 2^k2 columns).
-//   lo/hi: w_n^e = lo[e mod 4096] * hi[e / 4096] (column-pass form);
-//   rb/rc: row-pass form for a row with frequency index k1 read by T =
-//          2^k2 / 16 threads as elements i = t + T m (m < 16):
-//          w_n^(k1 i) = rb[k1 T + t] * rc[16 k1 + m].
+// For a row with frequency index k1 and T = 2^k2 / 16, element i = t + T m
+// (m < 16): w_n^(k1 i) = rb[k1 T + t] * rc[16 k1 + m].
 // The _f tables use w_n, the _i tables w_n^-1; all in Montgomery form.
 struct Outer {
     int k, k1, k2;        // the split these tables were built for
-    u32 *lo_f, *hi_f, *lo_i, *hi_i;
     u32 *rb_f, *rc_f, *rb_i, *rc_i;
 };
 
@@ -63,6 +59,7 @@ struct Outer {
 const Family *family_default(u32 p);
 const Family *family_for_root(u32 p, u32 w, int k);
 const Outer *outer_for(const Family *f, int k);   // for the current split of k
+const Outer *outer_for_split(const Family *f, int k, int k1, int k2);
 // The same lookups that never build (and so never allocate): nullptr when the
 // tables are not built yet.
 const Family *family_default_cached(u32 p);
@@ -176,9 +173,9 @@ hipError_t launch_mul_lds_one(int logn, const u32 *F, const u32 *G, u32 *H,
 hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, const MulDesc &sd,
                                   int count, const Family *fam, hipStream_t s);
 
-// In-place natural-order forward DFT of m rows of 2^k words (k <= 13),
-// outputs multiplied by the residue `scale` (1: none).
-hipError_t launch_ntt_lds(int k, u32 *X, int64_t m, bool inverse, u32 scale, const Family *fam,
+// In-place natural-order DFT of m rows of 2^k words (k <= 13); inverse uses
+// the inverse root and scales by 2^-k.
+hipError_t launch_ntt_lds(int k, u32 *X, int64_t m, bool inverse, const Family *fam,
                           hipStream_t s);
 
 // Operands of a batch of four-step multiplies of size n = 2^k: pair a reads
@@ -207,9 +204,8 @@ hipError_t launch_mul_strided(int logn, const u32 *F, int64_t fs, int lf, const 
                               int64_t gs, int lg, u32 *H, int64_t hs, int lh, int count,
                               const Family *fam, hipStream_t s);
 
-// Four-step natural-order forward DFT of cnt arrays of 2^k words (in place,
-// using Y as cnt * 2^k words of temporary space); inverse uses the inverse
-// table and scales by 2^-k.
+// Four-step natural-order DFT of cnt arrays of 2^k words (in place, using Y as
+// cnt * 2^k words of temporary space); inverse as in launch_ntt_lds.
 hipError_t launch_ntt_four_step(int k, u32 *X, u32 *Y, int cnt, bool inverse, const Family *fam,
                                 hipStream_t s);
 

@@ -203,4 +203,9 @@ CM_DEV void mx_row(u32 *lds, u32 *F, const u32 *G, int row0, int k1, const MxOut
     }
 }
 
+// Forward column transforms of cnt arrays of n = 2^(k1+k2) words, X -> Y
+// (mul_mx.hip).
+hipError_t launch_cols_out(int k1, const u32 *X, u32 *Y, int64_t n, int cnt, int k2,
+                           const MxCtx &cx, hipStream_t s);
+
 }  // namespace cm

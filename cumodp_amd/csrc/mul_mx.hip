@@ -220,8 +220,7 @@ bool set_col_tile_words(int words) {
 int col_tile_words() { return g_col_words; }
 
 static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCols &s1, int cnt0,
-                              int cnt1, int k2, bool small, const Family *fam, hipStream_t s) {
-    const MxCtx cx = mx_ctx(fam);
+                              int cnt1, int k2, bool small, const MxCtx &cx, hipStream_t s) {
 #define CM_COL(LC, V) return cols_t<K, LC, V>(inverse, s0, s1, cnt0, cnt1, k2, cx, s)
 #define CM_COLS(KK, LS, VS, LB)                       \
     case KK: {                                        \
@@ -229,9 +228,10 @@ static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCo
         if (small) CM_COL(LS, VS);                    \
         CM_COL(LB, 4);                                \
     }
-#define CM_COLB(KK, LB)                               \
+#define CM_COLB(KK, LB, LS)                           \
     case KK: {                                        \
         constexpr int K = KK;                         \
+        if (small) CM_COL(LS, 1);                     \
         if (g_col_words == 8192) CM_COL(LB - 1, 4);   \
         CM_COL(LB, 4);                                \
     }
@@ -241,9 +241,13 @@ static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCo
         CM_COLS(6, 3, 1, 4)
         CM_COLS(7, 4, 1, 4)
         CM_COLS(8, 3, 1, 4)
-        CM_COLB(9, 4)
-        CM_COLB(10, 4)
-        CM_COLB(11, 3)
+        CM_COLB(9, 4, 3)
+        CM_COLB(10, 4, 2)
+    case 11: {
+        constexpr int K = 11;
+        if (g_col_words == 8192) CM_COL(2, 4);
+        CM_COL(3, 4);
+    }
     case 12: {
         constexpr int K = 12;
         CM_COL(2, 4);
@@ -253,6 +257,12 @@ static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCo
 #undef CM_COLS
 #undef CM_COL
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_cols_out(int k1, const u32 *X, u32 *Y, int64_t n, int cnt, int k2,
+                           const MxCtx &cx, hipStream_t s) {
+    const MxCols c{X, Y, n, n, n, n};
+    return launch_cols(k1, false, c, c, cnt, 0, k2, n * cnt <= kMxSmallWords, cx, s);
 }
 
 template <int LOGL, int V>
@@ -294,12 +304,13 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
     const int64_t n = (int64_t)1 << o->k;
     const MxCols sf{io.f_in, io.f_ws, io.in_stride, io.f_len, n, n};
     const MxCols sg{io.g_in, io.g_ws, io.g_stride < 0 ? io.in_stride : io.g_stride, io.g_len, n, n};
+    const MxCtx cx = mx_ctx(fam);
     const bool small = n * io.cnt <= kMxSmallWords;
-    hipError_t e = launch_cols(o->k1, false, sf, sg, io.cnt, io.cnt, o->k2, small, fam, s);
+    hipError_t e = launch_cols(o->k1, false, sf, sg, io.cnt, io.cnt, o->k2, small, cx, s);
     if (e == hipSuccess) e = launch_rows(io, o, fam, s);
     if (e != hipSuccess) return e;
     const MxCols sh{io.f_ws, io.h_out, n, n, io.out_stride, io.h_len};
-    return launch_cols(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, fam, s);
+    return launch_cols(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, cx, s);
 }
 
 hipError_t launch_mul_four_step(int k, const FourStepIO &io, const Family *fam, hipStream_t s) {

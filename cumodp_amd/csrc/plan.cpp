@@ -231,23 +231,22 @@ bool set_four_step_split(int k, int k2) {
 const Outer *outer_for(const Family *f, int k) {
     int k1, k2;
     four_step_split(k, k1, k2);
+    return outer_for_split(f, k, k1, k2);
+}
+
+const Outer *outer_for_split(const Family *f, int k, int k1, int k2) {
     std::lock_guard<std::mutex> lk(g_plan_mutex);
     auto key = std::make_tuple(f, k, k2);
     auto it = g_outer.find(key);
     if (it != g_outer.end()) return it->second;
-    if (k > f->K || k <= kOuterLoBits) return nullptr;
+    if (k > f->K || k1 + k2 != k || k1 < 1 || k2 < 4) return nullptr;
     u32 p = f->p;
     u32 wn = cm_host_pow(f->wN, (u64)1 << (f->K - k), p);   // order 2^k
     u32 wni = cm_host_inv(wn, p);
-    size_t nlo = (size_t)1 << kOuterLoBits, nhi = (size_t)1 << (k - kOuterLoBits);
     Outer *o = new Outer();
     o->k = k;
     o->k1 = k1;
     o->k2 = k2;
-    o->lo_f = upload(power_table(wn, nlo, p));
-    o->hi_f = upload(power_table(cm_host_pow(wn, nlo, p), nhi, p));
-    o->lo_i = upload(power_table(wni, nlo, p));
-    o->hi_i = upload(power_table(cm_host_pow(wni, nlo, p), nhi, p));
     // row-pass tables
     const size_t n1 = (size_t)1 << k1, T = ((size_t)1 << k2) / 16;
     for (int dir = 0; dir < 2; ++dir) {
@@ -270,8 +269,7 @@ const Outer *outer_for(const Family *f, int k) {
         (dir ? o->rb_i : o->rb_f) = upload(rb);
         (dir ? o->rc_i : o->rc_f) = upload(rc);
     }
-    if (!o->lo_f || !o->hi_f || !o->lo_i || !o->hi_i || !o->rb_f || !o->rc_f || !o->rb_i ||
-        !o->rc_i) {
+    if (!o->rb_f || !o->rc_f || !o->rb_i || !o->rc_i) {
         delete o;
         return nullptr;
     }

@@ -149,3 +149,55 @@ def test_batched_rows_of_every_size(cm, orc):
         sign = np.where(w[:, 2] >> np.uint64(63), np.uint64(2**64 - 1), np.uint64(0))
         for j in range(3, wc):
             assert (r[:, j] == sign).all(), t
+
+
+def _root(k, p):
+    fac = [d for d in range(2, 1 << 16) if (p - 1) % d == 0 and all(d % q for q in range(2, d) if q * q <= d)]
+    g = next(x for x in range(2, 200) if all(pow(x, (p - 1) // d, p) != 1 for d in fac))
+    return pow(g, (p - 1) >> k, p)
+
+
+@pytest.mark.parametrize("p,top", [(P1, 15), (P2, 15), (TOP, 15), (257, 8), (12289, 12)])
+def test_row_transforms(cm, orc, p, top):
+    """Rows of 2^4 .. 2^15 words (one and two launches) in the forms of few and
+    of many words, with row counts that do not fill the last workgroup, at a
+    4-byte aligned address."""
+    rng = np.random.default_rng(p + 2)
+    for k in range(4, top + 1):
+        n, w = 1 << k, _root(k, p)
+        for m in (1, 3, max(5, ((1 << 19) >> k) + 1)):
+            X = rng.integers(0, p, m * n, dtype=np.int32)
+            d = cm.DeviceArray.from_host(np.concatenate([np.full(1, 7, np.int32), X,
+                                                         np.full(3, 9, np.int32)]))
+            cm.cxx("list_stockham_dev_w")(d.addr(1), m, k, w, p)
+            got = d.download()
+            assert got[0] == 7 and (got[-3:] == 9).all(), (p, k, m)
+            got = got[1:-3].reshape(m, n)
+            for r in sorted({0, m // 2, m - 1}):
+                assert (got[r] == orc.stockham(X[r * n:(r + 1) * n], w, p)).all(), (p, k, m, r)
+
+
+@pytest.mark.parametrize("k", list(range(4, 23)))
+def test_transform_and_inverse(cm, orc, k):
+    p = P2 if k & 1 else P1
+    rng = np.random.default_rng(k)
+    n, w = 1 << k, _root(k, p)
+    X = rng.integers(0, p, n, dtype=np.int32)
+    Y = cm.fft_uni(X, w, p)
+    assert (Y == orc.stockham(X, w, p)).all()
+    assert (cm.invfft_uni(Y, w, p) == X).all()
+    assert (cm.invfft_uni(X, w, p) == orc.inverse_stockham(X, w, p)).all()
+
+
+@pytest.mark.parametrize("k", [23, 24, 25, 26])
+def test_largest_transforms(cm, k):
+    """X = a x^3 + b x^i has Y_j = a w^(3j) + b w^(ij); and back."""
+    p, n = P2, 1 << k
+    w, i = _root(k, P2), (1 << k) - 12345
+    X = np.zeros(n, np.int32)
+    X[3], X[i] = 123456789, 987654321
+    Y = cm.fft_uni(X, w, p)
+    for j in (0, 1, 2, 5, 16, 255, 4096, n // 2 + 1, n - 1, 0x155555 % n):
+        want = (123456789 * pow(w, 3 * j, p) + 987654321 * pow(w, i * j, p)) % p
+        assert int(Y[j]) == want, (k, j)
+    assert (cm.invfft_uni(Y, w, p) == X).all()
