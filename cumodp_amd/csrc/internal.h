@@ -190,11 +190,20 @@ struct FourStepIO {
     int64_t h_len, out_stride;
     int cnt;
     int64_t g_stride = -1;   // stride of g_in when it differs from in_stride
+    // pair a takes array a >> g_shift of g (g_ws has cnt >> g_shift arrays) and
+    // writes output a ^ out_xor, words out_from .. h_len - 1; monic: operands
+    // are monic of n/2 + 1 words, outputs monic of n + 1
+    int g_shift = 0, out_from = 0, out_xor = 0, monic = 0;
 };
 hipError_t launch_mul_four_step(int k, const FourStepIO &io, const Family *fam, hipStream_t s);
 // the same with tables the caller looked up (no table is built here)
 hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, const Outer *o,
                                      hipStream_t s);
+
+// Level i of the subproduct tree from level i - 1: node d of `cur` (2^i + 1
+// words) is the product of nodes 2d and 2d + 1 of `prev` (2^(i-1) + 1 words).
+hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, const Family *fam,
+                             hipStream_t s);
 
 // count products of one shape: product d reads lf words at F + d fs and lg
 // words at G + d gs and writes the first lh words of the 2^logn-point cyclic

@@ -77,9 +77,12 @@ CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const
 }
 
 // The mirror: digit-reversed rows in, natural rows out (canonical, words at or
-// beyond lim not stored).
-template <int LOGL, int LOGC, int V>
-CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int lim, int logn2, const MxCtx &cx) {
+// beyond lim, relative to Y, not stored).  EDGES: words below `from` are not
+// stored either, and word `fix` is stored less one (tests that cost the plain
+// form 7%).
+template <int LOGL, int LOGC, int V, bool EDGES>
+CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fix, int logn2,
+                       const MxCtx &cx) {
     static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
                   "a wave's 256 V words lie inside the tile");
     using P = MxPlan<LOGL, LOGC>;
@@ -108,16 +111,19 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int lim, int logn2, const
     for (int r = 0; r < 4; ++r) {
         const int e = (int)(off + r * row);
 #pragma unroll
-        for (int s = 0; s < V; ++s) x[s][r] = mx_canon(x[s][r], cx);
+        for (int s = 0; s < V; ++s) {
+            x[s][r] = mx_canon(x[s][r], cx);
+            if (EDGES && e + s == fix) x[s][r] = cm_sub(x[s][r], 1u, cx.p);
+        }
         if constexpr (V == 4) {
-            if (e + V <= lim) {
+            if ((!EDGES || e >= from) && e + V <= lim) {
                 *(MxQuad *)(Y + e) = MxQuad{{x[0][r], x[1][r], x[2][r], x[3][r]}};
                 continue;
             }
         }
 #pragma unroll
         for (int s = 0; s < V; ++s)
-            if (e + s < lim) Y[e + s] = x[s][r];
+            if ((!EDGES || e + s >= from) && e + s < lim) Y[e + s] = x[s][r];
     }
 }
 

@@ -6,6 +6,8 @@
 
 namespace cm {
 
+enum : int { kStrided = 0, kDesc = 1, kMonic = 2 };
+
 // A single product is bound by its serial chain (load, rounds, exchanges), many
 // products by vector issue.  One 2048-point product mod 469762049, back to
 // back: 4.8 us per call with one set per lane (512 threads), 8.1 us with the
@@ -16,10 +18,12 @@ namespace cm {
 // multiplied in registers and the product transformed back (ntt_mx.h).
 // DESC: descriptors from `descs` (or the by-value `one` when descs is null);
 // otherwise product d reads F + d * one.f, G + d * one.g (one.lf / one.lg
-// words) and writes H + d * one.h (one.lh words).  H may alias F or G: a
+// words) and writes H + d * one.h (one.lh words); kMonic: the same with monic
+// operands of 2^LOGL / 2 + 1 words, whose product's leading term wraps onto word
+// 0 and is put into word 2^LOGL.  H may alias F or G: a
 // product's words are all loaded before any of its words is stored, by the
 // same wave or on the other side of a barrier.
-template <int LOGL, int LOGW, int V, bool DESC>
+template <int LOGL, int LOGW, int V, int DESC>
 __global__ __launch_bounds__((1 << LOGW) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
     const u32 *F, const u32 *G, u32 *H, const MulDesc *__restrict__ descs, int ndesc, MulDesc one,
@@ -34,7 +38,7 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
         const int d = blockIdx.x * C + row0 + (Map::off(s, 0) >> LOGL);
         MulDesc m{};
         if (d < ndesc) {
-            if (DESC) {
+            if (DESC == kDesc) {
                 m = descs ? descs[d] : one;
             } else {
                 m = one;
@@ -57,6 +61,13 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
         len = m.lg;
     });
     mx_tile_multiply<LOGL, V>(x, lds, lds + LW, cx, m, tw);
+    if constexpr (DESC == kMonic) {
+        // word 0 of a row: set s, r = 0 of the lane that holds its start
+#pragma unroll
+        for (int s = 0; s < V; ++s)
+            if (((Map::base() + Map::off(s, 0)) & ((1 << LOGL) - 1)) == 0)
+                x[0][s][0] = cm_sub(mx_canon(x[0][s][0], cx), 1u, cx.p);
+    }
     mx_store_rows<LOGL, V>(
         x[0],
         [&](int s, u32 *&q, int &len) {
@@ -65,13 +76,14 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
             len = std::min(m.lh, 1 << LOGL);
         },
         cx);
-    // words beyond the transform size (lh > L) are zero
+    // words beyond the transform size (lh > L) are zero, or the leading 1
     for (int c = 0; c < C; ++c) {
         const int d = blockIdx.x * C + c;
         if (d >= ndesc) break;
-        const MulDesc m = DESC && descs ? descs[d] : one;
-        const int64_t h = DESC ? m.h : (int64_t)d * one.h;
-        for (int i = (1 << LOGL) + threadIdx.x; i < m.lh; i += blockDim.x) H[h + i] = 0u;
+        const MulDesc m = DESC == kDesc && descs ? descs[d] : one;
+        const int64_t h = DESC == kDesc ? m.h : (int64_t)d * one.h;
+        for (int i = (1 << LOGL) + threadIdx.x; i < m.lh; i += blockDim.x)
+            H[h + i] = DESC == kMonic ? 1u : 0u;
     }
 }
 
@@ -81,7 +93,7 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
 // fit a workgroup).
 constexpr int64_t kMxSpreadWords = (int64_t)1 << 19;
 
-template <int LOGL, int V, bool DESC>
+template <int LOGL, int V, int DESC>
 static hipError_t mul_mx_v(const u32 *F, const u32 *G, u32 *H, const MulDesc *descs, int ndesc,
                            const MulDesc &one, const Family *fam, hipStream_t s) {
     constexpr int LOGW = std::max(LOGL, 8 + mx_log2(V));
@@ -92,7 +104,7 @@ static hipError_t mul_mx_v(const u32 *F, const u32 *G, u32 *H, const MulDesc *de
     return hipGetLastError();
 }
 
-template <int LOGL, bool DESC>
+template <int LOGL, int DESC>
 static hipError_t mul_mx_t(const u32 *F, const u32 *G, u32 *H, const MulDesc *descs, int ndesc,
                            const MulDesc &one, const Family *fam, hipStream_t s) {
     const int64_t words = (int64_t)ndesc << LOGL;
@@ -111,7 +123,7 @@ hipError_t launch_mul_lds_one(int logn, const u32 *F, const u32 *G, u32 *H,
                               const Family *fam, hipStream_t s) {
     if (ndesc <= 0) return hipSuccess;
     switch (logn) {
-#define CM_CASE(K) case K: return mul_mx_t<K, true>(F, G, H, d_descs, ndesc, one, fam, s);
+#define CM_CASE(K) case K: return mul_mx_t<K, kDesc>(F, G, H, d_descs, ndesc, one, fam, s);
         CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8) CM_CASE(9) CM_CASE(10)
         CM_CASE(11) CM_CASE(12) CM_CASE(13) CM_CASE(14)
 #undef CM_CASE
@@ -128,7 +140,7 @@ hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, 
                                   int count, const Family *fam, hipStream_t s) {
     if (count <= 0) return hipSuccess;
     switch (logn) {
-#define CM_CASE(K) case K: return mul_mx_t<K, false>(F, G, H, nullptr, count, sd, fam, s);
+#define CM_CASE(K) case K: return mul_mx_t<K, kStrided>(F, G, H, nullptr, count, sd, fam, s);
         CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8) CM_CASE(9) CM_CASE(10)
         CM_CASE(11) CM_CASE(12) CM_CASE(13)
 #undef CM_CASE
@@ -137,15 +149,49 @@ hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, 
 }
 
 
+hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, const Family *fam,
+                             hipStream_t s) {
+    const int64_t h = (int64_t)1 << (i - 1), n = 2 * h;
+    if (nodes <= 0 || nodes > INT32_MAX) return hipErrorInvalidValue;
+    const MulDesc sd{2 * (h + 1), 2 * (h + 1), n + 1, (int)(h + 1), (int)(h + 1), (int)(n + 1), i};
+    switch (i) {
+#define CM_CASE(K)                                                                        \
+    case K:                                                                               \
+        return mul_mx_t<K, kMonic>(prev, prev + (h + 1), cur, nullptr, (int)nodes, sd, fam, s);
+        CM_CASE(8) CM_CASE(9) CM_CASE(10) CM_CASE(11) CM_CASE(12) CM_CASE(13)
+#undef CM_CASE
+    }
+    // four-step straight from and into the tree, in chunks whose two slabs
+    // stay within 1 GiB each
+    const int64_t chunk = std::max<int64_t>(1, ((int64_t)1 << 28) / n);
+    for (int64_t c0 = 0; c0 < nodes; c0 += chunk) {
+        const int cnt = (int)std::min<int64_t>(chunk, nodes - c0);
+        u32 *sf = (u32 *)workspace(5, sizeof(u32) * (size_t)(n * cnt), s);
+        u32 *sg = (u32 *)workspace(6, sizeof(u32) * (size_t)(n * cnt), s);
+        if (!sf || !sg) return hipErrorOutOfMemory;
+        const u32 *f = prev + c0 * 2 * (h + 1);
+        FourStepIO io{f, f + (h + 1), h + 1, h + 1, 2 * (h + 1), sf, sg, cur + c0 * (n + 1),
+                      n, n + 1, cnt};
+        io.monic = 1;
+        const hipError_t e = launch_mul_four_step(i, io, fam, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // ---------------------------------------------------------------------------
 // four-step multiply: an n-word array viewed as 2^k1 rows x 2^k2 columns
 // ---------------------------------------------------------------------------
 // One set of arrays of the column passes: array a reads in[a in_stride + e]
-// for e < in_len (zero beyond) and writes out[a out_stride + e], e < out_len.
+// for e < in_len (zero beyond) and writes out[(a ^ out_xor) out_stride + e] for
+// out_from <= e < out_len.  monic: the product of two monic polynomials of
+// half the length, whose x^n wrapped onto word 0: that word less one, and a
+// leading 1 in word n.
 struct MxCols {
     const u32 *in;
     u32 *out;
     int64_t in_stride, in_len, out_stride, out_len;
+    int out_from = 0, out_xor = 0, monic = 0;
 };
 
 // Forward column transforms of 2^LOGC columns per workgroup (mx_col_fwd).
@@ -163,26 +209,34 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_fwd_mx(MxCols s0, MxCols s
                               S.out + a * S.out_stride + c0, logn2, cx);
 }
 
-// Inverse column transforms (mx_col_inv), truncated to out_len.
-template <int LOGL, int LOGC, int V>
+// Inverse column transforms (mx_col_inv), truncated to out_len.  EDGES: sets
+// with out_from, out_xor or monic.
+template <int LOGL, int LOGC, int V, bool EDGES>
 __global__ __launch_bounds__((1 << (LOGL + LOGC)) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_inv_mx(MxCols S, int logn2, MxCtx cx) {
     __shared__ __align__(16) u32 lds[mx_col_lds<LOGL, LOGC>()];
     const int64_t a = blockIdx.y;
     const int c0 = mx_xcd(blockIdx.x, gridDim.x) << LOGC;
-    mx_col_inv<LOGL, LOGC, V>(lds, S.in + a * S.in_stride + c0, S.out + a * S.out_stride + c0,
-                              (int)(S.out_len - c0), logn2, cx);
+    u32 *Y = S.out + (EDGES ? a ^ S.out_xor : a) * S.out_stride + c0;
+    mx_col_inv<LOGL, LOGC, V, EDGES>(lds, S.in + a * S.in_stride + c0, Y, S.out_from - c0,
+                                     (int)(S.out_len - c0), S.monic ? -c0 : INT32_MIN, logn2, cx);
+    if (EDGES && S.monic && c0 == 0 && threadIdx.x == 0)
+        Y[(int64_t)1 << (LOGL + logn2)] = 1u;
 }
 
-// Row pass (mx_row) over all rows of cnt arrays, in place on F.
+// Row pass (mx_row) over all rows of the arrays of F, in place.
 template <int LOGL, int V>
 __global__ __launch_bounds__((1 << mx_row_logw<LOGL, V>()) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_row_mx(u32 *F, const u32 *__restrict__ G, int k1,
-                                                         MxOuter o, MxCtx cx) {
+                                                         int g_shift, MxOuter o, MxCtx cx) {
     constexpr int LOGW = mx_row_logw<LOGL, V>();
     __shared__ __align__(16) u32 lds[2 * mx_lds_words(1 << LOGW)];
+    // array a of F meets array a >> g_shift of G
+    const int la = k1 + LOGL - LOGW;   // log2 of the tiles per array
     const int64_t t0 = (int64_t)blockIdx.x << LOGW;
-    mx_row<LOGL, V>(lds, F + t0, G + t0, (int)(blockIdx.x << (LOGW - LOGL)), k1, o, cx);
+    const int64_t ga = (int64_t)(blockIdx.x >> la) >> g_shift;
+    const int64_t tg = ((ga << la) + (blockIdx.x & ((1u << la) - 1))) << LOGW;
+    mx_row<LOGL, V>(lds, F + t0, G + tg, (int)(blockIdx.x << (LOGW - LOGL)), k1, o, cx);
 }
 
 template <int LOGL, int LOGC, int V>
@@ -191,8 +245,10 @@ static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int c
     constexpr int T = (1 << (LOGL + LOGC)) / (4 * V);
     ProfScope ps(inverse ? kProfColInv : kProfColFwd, s);
     const dim3 g(1u << (k2 - LOGC), cnt0 + cnt1);
-    if (inverse)
-        hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V>), g, dim3(T), 0, s, s0, k2, cx);
+    if (inverse && (s0.out_from || s0.out_xor || s0.monic))
+        hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V, true>), g, dim3(T), 0, s, s0, k2, cx);
+    else if (inverse)
+        hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V, false>), g, dim3(T), 0, s, s0, k2, cx);
     else
         hipLaunchKernelGGL((k_col_fwd_mx<LOGL, LOGC, V>), g, dim3(T), 0, s, s0, s1, cnt0, k2, cx);
     return hipGetLastError();
@@ -271,7 +327,7 @@ static hipError_t rows_t(const FourStepIO &io, const Outer *o, const Family *fam
     ProfScope ps(kProfRowMul, s);
     const int64_t words = (int64_t)io.cnt << o->k;
     hipLaunchKernelGGL((k_row_mx<LOGL, V>), dim3((unsigned)(words >> LOGW)),
-                       dim3((1 << LOGW) / (4 * V)), 0, s, io.f_ws, io.g_ws, o->k1,
+                       dim3((1 << LOGW) / (4 * V)), 0, s, io.f_ws, io.g_ws, o->k1, io.g_shift,
                        mx_outer_of(o), mx_ctx(fam));
     return hipGetLastError();
 }
@@ -306,10 +362,12 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
     const MxCols sg{io.g_in, io.g_ws, io.g_stride < 0 ? io.in_stride : io.g_stride, io.g_len, n, n};
     const MxCtx cx = mx_ctx(fam);
     const bool small = n * io.cnt <= kMxSmallWords;
-    hipError_t e = launch_cols(o->k1, false, sf, sg, io.cnt, io.cnt, o->k2, small, cx, s);
+    hipError_t e =
+        launch_cols(o->k1, false, sf, sg, io.cnt, io.cnt >> io.g_shift, o->k2, small, cx, s);
     if (e == hipSuccess) e = launch_rows(io, o, fam, s);
     if (e != hipSuccess) return e;
-    const MxCols sh{io.f_ws, io.h_out, n, n, io.out_stride, io.h_len};
+    const MxCols sh{io.f_ws, io.h_out, n, n, io.out_stride, io.h_len,
+                    io.out_from, io.out_xor, io.monic};
     return launch_cols(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, cx, s);
 }
 

@@ -8,14 +8,13 @@
 // the monic product of 2^i consecutive (x - x_j) stored with its leading
 // coefficient (2^i + 1 canonical words), level i starting at word
 //     off(i) = sum_{l < i} 2^(k-l) (2^l + 1).
-// Level i comes from level i-1 by the same monic identity the reference uses
-// (:601-650): with A = x^h + a and B = x^h + b (h = 2^(i-1), deg a, b < h),
-//     A B = x^(2h) + x^h (a + b) + a b,
-// where all products a b of a level are one call of the strided multiply:
-// halves of up to 256 coefficients take the wavefront schoolbook kernel
-// (plain.hip), larger ones the NTT multiply (one LDS workgroup per product,
-// or four-step for 2^i > 2^13).  Levels 0 .. 8 are built before that in one
-// launch, a 256-point subtree per workgroup (k_tree_bottom).
+// Level i is one batch of products on 2^i points of the whole monic nodes of
+// level i-1 (leading 1 included): the product's x^(2^i) wraps onto its constant
+// term, which the store takes back while it writes the leading 1, so a level
+// is one launch up to 2^13 points and three above, with no pass that adds the
+// leading terms.  (The reference multiplies without the leading terms and adds
+// x^h (a + b) afterwards, :601-650.)  Levels 0 .. 8 are built before that in
+// one launch, a 256-point subtree per workgroup (k_tree_bottom).
 #include "accum.h"
 #include "internal.h"
 
@@ -25,26 +24,6 @@ int64_t tree_level_offset(int k, int i) {
     int64_t off = 0;
     for (int l = 0; l < i; ++l) off += ((int64_t)1 << (k - l)) * (((int64_t)1 << l) + 1);
     return off;
-}
-
-// after H[0 .. 2h-2] = a b: add (a + b) x^h and the leading 1
-__global__ void k_tree_combine(u32 *__restrict__ tree, int64_t off_prev, int64_t off_cur, int h,
-                               int64_t nprod, u32 p) {
-    const int len = 2 * h + 1;
-    for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < nprod * (h + 1);
-         g += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t j = g / (h + 1);
-        const int t = h + (int)(g % (h + 1));        // h .. 2h
-        const u32 *A = tree + off_prev + (2 * j) * (h + 1);
-        const u32 *B = A + (h + 1);
-        u32 *C = tree + off_cur + j * len;
-        if (t == 2 * h) {
-            C[t] = 1u;
-        } else {
-            const u32 s = cm_add(A[t - h], B[t - h], p);
-            C[t] = (t < 2 * h - 1) ? cm_add(C[t], s, p) : s;
-        }
-    }
 }
 
 // Levels 0 .. pin of the tree in one launch: workgroup J (blockDim.x =
@@ -94,11 +73,6 @@ __global__ __launch_bounds__(1 << kTreeFuse) void k_tree_bottom(const u32 *__res
     }
 }
 
-static int tblocks(int64_t n) {
-    int64_t b = (n + 255) / 256;
-    return (int)(b < 1 ? 1 : (b > 16384 ? 16384 : b));
-}
-
 hipError_t launch_subproduct_tree(const u32 *pts, int k, u32 p, u32 *tree, const Family *fam,
                                   hipStream_t s) {
     const int64_t n = (int64_t)1 << k;
@@ -108,21 +82,8 @@ hipError_t launch_subproduct_tree(const u32 *pts, int k, u32 p, u32 *tree, const
                        plain_mod(p), tree, n);
     hipError_t e = hipGetLastError();
     for (int i = pin + 1; i <= k && e == hipSuccess; ++i) {
-        const int h = 1 << (i - 1);
-        const int64_t nprod = n >> i;
-        const int64_t op = tree_level_offset(k, i - 1), oc = tree_level_offset(k, i);
-        // the level's products share one shape: a = node 2j and b = node 2j+1
-        // of level i-1 (their non-leading h coefficients, 2(h+1) words apart),
-        // a b (2h-1 words) at node j of level i; no descriptors.  Up to 256
-        // coefficients each the strided multiply takes the schoolbook kernel
-        // (faster than the transform there), above it the NTT multiply on
-        // 2h points
-        e = launch_mul_strided(i, tree + op, 2 * (h + 1), h, tree + op + (h + 1), 2 * (h + 1), h,
-                               tree + oc, 2 * h + 1, 2 * h - 1, (int)nprod, fam, s);
-        if (e != hipSuccess) break;
-        hipLaunchKernelGGL(k_tree_combine, dim3(tblocks(nprod * (h + 1))), dim3(256), 0, s, tree,
-                           op, oc, h, nprod, p);
-        e = hipGetLastError();
+        e = launch_tree_level(i, tree + tree_level_offset(k, i - 1),
+                              tree + tree_level_offset(k, i), n >> i, fam, s);
     }
     return e;
 }

@@ -201,3 +201,28 @@ def test_largest_transforms(cm, k):
         want = (123456789 * pow(w, 3 * j, p) + 987654321 * pow(w, i * j, p)) % p
         assert int(Y[j]) == want, (k, j)
     assert (cm.invfft_uni(Y, w, p) == X).all()
+
+
+@pytest.mark.parametrize("p,top", [(P1, 15), (P2, 15), (12289, 12), (65537, 14)])
+def test_tree_levels_with_wrapped_leading_terms(cm, orc, p, top):
+    """Levels above 8 multiply whole monic nodes on exactly their length: the
+    leading term wraps onto the constant one.  Zero, equal and largest points
+    make constant terms 0 and p - 1."""
+    for k in range(9, top + 1):
+        rng = np.random.default_rng(k)
+        for pts in (rng.integers(0, p, 1 << k, dtype=np.int32), np.zeros(1 << k, np.int32),
+                    np.full(1 << k, p - 1, np.int32)):
+            tree = cm.subproduct_tree(pts, p)
+            lev = tree[k - 1]
+            want = orc.ntt_polymul(lev[0], lev[1], p) if (1 << k) < p - 1 else None
+            for i in range(9, k + 1):
+                a, b = tree[i - 1][-2], tree[i - 1][-1]
+                assert int(tree[i][-1][-1]) == 1
+                low = orc.plain_polymul(a[:40], b[:40], p)[:40]
+                assert (tree[i][-1][:40] == low).all(), (p, k, i)
+                high = orc.plain_polymul(a[::-1][:40].copy(), b[::-1][:40].copy(), p)[:40]
+                assert (tree[i][-1][::-1][:40] == high).all(), (p, k, i)
+            x = int(pts[1])
+            assert int(orc.poly_eval(tree[k][0], np.array([x], np.int32), p)[0]) == 0
+            if want is not None and p % (1 << (k + 1)) == 1:
+                assert (tree[k][0] == want).all(), (p, k)
