@@ -5,7 +5,10 @@
 // by going down the subproduct tree, replacing each remainder by its
 // remainders modulo the two children.  It uses Newton-iteration inverses of
 // the reversed node polynomials (the "subinverse tree") for the divisions
-// above level plainMulLimit and plain division below.  Here:
+// above level plainMulLimit and plain division below.  The values alone come
+// from the transposed algorithm (eval_mid.hip) where the modulus allows its
+// root product.  Here, for callers that keep the inverses or the remainders,
+// for fewer than 2^9 points and for the largest size of a modulus:
 //   * the subproduct tree is built by launch_subproduct_tree (tree.hip);
 //   * subinverse tree: I_i(j) = rev(M_i(j))^-1 mod x^(2^i).  At level L0 it
 //     comes from a direct power-series inversion (one thread per node).
@@ -375,6 +378,8 @@ hipError_t launch_fast_evaluation(const u32 *F_in, const u32 *pts, int k, u32 p,
 
     hipError_t e = launch_subproduct_tree(pts, k, p, tree, fam, s);
     if (e != hipSuccess) return e;
+    if (!(keep && (keep->rem || keep->trees_only)) && evaluate_transposed_takes(k, fam))
+        return launch_evaluate_transposed(F_in, k, tree, inv, values, fam, s);
     // ---- subinverse tree, levels L0 .. k-1: levels L0 .. pinv in one launch
     // (k_inv_bottom) when pinv = min(k - 1, kEvalFuse) > L0, else the base
     // level alone (k_inv_base); Newton steps up from there

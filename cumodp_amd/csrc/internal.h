@@ -192,8 +192,8 @@ struct FourStepIO {
     int64_t g_stride = -1;   // stride of g_in when it differs from in_stride
     // pair a takes array a >> g_shift of g (g_ws has cnt >> g_shift arrays) and
     // writes output a ^ out_xor, words out_from .. h_len - 1; monic: operands
-    // are monic of n/2 + 1 words, outputs monic of n + 1
-    int g_shift = 0, out_from = 0, out_xor = 0, monic = 0;
+    // are monic of n/2 + 1 words, outputs monic of n + 1; neg: outputs negated
+    int g_shift = 0, out_from = 0, out_xor = 0, monic = 0, neg = 0;
 };
 hipError_t launch_mul_four_step(int k, const FourStepIO &io, const Family *fam, hipStream_t s);
 // the same with tables the caller looked up (no table is built here)
@@ -204,6 +204,19 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
 // words) is the product of nodes 2d and 2d + 1 of `prev` (2^(i-1) + 1 words).
 hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, const Family *fam,
                              hipStream_t s);
+
+// Middle products of one shape on 2^logn points (9 <= logn <= kMaxLog): product
+// a reads lf words at f + a fs and lg words at g + (a >> 1) gs and writes words
+// from .. from + len - 1 of the cyclic product to h + (a ^ 1) hs (a single
+// product: fs, gs and hs 0).  neg: negated (logn > kMaxLdsLog only).
+struct MidProduct {
+    const u32 *f, *g;
+    int64_t fs, gs, hs, lf, lg;
+    u32 *h;
+    int64_t from, len;
+    int cnt, neg;
+};
+hipError_t launch_mul_middle(int logn, const MidProduct &q, const Family *fam, hipStream_t s);
 
 // count products of one shape: product d reads lf words at F + d fs and lg
 // words at G + d gs and writes the first lh words of the 2^logn-point cyclic
@@ -303,6 +316,12 @@ int64_t eval_inverse_offset(int k);
 // tree level 0 in the reference's layout: (-x, 1) per point, the first nh
 // points to left, the next nh to right (2 nh words each)
 hipError_t launch_ref_leaves(const u32 *pts, int64_t nh, u32 *left, u32 *right, hipStream_t s);
+// the values alone, by the transposed algorithm (eval_mid.hip), from the
+// subproduct tree at `tree` and 4 2^k further words at `work`, where
+// evaluate_transposed_takes holds
+bool evaluate_transposed_takes(int k, const Family *fam);
+hipError_t launch_evaluate_transposed(const u32 *F, int k, const u32 *tree, u32 *work, u32 *values,
+                                      const Family *fam, hipStream_t s);
 hipError_t launch_fast_evaluation(const u32 *F, const u32 *pts, int k, u32 p, u32 *values,
                                   u32 *scratch, const Family *fam, hipStream_t s,
                                   const EvalKeep *keep = nullptr);

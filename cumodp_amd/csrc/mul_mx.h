@@ -79,10 +79,10 @@ CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const
 // The mirror: digit-reversed rows in, natural rows out (canonical, words at or
 // beyond lim, relative to Y, not stored).  EDGES: words below `from` are not
 // stored either, and word `fix` is stored less one (tests that cost the plain
-// form 7%).
+// form 7%); neg negates all.
 template <int LOGL, int LOGC, int V, bool EDGES>
-CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fix, int logn2,
-                       const MxCtx &cx) {
+CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fix, bool neg,
+                       int logn2, const MxCtx &cx) {
     static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
                   "a wave's 256 V words lie inside the tile");
     using P = MxPlan<LOGL, LOGC>;
@@ -114,6 +114,7 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fi
         for (int s = 0; s < V; ++s) {
             x[s][r] = mx_canon(x[s][r], cx);
             if (EDGES && e + s == fix) x[s][r] = cm_sub(x[s][r], 1u, cx.p);
+            if (EDGES && neg) x[s][r] = cm_sub(0u, x[s][r], cx.p);
         }
         if constexpr (V == 4) {
             if ((!EDGES || e >= from) && e + V <= lim) {

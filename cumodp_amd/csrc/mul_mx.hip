@@ -6,7 +6,7 @@
 
 namespace cm {
 
-enum : int { kStrided = 0, kDesc = 1, kMonic = 2 };
+enum : int { kStrided = 0, kDesc = 1, kMonic = 2, kMiddle = 3 };
 
 // A single product is bound by its serial chain (load, rounds, exchanges), many
 // products by vector issue.  One 2048-point product mod 469762049, back to
@@ -20,7 +20,8 @@ enum : int { kStrided = 0, kDesc = 1, kMonic = 2 };
 // otherwise product d reads F + d * one.f, G + d * one.g (one.lf / one.lg
 // words) and writes H + d * one.h (one.lh words); kMonic: the same with monic
 // operands of 2^LOGL / 2 + 1 words, whose product's leading term wraps onto word
-// 0 and is put into word 2^LOGL.  H may alias F or G: a
+// 0 and is put into word 2^LOGL; kMiddle: product d of G array d >> 1 goes to
+// output d ^ 1, from word one.logn on.  H may alias F or G: a
 // product's words are all loaded before any of its words is stored, by the
 // same wave or on the other side of a barrier.
 template <int LOGL, int LOGW, int V, int DESC>
@@ -42,7 +43,9 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
                 m = descs ? descs[d] : one;
             } else {
                 m = one;
-                m.f = (int64_t)d * one.f; m.g = (int64_t)d * one.g; m.h = (int64_t)d * one.h;
+                m.f = (int64_t)d * one.f;
+                m.g = (int64_t)(DESC == kMiddle ? d >> 1 : d) * one.g;
+                m.h = (int64_t)(DESC == kMiddle ? d ^ 1 : d) * one.h;
             }
         }
         return m;
@@ -68,14 +71,15 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_mul_mx(
             if (((Map::base() + Map::off(s, 0)) & ((1 << LOGL) - 1)) == 0)
                 x[0][s][0] = cm_sub(mx_canon(x[0][s][0], cx), 1u, cx.p);
     }
-    mx_store_rows<LOGL, V>(
+    mx_store_rows<LOGL, V, DESC == kMiddle>(
         x[0],
         [&](int s, u32 *&q, int &len) {
             const MulDesc m = desc(s);
             q = H + m.h;
             len = std::min(m.lh, 1 << LOGL);
         },
-        cx);
+        cx, one.logn);
+    if (DESC == kMiddle) return;
     // words beyond the transform size (lh > L) are zero, or the leading 1
     for (int c = 0; c < C; ++c) {
         const int d = blockIdx.x * C + c;
@@ -179,6 +183,38 @@ hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, co
     return hipSuccess;
 }
 
+hipError_t launch_mul_middle(int logn, const MidProduct &q, const Family *fam, hipStream_t s) {
+    const int64_t n = (int64_t)1 << logn;
+    if (q.cnt < 1 || q.from < 0 || q.from + q.len > n || (q.cnt > 1 && (q.cnt & 1)))
+        return hipErrorInvalidValue;
+    u32 *h = q.h - q.from;
+    const MulDesc sd{q.fs, q.gs, q.hs, (int)q.lf, (int)q.lg, (int)(q.from + q.len), (int)q.from};
+    switch (logn) {
+#define CM_CASE(K) \
+    case K: return q.neg ? hipErrorInvalidValue \
+                         : mul_mx_t<K, kMiddle>(q.f, q.g, h, nullptr, q.cnt, sd, fam, s);
+        CM_CASE(9) CM_CASE(10) CM_CASE(11) CM_CASE(12) CM_CASE(13)
+#undef CM_CASE
+    }
+    // four-step, in chunks whose two slabs stay within 1 GiB each
+    const int64_t chunk = std::max<int64_t>(2, ((int64_t)1 << 28) / n);
+    for (int64_t c0 = 0; c0 < q.cnt; c0 += chunk) {
+        const int cnt = (int)std::min<int64_t>(chunk, q.cnt - c0), pairs = cnt > 1;
+        u32 *sf = (u32 *)workspace(5, sizeof(u32) * (size_t)(n * cnt), s);
+        u32 *sg = (u32 *)workspace(6, sizeof(u32) * (size_t)(n * (cnt >> pairs)), s);
+        if (!sf || !sg) return hipErrorOutOfMemory;
+        FourStepIO io{q.f + c0 * q.fs, q.g + (c0 >> 1) * q.gs, q.lf, q.lg, q.fs, sf, sg,
+                      h + c0 * q.hs, q.from + q.len, q.hs, cnt};
+        io.g_stride = q.gs;
+        io.g_shift = io.out_xor = pairs;
+        io.out_from = (int)q.from;
+        io.neg = q.neg;
+        const hipError_t e = launch_mul_four_step(logn, io, fam, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // ---------------------------------------------------------------------------
 // four-step multiply: an n-word array viewed as 2^k1 rows x 2^k2 columns
 // ---------------------------------------------------------------------------
@@ -186,12 +222,12 @@ hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, co
 // for e < in_len (zero beyond) and writes out[(a ^ out_xor) out_stride + e] for
 // out_from <= e < out_len.  monic: the product of two monic polynomials of
 // half the length, whose x^n wrapped onto word 0: that word less one, and a
-// leading 1 in word n.
+// leading 1 in word n.  neg: outputs negated.
 struct MxCols {
     const u32 *in;
     u32 *out;
     int64_t in_stride, in_len, out_stride, out_len;
-    int out_from = 0, out_xor = 0, monic = 0;
+    int out_from = 0, out_xor = 0, monic = 0, neg = 0;
 };
 
 // Forward column transforms of 2^LOGC columns per workgroup (mx_col_fwd).
@@ -210,7 +246,7 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_fwd_mx(MxCols s0, MxCols s
 }
 
 // Inverse column transforms (mx_col_inv), truncated to out_len.  EDGES: sets
-// with out_from, out_xor or monic.
+// with out_from, out_xor, monic or neg.
 template <int LOGL, int LOGC, int V, bool EDGES>
 __global__ __launch_bounds__((1 << (LOGL + LOGC)) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_inv_mx(MxCols S, int logn2, MxCtx cx) {
@@ -219,7 +255,7 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_inv_mx(MxCols S, int logn2
     const int c0 = mx_xcd(blockIdx.x, gridDim.x) << LOGC;
     u32 *Y = S.out + (EDGES ? a ^ S.out_xor : a) * S.out_stride + c0;
     mx_col_inv<LOGL, LOGC, V, EDGES>(lds, S.in + a * S.in_stride + c0, Y, S.out_from - c0,
-                                     (int)(S.out_len - c0), S.monic ? -c0 : INT32_MIN, logn2, cx);
+                                     (int)(S.out_len - c0), S.monic ? -c0 : INT32_MIN, S.neg, logn2, cx);
     if (EDGES && S.monic && c0 == 0 && threadIdx.x == 0)
         Y[(int64_t)1 << (LOGL + logn2)] = 1u;
 }
@@ -245,7 +281,7 @@ static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int c
     constexpr int T = (1 << (LOGL + LOGC)) / (4 * V);
     ProfScope ps(inverse ? kProfColInv : kProfColFwd, s);
     const dim3 g(1u << (k2 - LOGC), cnt0 + cnt1);
-    if (inverse && (s0.out_from || s0.out_xor || s0.monic))
+    if (inverse && (s0.out_from || s0.out_xor || s0.monic || s0.neg))
         hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V, true>), g, dim3(T), 0, s, s0, k2, cx);
     else if (inverse)
         hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V, false>), g, dim3(T), 0, s, s0, k2, cx);
@@ -367,7 +403,7 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
     if (e == hipSuccess) e = launch_rows(io, o, fam, s);
     if (e != hipSuccess) return e;
     const MxCols sh{io.f_ws, io.h_out, n, n, io.out_stride, io.h_len,
-                    io.out_from, io.out_xor, io.monic};
+                    io.out_from, io.out_xor, io.monic, io.neg};
     return launch_cols(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, cx, s);
 }
 

@@ -484,9 +484,9 @@ CM_DEV void mx_load_rows(u32 (&x)[V][4], RowFn &&row) {
     }
 }
 
-// the same for canonical stores
-template <int LOGL, int V, class RowFn>
-CM_DEV void mx_store_rows(const u32 (&x)[V][4], RowFn &&row, const MxCtx &cx) {
+// the same for canonical stores; FROM: words below `from` are not stored
+template <int LOGL, int V, bool FROM = false, class RowFn>
+CM_DEV void mx_store_rows(const u32 (&x)[V][4], RowFn &&row, const MxCtx &cx, int from = 0) {
     constexpr int LOGS = MxPlan<LOGL>::words(0);
     using Map = MxMap<LOGS, V>;
     const int i0 = Map::base() & ((1 << LOGL) - 1);
@@ -500,12 +500,12 @@ CM_DEV void mx_store_rows(const u32 (&x)[V][4], RowFn &&row, const MxCtx &cx) {
             MxQuad v;
 #pragma unroll
             for (int s = 0; s < 4; ++s) v.v[s] = mx_canon(x[s][r], cx);
-            if (i + 4 <= len) {
+            if (i + 4 <= len && (!FROM || i >= from)) {
                 *(MxQuad *)(q + i) = v;
             } else {
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
-                    if (i + s < len) q[i + s] = v.v[s];
+                    if (i + s < len && (!FROM || i + s >= from)) q[i + s] = v.v[s];
             }
         }
     } else {
@@ -517,7 +517,7 @@ CM_DEV void mx_store_rows(const u32 (&x)[V][4], RowFn &&row, const MxCtx &cx) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int i = i0 + (Map::off(s, r) & ((1 << LOGL) - 1));
-                if (i < len) q[i] = mx_canon(x[s][r], cx);
+                if (i < len && (!FROM || i >= from)) q[i] = mx_canon(x[s][r], cx);
             }
         }
     }

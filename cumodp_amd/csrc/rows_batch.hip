@@ -142,7 +142,7 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_rows_col_inv(SRC src, int a0) 
     const int c0 = mx_xcd(blockIdx.x, tiles) << LOGC;
     u32 *X = S.f + ((int64_t)row << S.e) + c0;
     const MxCtx cx = S.cx;
-    mx_col_inv<LOGL, LOGC, V, false>(lds, X, X, 0, (1 << S.e) - c0, 0, logn2, cx);
+    mx_col_inv<LOGL, LOGC, V, false>(lds, X, X, 0, (1 << S.e) - c0, 0, false, logn2, cx);
 }
 
 template <class SRC, int LOGL, int V>

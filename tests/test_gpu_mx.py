@@ -226,3 +226,25 @@ def test_tree_levels_with_wrapped_leading_terms(cm, orc, p, top):
             assert int(orc.poly_eval(tree[k][0], np.array([x], np.int32), p)[0]) == 0
             if want is not None and p % (1 << (k + 1)) == 1:
                 assert (tree[k][0] == want).all(), (p, k)
+
+
+@pytest.mark.parametrize("p,ks", [(P1, (8, 9, 10, 11, 12, 13, 14, 15, 18)), (P2, (9, 13, 14)),
+                                  (TOP, (9, 16, 17)), (12289, (10, 11, 12))])
+def test_transposed_evaluation(cm, orc, p, ks):
+    """Values by the transposed algorithm (k >= 9 with 2^(k+1) | p - 1) against
+    the remainder tree, which runs when the remainders are kept, and Horner's
+    rule on a sample; coefficients are any 32-bit words."""
+    rng = np.random.default_rng(p + 3)
+    for k in ks:
+        n = 1 << k
+        pts = rng.integers(0, p, n, dtype=np.int32)
+        pts[0], pts[-1], pts[n // 2] = 0, p - 1, pts[1]
+        F = rng.integers(0, 1 << 32, n, dtype=np.uint64)
+        F[:3] = (1 << 32) - 1
+        got = cm.fast_evaluation(F.astype(np.uint32).view(np.int32), pts, p)
+        Fp = (F % p).astype(np.int32)
+        if k <= 14:
+            r = cm.eval_steps("fastEvaluation", pts, p, Fp, flag=1)
+            assert (got == np.concatenate([r["fL"][1], r["fR"][1]])).all(), (p, k)
+        idx = np.unique(np.concatenate([[0, 1, n // 2, n - 1], rng.integers(0, n, 60)]))
+        assert (got[idx] == orc.poly_eval(Fp, pts[idx], p)).all(), (p, k)
