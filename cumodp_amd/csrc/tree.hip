@@ -27,49 +27,76 @@ int64_t tree_level_offset(int k, int i) {
 }
 
 // Levels 0 .. pin of the tree in one launch: workgroup J (blockDim.x =
-// 2^pin threads, pin <= kTreeFuse) builds the subtree over points
+// kTreeParts 2^pin threads, 1 <= pin <= kTreeFuse) builds the subtree over points
 // J 2^pin .. J 2^pin + 2^pin - 1 in LDS, level by level, and writes every
-// level's nodes (a contiguous block of each level) to the tree.  Node
-// coefficient r of level i (children a, b of level i-1, h + 1 words each,
-// h = 2^(i-1)) is sum_u a_u b_(r-u), a schoolbook sum in a 64-bit
-// accumulator (accum.h); the leading coefficients are 1 and come out of the
-// same sum.
+// level's nodes (a contiguous block of each level) to the tree.  LDS holds the
+// nodes without their leading 1.  Word r of a node of 2h words (children a, b of
+// h words) is sum_u a_u b_(r-u) and, from the children's leading terms,
+// a_(r-h) + b_(r-h) for r >= h: a schoolbook sum in a 64-bit accumulator
+// (accum.h).
+//
+// Bound by the chain of LDS loads and multiply-adds of a thread: 256 one after
+// the other if a word has one thread.  The levels above 64 words split each sum
+// over kTreeParts threads; up to 64 words a node stays within a wave, which
+// needs no barrier.
 constexpr int kTreeFuse = 8;
+constexpr int kTreeParts = 4;
 
-__global__ __launch_bounds__(1 << kTreeFuse) void k_tree_bottom(const u32 *__restrict__ pts,
-                                                               int pin, PlainMod pm,
-                                                               u32 *__restrict__ tree,
-                                                               int64_t n) {
-    constexpr int BMAX = 1 << kTreeFuse;
-    __shared__ u32 buf[2][2 * BMAX];
+__global__ __launch_bounds__(kTreeParts << kTreeFuse) void k_tree_bottom(
+    const u32 *__restrict__ pts, int pin, PlainMod pm, u32 *__restrict__ tree, int64_t n) {
+    constexpr int BMAX = 1 << kTreeFuse, WAVE = 6;
+    __shared__ u32 buf[2][BMAX], pp[kTreeParts * BMAX];
+    static_assert(kTreeParts == 4, "the partial sums are added as four terms");
     const int B = 1 << pin;
     const int64_t J = blockIdx.x;
-    const int t = threadIdx.x;
-    {
-        const u32 x = pts[J * B + t] % pm.p;
-        const u32 lo = x ? pm.p - x : 0u;
-        buf[0][2 * t] = lo;
-        buf[0][2 * t + 1] = 1u;
-        tree[2 * (J * B + t)] = lo;
-        tree[2 * (J * B + t) + 1] = 1u;
+    const int tid = threadIdx.x, t = tid & (B - 1), part = tid >> pin;
+    const u32 p = pm.p;
+    // word r of node c of level i, of 2h words, to the tree; then its leading 1
+    auto put = [&](int i, int64_t off, u32 v) {
+        const int H = 1 << i, c = t >> i, r = t & (H - 1);
+        u32 *out = tree + off + ((J << (pin - i)) + c) * (H + 1) + r;
+        buf[i & 1][t] = v;
+        out[0] = v;
+        if (r == H - 1) out[1] = 1u;
+    };
+    // part q of the sum of word t of level i, and what the leading terms add
+    auto sum = [&](int i, int q, int parts) {
+        const int h = 1 << (i - 1), r = t & (2 * h - 1);
+        const u32 *a = buf[(i - 1) & 1] + (t - r), *b = a + h;
+        const int lo = r < h ? 0 : r - h + 1, cnt = r < h ? r + 1 : 2 * h - 1 - r;
+        const int k0 = cnt * q / parts, k1 = cnt * (q + 1) / parts;
+        return plain_dot<1, -1>(a + lo + k0, b + (r - lo - k0), k1 - k0, pm);
+    };
+    auto lead = [&](int i) {
+        const int h = 1 << (i - 1), r = t & (2 * h - 1);
+        const u32 *a = buf[(i - 1) & 1] + (t - r);
+        return r < h ? 0u : cm_add(a[r - h], a[r], p);
+    };
+    int64_t off = 0;                          // level i of the tree
+    if (part == 0) {
+        const u32 x = pts[J * B + t] % p;
+        put(0, 0, x ? p - x : 0u);
     }
-    int64_t off = 0;                          // word offset of level i - 1 in the tree
-    for (int i = 1; i <= pin; ++i) {
+#pragma unroll
+    for (int i = 1; i <= WAVE; ++i) {
+        if (i > pin) return;
+        off += (n >> (i - 1)) * ((1 << (i - 1)) + 1);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (part == 0) put(i, off, cm_add(sum(i, 0, 1), lead(i), p));
+    }
+#pragma unroll
+    for (int i = WAVE + 1; i <= kTreeFuse; ++i) {
+        if (i > pin) return;
+        off += (n >> (i - 1)) * ((1 << (i - 1)) + 1);
         __syncthreads();
-        const int h = 1 << (i - 1);
-        const int len = 2 * h + 1, nodes = B >> i;
-        off += (n >> (i - 1)) * (h + 1);      // level i
-        const u32 *prev = buf[(i - 1) & 1];
-        u32 *cur = buf[i & 1];
-        u32 *out = tree + off + (J * nodes) * len;
-        for (int x = t; x < nodes * len; x += B) {
-            const int c = x / len, r = x - c * len;
-            const u32 *a = prev + (2 * c) * (h + 1), *b = a + (h + 1);
-            const int lo = r > h ? r - h : 0, hi = r < h ? r : h;
-            const u32 v = plain_dot<1, -1>(a + lo, b + (r - lo), hi - lo + 1, pm);
-            cur[x] = v;
-            out[x] = v;
-        }
+        pp[tid] = sum(i, part, kTreeParts);
+        __syncthreads();
+        if (part == 0)
+            put(i, off, cm_add(cm_add(cm_add(pp[t], pp[B + t], p),
+                                      cm_add(pp[2 * B + t], pp[3 * B + t], p), p),
+                               lead(i), p));
     }
 }
 
@@ -78,8 +105,8 @@ hipError_t launch_subproduct_tree(const u32 *pts, int k, u32 p, u32 *tree, const
     const int64_t n = (int64_t)1 << k;
     // levels 0 .. pin in one launch, one workgroup per 2^pin points
     const int pin = k < kTreeFuse ? k : kTreeFuse;
-    hipLaunchKernelGGL(k_tree_bottom, dim3((unsigned)(n >> pin)), dim3(1 << pin), 0, s, pts, pin,
-                       plain_mod(p), tree, n);
+    hipLaunchKernelGGL(k_tree_bottom, dim3((unsigned)(n >> pin)), dim3(kTreeParts << pin), 0, s, pts,
+                       pin, plain_mod(p), tree, n);
     hipError_t e = hipGetLastError();
     for (int i = pin + 1; i <= k && e == hipSuccess; ++i) {
         e = launch_tree_level(i, tree + tree_level_offset(k, i - 1),
