@@ -152,13 +152,22 @@ hipError_t launch_mul_lds_strided(int logn, const u32 *F, const u32 *G, u32 *H, 
     return hipErrorInvalidValue;
 }
 
+// 2 to 32 products of 2^13 points leave most of the chip idle as one workgroup
+// each (15 us): as four-step multiplies on 2^5 x 2^8 words they take three
+// launches of 3.5 us.  Trees of 2^14, 2^16 and 2^18 points: 58.7, 81.3 and 122.8
+// us with workgroups, 52.2, 76.2 and 119.8 so; at 64 products both take the
+// same and at 128 the workgroups win.  A single product, queued from the host,
+// waits for three launches instead of one: 12.2 us either way.
+static bool four_step_13(int logn, int64_t count) {
+    return logn == kMaxLdsLog && count >= 2 && count <= 32;
+}
 
 hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, const Family *fam,
                              hipStream_t s) {
     const int64_t h = (int64_t)1 << (i - 1), n = 2 * h;
     if (nodes <= 0 || nodes > INT32_MAX) return hipErrorInvalidValue;
     const MulDesc sd{2 * (h + 1), 2 * (h + 1), n + 1, (int)(h + 1), (int)(h + 1), (int)(n + 1), i};
-    switch (i) {
+    switch (four_step_13(i, nodes) ? 0 : i) {
 #define CM_CASE(K)                                                                        \
     case K:                                                                               \
         return mul_mx_t<K, kMonic>(prev, prev + (h + 1), cur, nullptr, (int)nodes, sd, fam, s);
@@ -189,7 +198,7 @@ hipError_t launch_mul_middle(int logn, const MidProduct &q, const Family *fam, h
         return hipErrorInvalidValue;
     u32 *h = q.h - q.from;
     const MulDesc sd{q.fs, q.gs, q.hs, (int)q.lf, (int)q.lg, (int)(q.from + q.len), (int)q.from};
-    switch (logn) {
+    switch (four_step_13(logn, q.cnt) ? 0 : logn) {
 #define CM_CASE(K) \
     case K: return q.neg ? hipErrorInvalidValue \
                          : mul_mx_t<K, kMiddle>(q.f, q.g, h, nullptr, q.cnt, sd, fam, s);
@@ -392,7 +401,7 @@ static hipError_t launch_rows(const FourStepIO &io, const Outer *o, const Family
 
 hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, const Outer *o,
                                      hipStream_t s) {
-    if (!o || o->k > fam->K || o->k <= kMaxLdsLog) return hipErrorInvalidValue;
+    if (!o || o->k > fam->K || o->k < kMaxLdsLog) return hipErrorInvalidValue;
     const int64_t n = (int64_t)1 << o->k;
     const MxCols sf{io.f_in, io.f_ws, io.in_stride, io.f_len, n, n};
     const MxCols sg{io.g_in, io.g_ws, io.g_stride < 0 ? io.in_stride : io.g_stride, io.g_len, n, n};
@@ -408,7 +417,7 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
 }
 
 hipError_t launch_mul_four_step(int k, const FourStepIO &io, const Family *fam, hipStream_t s) {
-    if (k <= kMaxLdsLog || k > kMaxLog || k > fam->K) return hipErrorInvalidValue;
+    if (k < kMaxLdsLog || k > kMaxLog || k > fam->K) return hipErrorInvalidValue;
     const Outer *o = outer_for(fam, k);
     if (!o) return hipErrorOutOfMemory;
     return launch_mul_four_step_with(io, fam, o, s);

@@ -210,8 +210,14 @@ int nominal_split(int k) {
 
 // The nominal value stands for the library's own choice: columns short enough
 // that both passes fill the chip (measured over every split of 2^14 .. 2^24).
-// Columns have 2^4 .. 2^12 words.
+// Columns have 2^4 .. 2^12 words.  2^13 points (a few products of a tree level)
+// have no choice.
 void four_step_split(int k, int &k1, int &k2) {
+    if (k <= kMaxLdsLog) {
+        k1 = 5;
+        k2 = k - k1;
+        return;
+    }
     static const int own[kMaxLog - kMaxLdsLog] = {6, 6, 6, 7, 8, 8, 8, 8, 10, 10, 11, 11, 12};
     const int c = nominal_split(k);
     k1 = c == default_split(k) ? own[k - kMaxLdsLog - 1] : k - c;
