@@ -153,129 +153,282 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 
 // ---- one launch for the whole list ------------------------------------------
 // One launch for every product of a list call up to 2^15 points, schoolbook
-// and NTT alike: one workgroup per task (1024 threads, about 136 KiB of LDS,
-// so one per CU at a time).  Each workgroup takes its task from a list in
-// descending order of estimated cost through an atomic counter, so the tasks
-// start largest first whatever order the hardware dispatches workgroups in:
-//   * tile: 16384 words of products of one size 2^logn <= 2^14 (16384 >>
-//     logn products; one 2^14 product), multiplied in LDS as by k_mul_mixed;
-//   * big half: one of the two 2^14-point halves (cyclic, negacyclic) of a
-//     2^15-point product, recombined by a short kernel after the launch;
-//   * plain: 4096 consecutive outputs of one schoolbook product (16 waves of
+// and NTT alike: one workgroup of 512 threads and 68 KiB of LDS per task, so
+// that two run on a CU and one's loads and stores go on under the other's
+// transforms.  Each workgroup takes its task from a list in descending order of
+// estimated cost through an atomic counter, so the tasks start largest first
+// whatever order the hardware dispatches workgroups in:
+//   * tile: 8192 words of products of one size 2^logn <= 2^13 (8192 >> logn
+//     products), multiplied in LDS;
+//   * big: a product of 2^14 or 2^15 points, modulo 2 to 4 factors x^8192 -
+//     omega one after the other (omega = 1, -1, i, -i; 3 reach 24576 words), or
+//     one of them when the list has too few tasks for the chip; then a short
+//     kernel recombines them after the launch;
+//   * plain: 2048 consecutive outputs of one schoolbook product (8 waves of
 //     256 outputs, each wave on its own, the arithmetic of k_plain_mul).
-// The 4096 uneven pairs (degrees 32 .. 16384) take 226 us per call with the
-// tile products on the matrix cores, 256 us as radix-2 butterflies.
+// Bound by vector issue (59.9 M wave instructions of 6.9 cycles on 1024 SIMDs,
+// most of them 32-bit multiplies).  4096 pairs of degrees 32 .. 16384: 197 us per
+// call against 226 us with 1024 threads and 16384-word tiles, one workgroup per
+// CU, 2^15 points as two halves; a product of up to 12288 words as 8192 + 4096
+// points takes 5 us of that.  2^24 points in all of 2^13-point products take 96
+// us, of 2^14 117 us (twists and two reads of the operands), of 2^15 142 us in
+// four pieces and 100 us in three.
 // Largest tasks first keeps the tail short; the counter starts at zero in
 // every call's uploaded descriptor blob.  (A loop over tasks in fewer
 // workgroups was measured slower: inlined into the loop, the task bodies'
 // thread-index arithmetic is hoisted out of it and spills, and called out of
 // line they take their uniform pointers in vector registers.)
-constexpr int kPT = 1024;                    // threads of the persistent workgroup
-constexpr int kPW = 16384;                   // words per product tile
-constexpr int kPlainTaskOut = 4096;          // outputs of a plain task (16 waves x 256)
+constexpr int kPT = 512;                     // threads of the persistent workgroup
+constexpr int kPLog = 13;
+constexpr int kPW = 1 << kPLog;              // words per product tile
+constexpr int kPlainTaskOut = kPT / 64 * 256;   // outputs of a plain task
 constexpr int kPlainJT = 512;                // B coefficients per pass of a plain task
 
-enum : int32_t { kTaskTile = 0, kTaskBigCyc = 1, kTaskBigNeg = 2, kTaskPlain = 3 };
+enum : int32_t { kTaskTile = 0, kTaskBig = 1, kTaskPlain = 2 };
 
 struct ListTask {
     int32_t kind;
-    int32_t first;   // tile: first descriptor; big half, plain: the descriptor
-    int32_t count;   // tile: products; big half: the product's scratch slot;
-                     // plain: first output of the task
-    int32_t logn;    // tile: transform size
+    int32_t first;   // tile: first descriptor; else the descriptor
+    int32_t count;   // tile: products; big: pieces, kShort, or the product's slot in the
+                     // scratch; plain: first output of the task
+    int32_t logn;    // tile: transform size; big: -1 for all pieces, or which
 };
 
-// One 2^15-point product as two 2^14-point products in LDS (n = 2^14, the
-// F and G tiles of a 2^15-point product would not fit together):
-//   A = H mod x^n - 1, the cyclic product of F_lo + F_hi and G_lo + G_hi;
-//   B = H mod x^n + 1, the negacyclic product of F_lo - F_hi and G_lo - G_hi,
-//       taken as the cyclic product of the operands twisted by psi^i (psi a
-//       primitive 2^15-th root, psi^n = -1) and untwisted by psi^-i.
-// Then 2 H_i = A_i + psi^-i B'_i and 2 H_(n+i) = A_i - psi^-i B'_i.  psi^i and
-// psi^-i are entries of the 2^15 level tables.
-// The halves are separate tasks: the cyclic one leaves A in H_0 .. H_(n-1)
-// (inside the output: the product has more than n coefficients), the
-// negacyclic one psi^-i B' in the product's slot of the scratch S, and
-// k_big_combine adds, subtracts and halves them after the launch.
-template <bool NEGA>
-CM_DEV void task_big_half(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp,
-                          u32 *S, int slot, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
-    constexpr int LOGN = 14, n = 1 << LOGN, V = 4, LT = LOGN - 4;
-    using Map = MxMap<LT, V>;
-    const MulDesc d = *dp;
+constexpr int32_t kShort = -1;   // ListTask::count of a product of up to 3/2 kPW words
+
+// Pieces modulo x^kPW - omega that a product of `words` words needs.
+static int big_pieces(int words) { return (words + kPW - 1) / kPW; }
+
+// x[0] <- (canonical, natural order) the product d modulo x^kPW - omega, omega =
+// 1, -1, i, -i for q = 0 .. 3 (i = w_4): the operands' chunks of kPW words are
+// folded by powers of omega, twisted by psi^j (psi^kPW = omega: w_2M, w_4M or
+// its inverse, M = kPW; entries of the level tables) and untwisted after the
+// cyclic product.
+CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u32 *G,
+                      const MulDesc &d, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
+    constexpr int V = 4, M = kPW;
+    using Map = MxMap<kPLog - 4, V>;
     const int i0 = Map::base();
-    MxMat m;
-    u32 x[2][V][4], tw[V][4];
-    mx_forward_begin<LOGN, 0, V>(m, tw, cx);
-    // F_lo +- F_hi (the sum of two residues fits a word; p is added to the
-    // difference), the negacyclic operands times psi^i
-    auto operand = [&](u32 (&y)[V][4], const u32 *q, int len) {
+    const u32 p = cx.p;
+    const int lev = q == 1 ? M - 1 : 2 * M - 1;
+    const u32 *const tw_f = (q == 3 ? lvi : lv) + lev, *const tw_i = (q == 3 ? lv : lvi) + lev;
+    auto operand = [&](u32 (&y)[V][4], const u32 *src, int len) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = i0 + Map::off(0, r);
-            MxQuad lo, hi;
-            if (i + 4 <= len) {
-                lo = *(const MxQuad *)(q + i);
-            } else {
+            auto chunk = [&](int c) {
+                MxQuad v;
+                const int k = c * M + i;
+                if (k + 4 <= len) {
+                    v = *(const MxQuad *)(src + k);
+                } else {
 #pragma unroll
-                for (int s = 0; s < 4; ++s) lo.v[s] = i + s < len ? q[i + s] : 0u;
+                    for (int s = 0; s < 4; ++s) v.v[s] = k + s < len ? src[k + s] : 0u;
+                }
+                return v;
+            };
+            MxQuad a = chunk(0), b = chunk(1);
+            if (len > 2 * M) {
+                const MxQuad c = chunk(2), e = chunk(3);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    a.v[s] = cm_add(a.v[s], q < 2 ? c.v[s] : cm_sub(0u, c.v[s], p), p);
+                    b.v[s] = cm_add(b.v[s], q < 2 ? e.v[s] : cm_sub(0u, e.v[s], p), p);
+                }
             }
-            if (n + i + 4 <= len) {
-                hi = *(const MxQuad *)(q + n + i);
-            } else {
+            if (q < 2) {
 #pragma unroll
-                for (int s = 0; s < 4; ++s) hi.v[s] = n + i + s < len ? q[n + i + s] : 0u;
+                for (int s = 0; s < 4; ++s) y[s][r] = a.v[s] + (q ? p - b.v[s] : b.v[s]);
+            } else {   // omega psi^j = psi^(j + M)
+                const MxQuad w = *(const MxQuad *)(tw_f + i), w1 = *(const MxQuad *)(tw_f + M + i);
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    y[s][r] = cm_mul_tw(a.v[s], w.v[s], p, cx.np) +
+                              cm_mul_tw(b.v[s], w1.v[s], p, cx.np);
             }
-#pragma unroll
-            for (int s = 0; s < 4; ++s) y[s][r] = NEGA ? lo.v[s] - hi.v[s] + cx.p : lo.v[s] + hi.v[s];
         }
-        if constexpr (NEGA) {
+        if (q == 1) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const MxQuad w = *(const MxQuad *)(lv + n - 1 + i0 + Map::off(0, r));
+                const MxQuad w = *(const MxQuad *)(tw_f + i0 + Map::off(0, r));
 #pragma unroll
-                for (int s = 0; s < 4; ++s) y[s][r] = cm_mont_lazy(y[s][r], w.v[s], cx.p, cx.np);
+                for (int s = 0; s < 4; ++s) y[s][r] = cm_mont_lazy(y[s][r], w.v[s], p, cx.np);
             }
         }
+        mx_fence<V>();
     };
     operand(x[0], F + d.f, d.lf);
     operand(x[1], G + d.g, d.lg);
-    mx_tile_multiply<LOGN, V>(x, lds, lds + mx_lds_words(n), cx, m, tw);
-    u32 *out = NEGA ? S + (int64_t)slot * n : H + d.h;
+    MxMat m;
+    u32 tw[V][4];
+    mx_forward_begin<kPLog, 0, V>(m, tw, cx);
+    mx_tile_multiply<kPLog, V>(x, lds, lds + mx_lds_words(kPW), cx, m, tw);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (q == 0) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[0][s][r] = mx_canon(x[0][s][r], cx);
+        } else {
+            const MxQuad w = *(const MxQuad *)(tw_i + i0 + Map::off(0, r));
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[0][s][r] = cm_mul_tw(x[0][s][r], w.v[s], p, cx.np);
+        }
+    }
+}
+
+// The chunks h[c] (h = sum_c h[c] x^(c kPW)) from its residues a[q] modulo
+// x^kPW - omega_q, np = 2, 3 or 4 of them (h[3] = 0 for 3).
+CM_DEV void big_recombine(u32 (&a)[4], int np, u32 w4, u32 w4i, const MxCtx &cx) {
+    const u32 p = cx.p;
+    auto half = [&](u32 v) { return (v + (v & 1 ? p : 0u)) >> 1; };
+    const u32 s = half(cm_add(a[0], a[1], p)), d = half(cm_sub(a[0], a[1], p));
+    if (np == 2) {          // h0 + h2 = s, h1 + h3 = d
+        a[0] = s;
+        a[1] = d;
+        return;
+    }
+    u32 t, v;               // t = h0 - h2, v = h1 - h3
+    if (np == 3) {
+        v = d;
+        t = cm_sub(a[2], cm_mul_tw(d, w4, p, cx.np), p);
+    } else {
+        t = half(cm_add(a[2], a[3], p));
+        v = cm_mul_tw(half(cm_sub(a[2], a[3], p)), w4i, p, cx.np);
+    }
+    a[0] = half(cm_add(s, t, p));
+    a[2] = half(cm_sub(s, t, p));
+    a[1] = half(cm_add(d, v, p));
+    a[3] = half(cm_sub(d, v, p));
+}
+
+// Pieces q0 .. q1 - 1 of one product.  With S, a piece goes there; else all but
+// the last wait in the output (which has more than (q1 - 1) kPW words), each
+// word where this lane put it, and the last recombines them.
+CM_DEV void task_big(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp, int q0,
+                     int q1, u32 *S, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
+    using Map = MxMap<kPLog - 4, 4>;
+    const MulDesc d = *dp;
+    u32 x[2][4][4];
+    u32 *h = H + d.h;
+    const int i0 = Map::base();
+    for (int q = q0;; ++q) {
+        big_piece(q, x, lds, F, G, d, lv, lvi, cx);
+        if (q == q1 - 1 && !S) break;
+        u32 *out = S ? S : h + q * kPW;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *(MxQuad *)(out + i0 + Map::off(0, r)) =
+                MxQuad{{x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]}};
+        if (S) return;
+        __syncthreads();    // the next piece writes LDS words that others still read
+    }
+    const u32 w4 = lv[2], w4i = lvi[2];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int i = i0 + Map::off(0, r);
-        MxQuad v;
-        if constexpr (NEGA) {
-            const MxQuad w = *(const MxQuad *)(lvi + n - 1 + i);
+        MxQuad c[3] = {};
 #pragma unroll
-            for (int s = 0; s < 4; ++s) v.v[s] = cm_mont_lazy(x[0][s][r], w.v[s], cx.p, cx.np);
-        } else {
+        for (int q = 0; q < 3; ++q)
+            if (q < q1 - 1) c[q] = *(const MxQuad *)(h + q * kPW + i);
+        MxQuad o[4];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) v.v[s] = x[0][s][r];
+        for (int s = 0; s < 4; ++s) {
+            const u32 l = x[0][s][r];
+            u32 a[4] = {c[0].v[s], q1 == 2 ? l : c[1].v[s], q1 == 3 ? l : c[2].v[s], l};
+            big_recombine(a, q1, w4, w4i, cx);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q].v[s] = a[q];
         }
-        *(MxQuad *)(out + i) = v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q >= q1) break;
+            const int k = q * kPW + i;
+            if (k + 4 <= d.lh) {
+                *(MxQuad *)(h + k) = o[q];
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (k + s < d.lh) h[k + s] = o[q].v[s];
+            }
+        }
     }
 }
 
-// H_i = (A_i + S_i) / 2, H_(n+i) = (A_i - S_i) / 2 for the 2^15-point products
-// (descriptors descs[0 .. count), slot j at S + j n), canonical out.  A is a
-// matrix step's word (below p + 4200), S a Montgomery product's (below 2p).
-__global__ void k_big_combine(u32 *__restrict__ H, const MulDesc *__restrict__ descs,
-                              const u32 *__restrict__ S, MxCtx cx) {
-    constexpr int n = 1 << 14;
-    const MulDesc d = descs[blockIdx.y];
-    const u32 *Sp = S + (int64_t)blockIdx.y * n;
+// A product of kPW < words <= 3/2 kPW, with M = kPW / 2: A = H mod x^(2M) - 1 = (H0
+// + H2) + H1 x^M, then B = H mod x^M - i = H0 + i H1 - H2 on M points, which
+// leaves H2 = (A_lo + i A_hi - B) / 2.  A waits in the output.
+CM_DEV void task_big_short(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp,
+                           const u32 *lv, const u32 *lvi, const MxCtx &cx) {
+    constexpr int V = 2, L = kPLog - 1, M = 1 << L;
+    using Map = MxMap<L - 4, V>;
+    const MulDesc d = *dp;
     const u32 p = cx.p;
-    auto half = [&](u32 v) { return (v + (v & 1 ? p : 0u)) >> 1; };
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const u32 a = mx_canon(H[d.h + i], cx), u = cm_reduce2p(Sp[i], p);
-        H[d.h + i] = half(cm_add(a, u, p));
-        if (n + i < d.lh) H[d.h + n + i] = half(cm_sub(a, u, p));
+    u32 *h = H + d.h;
+    {
+        using Map4 = MxMap<kPLog - 4, 4>;
+        u32 x[2][4][4];
+        big_piece(0, x, lds, F, G, d, lv, lvi, cx);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *(MxQuad *)(h + Map4::base() + Map4::off(0, r)) =
+                MxQuad{{x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]}};
+    }
+    __syncthreads();        // A is read by other lanes, and so is the LDS
+    u32 x[2][V][4], tw[V][4];
+    MxMat m;
+    const int i0 = Map::base();
+    const u32 *const wf = lv + kPW - 1, *const wi = lvi + kPW - 1;   // psi^j, psi = w_4M
+    auto operand = [&](u32 (&y)[V][4], const u32 *q, int len) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int s = 0; s < V; ++s) {
+                const int j = i0 + Map::off(s, r);
+                const u32 a = j < len ? q[j] : 0u, b = M + j < len ? q[M + j] : 0u,
+                          c = 2 * M + j < len ? q[2 * M + j] : 0u;
+                y[s][r] = cm_mul_tw(cm_sub(a, c, p), wf[j], p, cx.np) +
+                          cm_mul_tw(b, wf[M + j], p, cx.np);
+            }
+    };
+    operand(x[0], F + d.f, d.lf);
+    operand(x[1], G + d.g, d.lg);
+    mx_forward_begin<L, 0, V>(m, tw, cx);
+    mx_tile_multiply<L, V>(x, lds, lds + mx_lds_words(M), cx, m, tw);
+    const u32 w4 = lv[2];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int s = 0; s < V; ++s) {
+            const int j = i0 + Map::off(s, r);
+            const u32 lo = h[j], hi = cm_mul_tw(h[M + j], w4, p, cx.np),
+                      b = cm_mul_tw(x[0][s][r], wi[j], p, cx.np);
+            const u32 e = cm_sub(cm_add(lo, hi, p), b, p), h2 = (e + (e & 1 ? p : 0u)) >> 1;
+            h[j] = cm_sub(lo, h2, p);
+            if (2 * M + j < d.lh) h[2 * M + j] = h2;
+        }
+}
+
+// The pieces of the products descs[0 .. count) (slot j at S + 4 j kPW) put
+// together.
+__global__ void k_big_combine(u32 *__restrict__ H, const MulDesc *__restrict__ descs,
+                              const u32 *__restrict__ S, const u32 *__restrict__ lv,
+                              const u32 *__restrict__ lvi, MxCtx cx) {
+    const MulDesc d = descs[blockIdx.y];
+    const u32 *Sp = S + (int64_t)blockIdx.y * (4 * kPW);
+    const int np = (d.lf + d.lg - 1 + kPW - 1) / kPW;
+    const u32 w4 = lv[2], w4i = lvi[2];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kPW; i += gridDim.x * blockDim.x) {
+        u32 a[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = q < np ? Sp[q * kPW + i] : 0u;
+        big_recombine(a, np, w4, w4i, cx);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (q < np && q * kPW + i < d.lh) H[d.h + q * kPW + i] = a[q];
     }
 }
 
-// Outputs c0 .. c0 + 4095 of the schoolbook product d: wave w computes the
+// Outputs c0 .. c0 + kPlainTaskOut - 1 of the schoolbook product d: wave w computes the
 // 256 outputs from c0 + 256 w on its own (its own LDS region, no workgroup
 // barrier; a wave past the end of the product leaves at once), lane t four of
 // them, with the arithmetic of k_plain_mul.  LDS operations of one wavefront
@@ -355,7 +508,7 @@ CM_DEV void task_plain(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDe
     }
 }
 
-// One tile of products of 2^K points (16384 >> K of them).
+// One tile of products of 2^K points (kPW >> K of them).
 template <int K>
 CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *d, int cnt,
                       const MxCtx &cx) {
@@ -390,7 +543,7 @@ CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDes
         cx);
 }
 
-__global__ __launch_bounds__(kPT) void k_list_persistent(
+__global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_list_persistent(
     const u32 *__restrict__ F, const u32 *__restrict__ G, u32 *__restrict__ H,
     const MulDesc *__restrict__ descs, const ListTask *__restrict__ tasks, int ntasks,
     int *__restrict__ counter, u32 *__restrict__ big_s, const u32 *__restrict__ lv,
@@ -405,10 +558,14 @@ __global__ __launch_bounds__(kPT) void k_list_persistent(
     const ListTask t = tasks[ti];
     if (t.kind == kTaskPlain) {
         task_plain(lds, F, G, H, descs + t.first, t.count, pm);
-    } else if (t.kind == kTaskBigCyc) {
-        task_big_half<false>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, cx);
-    } else if (t.kind == kTaskBigNeg) {
-        task_big_half<true>(lds, F, G, H, descs + t.first, big_s, t.count, lv, lvi, cx);
+    } else if (t.kind == kTaskBig) {
+        if (t.count == kShort) {
+            task_big_short(lds, F, G, H, descs + t.first, lv, lvi, cx);
+            return;
+        }
+        const bool all = t.logn < 0;
+        task_big(lds, F, G, H, descs + t.first, all ? 0 : t.logn, all ? t.count : t.logn + 1,
+                 all ? nullptr : big_s + ((int64_t)t.count * 4 + t.logn) * kPW, lv, lvi, cx);
     } else {
         const MulDesc *d = descs + t.first;
 #define CM_PMIX(K)                                       \
@@ -417,7 +574,7 @@ __global__ __launch_bounds__(kPT) void k_list_persistent(
         break;
         switch (t.logn) {
             CM_PMIX(4) CM_PMIX(5) CM_PMIX(6) CM_PMIX(7) CM_PMIX(8) CM_PMIX(9) CM_PMIX(10)
-            CM_PMIX(11) CM_PMIX(12) CM_PMIX(13) CM_PMIX(14)
+            CM_PMIX(11) CM_PMIX(12) CM_PMIX(13)
         default: break;
         }
 #undef CM_PMIX
@@ -728,9 +885,23 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     off[0] = 0;
     for (int c = 0; c < 33; ++c) off[c + 1] = off[c] + ncls[c];
     int64_t ntile = 0;
-    for (int e = 4; e < kBigLog; ++e) ntile += (ncls[e] + (kPW >> e) - 1) / (kPW >> e);
-    const int64_t nbig = ncls[kBigLog];
-    const int64_t ntasks = nplain_tasks + ntile + 2 * nbig;
+    for (int e = 4; e <= kPLog; ++e) ntile += (ncls[e] + (kPW >> e) - 1) / (kPW >> e);
+    const int64_t nbig = ncls[kPLog + 1] + ncls[kBigLog];
+    int64_t ntasks = nplain_tasks + ntile + nbig;
+    // Below four tasks per CU (two rounds of workgroups) a long task leaves the
+    // chip waiting at the end, so every piece is a task, at the price of a
+    // recombining pass over scratch (whose allocation a capture does without).
+    // 40 pairs of degrees 32 .. 16384: 26.5 us against 35.3 as 2^14-word
+    // workgroups, 1000 pairs: 82 us so and 105 with whole products.
+    u32 *big_s = nullptr;
+    if (nbig > 0 && ntasks < 4 * device_cus() && !stream_capturing(s)) {
+        big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig * 4 * kPW), s);
+        if (!big_s) return hipErrorOutOfMemory;
+        ntasks -= nbig;
+        for (int64_t i = 0; i < count; ++i)
+            if (!is_plain(descs[i]) && (descs[i].logn == kPLog + 1 || descs[i].logn == kBigLog))
+                ntasks += big_pieces(descs[i].lf + descs[i].lg - 1);
+    }
     if (ntasks > INT32_MAX) return hipErrorInvalidValue;
 
     // blob: the task counter (16 bytes), the sorted descriptors, the tasks;
@@ -768,7 +939,7 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
                     emit(ListTask{kTaskPlain, (int32_t)i, c0, 0}, (double)outs * lb / 8.0);
                 }
             }
-            for (int e2 = 4; e2 < kBigLog; ++e2) {
+            for (int e2 = 4; e2 <= kPLog; ++e2) {
                 const int per = kPW >> e2;
                 for (int64_t i = off[e2]; i < off[e2 + 1]; i += per) {
                     const int cnt = (int)std::min<int64_t>(per, off[e2 + 1] - i);
@@ -776,11 +947,16 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
                          3.0 * e2 * (double)cnt * (1 << (e2 - 1)));
                 }
             }
-            for (int64_t i = off[kBigLog]; i < off[kBigLog + 1]; ++i) {   // two 2^14-point halves
-                const int32_t slot = (int32_t)(i - off[kBigLog]);
-                const double half = 3.0 * (kBigLog - 1) * (1 << (kBigLog - 2));
-                emit(ListTask{kTaskBigCyc, (int32_t)i, slot, kBigLog}, half);
-                emit(ListTask{kTaskBigNeg, (int32_t)i, slot, kBigLog}, half);
+            for (int64_t i = off[kPLog + 1]; i < off[kBigLog + 1]; ++i) {
+                const int np = big_pieces(sorted[i].lf + sorted[i].lg - 1);
+                const double piece = 3.0 * kPLog * (1 << (kPLog - 1));
+                if (!big_s) {
+                    const bool sh = sorted[i].lf + sorted[i].lg - 1 <= kPW / 2 * 3;
+                    emit(ListTask{kTaskBig, (int32_t)i, sh ? kShort : np, -1},
+                         (sh ? 1.5 : np) * piece);
+                }
+                for (int q = 0; big_s && q < np; ++q)
+                    emit(ListTask{kTaskBig, (int32_t)i, (int32_t)(i - off[kPLog + 1]), q}, piece);
             }
         };
         int64_t nb[64] = {0};
@@ -798,11 +974,6 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     int *d_counter = (int *)dblob;
     const MulDesc *d_descs = (const MulDesc *)(dblob + desc_off);
     const ListTask *d_tasks = (const ListTask *)(dblob + task_off);
-    u32 *big_s = nullptr;   // psi^-i B' of each 2^15-point product, 2^14 words each
-    if (nbig > 0) {
-        big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig << 14), s);
-        if (!big_s) return hipErrorOutOfMemory;
-    }
     if (ntasks > 0) {
         ProfScope ps(kProfListPersistent, s);
         const dim3 grid((unsigned)ntasks);
@@ -812,10 +983,10 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    if (nbig > 0) {
+    if (big_s) {
         ProfScope ps(kProfListPersistent, s);
-        hipLaunchKernelGGL(k_big_combine, dim3(16, (unsigned)nbig), dim3(1024), 0, s, H,
-                           d_descs + off[kBigLog], big_s, mx_ctx(fam));
+        hipLaunchKernelGGL(k_big_combine, dim3(kPW / 1024, (unsigned)nbig), dim3(1024), 0, s, H,
+                           d_descs + off[kPLog + 1], big_s, fam->lv, fam->lvi, mx_ctx(fam));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -248,3 +248,39 @@ def test_transposed_evaluation(cm, orc, p, ks):
             assert (got == np.concatenate([r["fL"][1], r["fR"][1]])).all(), (p, k)
         idx = np.unique(np.concatenate([[0, 1, n // 2, n - 1], rng.integers(0, n, 60)]))
         assert (got[idx] == orc.poly_eval(Fp, pts[idx], p)).all(), (p, k)
+
+
+@pytest.mark.parametrize("p", [P1, P2])
+def test_list_products_in_pieces(cm, orc, p):
+    """List products above 2^13 points run modulo 2, 3 or 4 factors x^8192 - omega,
+    or 8192 + 4096 points up to 12288 words; in one task each when the list is
+    long and one task per factor when it is short.  The operands' chunks of
+    8192 words are folded, so one side is also taken shorter and longer than
+    that."""
+    rng = np.random.default_rng(p + 4)
+    words = (8193, 12287, 12288, 12289, 16384, 16385, 24576, 24577, 32768)
+    shapes = [(s, lf) for s in words for lf in (s // 2, s - 40, 41)]
+    F, G, want, items, fo, go = [], [], [], [], 0, 0
+    for s, lf in shapes:
+        lg = s + 1 - lf
+        f, g = (rng.integers(0, p, n, dtype=np.int32) for n in (lf, lg))
+        f[:2], g[:2] = p - 1, p - 1
+        items.append((fo, go, lf - 1, lg - 1))
+        F.append(f), G.append(g), want.append(orc.ntt_polymul(f, g, p))
+        fo, go = fo + lf, go + lg
+    dF = cm.DeviceArray.from_host(np.concatenate(F))
+    dG = cm.DeviceArray.from_host(np.concatenate(G))
+    for copies in (1, 40):
+        n = len(items) * copies
+        arr, ho = (cm.MulItem * n)(), 0
+        for i in range(n):
+            x = arr[i]
+            x.f_off, x.g_off, x.df, x.dg = items[i % len(items)]
+            x.h_off = ho
+            ho += x.df + x.dg + 1
+        H = cm.DeviceArray.from_host(np.full(ho, -1, np.int32))
+        cm.list_fftmul_dev(arr, dF, dG, H, p)
+        got = H.download()
+        for i in range(n):
+            w = want[i % len(items)]
+            assert (got[arr[i].h_off:arr[i].h_off + len(w)] == w).all(), (i, shapes[i % len(items)])
