@@ -27,9 +27,10 @@ constexpr int mx_col_lds() {
 
 // The forward pass of 2^24 points (2^11 rows, 8 columns per tile) takes 82 us
 // and the inverse 39 us, where the same addresses copied without a transform
-// take 36 and 26 us: one workgroup of 16 waves fits a CU (86 registers), so a
-// tile's loads, rounds and stores follow each other.  16 columns of 2^10 rows
-// (64-byte segments) take 71 and 34 us but leave rows of 2^14.
+// take 52 and 40 us: one workgroup of 16 waves fits a CU (86 registers), so a
+// tile's loads, rounds and stores follow each other (k_cols_loop of mul_mx.hip
+// overlaps them: 74 us).  16 columns of 2^10 rows (64-byte segments) take 71 and
+// 34 us but leave rows of 2^14.
 //
 // Forward transforms of 2^LOGC columns: rows straight from global memory into
 // the first round (words at or beyond lim, relative to X, are zero), the last
@@ -127,6 +128,140 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fi
             if ((!EDGES || e + s >= from) && e + s < lim) Y[e + s] = x[s][r];
     }
 }
+
+// The same passes over many tiles, one workgroup per CU for all of them
+// (mul_mx.hip, k_cols_loop): what a tile needs besides its words is loaded
+// once, so that the words of the next tile can be in flight during the rounds of
+// this one: the twiddles, which the columns of a tile and all tiles share, into
+// registers, the two matrices into LDS (both in registers would spill).
+template <int LOGL, int LOGC>
+struct MxCols4 {
+    static constexpr int V = 4, C = 1 << LOGC;
+    using P = MxPlan<LOGL, LOGC>;
+    static_assert(P::NR >= 2 && P::NR <= 3 && LOGC >= 2, "rounds");
+    static constexpr int kMats = 2 * kMxMatWords * 4;   // words of `mats`
+    const mx_v4i *mats;     // radix-16, and the last digit's
+    u32 tw[P::NR - 1][4];
+
+    CM_DEV void begin(bool inverse, u32 *lds_mats, const MxCtx &cx) {
+        mx_v4i *dst = (mx_v4i *)lds_mats;
+        const mx_v4i *src = cx.mat + (inverse ? kMxInv : kMxFwd) * kMxMatWords;
+        for (int i = threadIdx.x; i < kMxMatWords; i += blockDim.x) {
+            dst[i] = src[i];
+            dst[kMxMatWords + i] = src[P::T * kMxMatWords + i];
+        }
+        mats = dst + (threadIdx.x & 63);
+        __syncthreads();
+        const u32 *tab = inverse ? cx.ti : cx.tf;
+        u32 t[V][4];
+        mx_load_tw<P::logs(0), LOGC, V>(t, tab);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tw[0][r] = t[0][r];
+        if constexpr (P::NR == 3) {
+            mx_load_tw<P::logs(1), LOGC, V>(t, tab);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) tw[1][r] = t[0][r];
+        }
+    }
+    CM_DEV MxMat mat(bool last) const {
+        const mx_v4i *q = mats + (last && P::T ? kMxMatWords : 0);
+        return MxMat{q[0], q[64], q[128], q[192], q[256]};
+    }
+    CM_DEV static void mul(u32 (&x)[V][4], const u32 (&w)[4], const MxCtx &cx) {
+#pragma unroll
+        for (int s = 0; s < V; ++s)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[s][r] = cm_mont_lazy(x[s][r], w[r], cx.p, cx.np);
+        mx_fence<V>();
+    }
+    template <int J>
+    CM_DEV void forward(u32 (&x)[V][4], u32 *lds, const MxCtx &cx) const {
+        mx_dft<V>(x, mat(J == P::NR - 1), cx);
+        if constexpr (J < P::NR - 1) {
+            mul(x, tw[J], cx);
+            MxMap<P::words(J), V>::store(lds, x);
+            mx_sync<P::words(J), V>();
+            MxMap<P::words(J + 1), V>::load(lds, x);
+            forward<J + 1>(x, lds, cx);
+        }
+    }
+    template <int J>
+    CM_DEV void inverse(u32 (&x)[V][4], u32 *lds, const MxCtx &cx) const {
+        if constexpr (J < P::NR - 1) mul(x, tw[J], cx);
+        mx_dft<V>(x, mat(J == P::NR - 1), cx);
+        if constexpr (J > 0) {
+            MxMap<P::words(J), V>::store(lds, x);
+            mx_sync<P::words(J - 1), V>();
+            MxMap<P::words(J - 1), V>::load(lds, x);
+            inverse<J - 1>(x, lds, cx);
+        }
+    }
+    // natural rows (round 0's words; at or beyond lim: zero, or not stored).
+    // Quads beyond lim (none straddles it) are read at `safe` and cleared by
+    // clear_nat when the words are used: a branch here would wait for the
+    // loads before it.
+    CM_DEV static void load_nat(u32 (&x)[V][4], const u32 *X, const u32 *safe, int lim, int logn2) {
+        const int b = MxMap<P::words(0), V>::base();
+        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+        const u32 row = 1u << (logn2 + P::logs(0));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = (int)(off + r * row);
+            const MxQuad v = *(const MxQuad *)(e + V <= lim ? X + e : safe);
+#pragma unroll
+            for (int s = 0; s < V; ++s) x[s][r] = v.v[s];
+        }
+    }
+    CM_DEV static void clear_nat(u32 (&x)[V][4], int lim, int logn2) {
+        const int b = MxMap<P::words(0), V>::base();
+        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+        const u32 row = 1u << (logn2 + P::logs(0));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool in = (int)(off + r * row) + V <= lim;
+#pragma unroll
+            for (int s = 0; s < V; ++s) x[s][r] = in ? x[s][r] : 0u;
+        }
+    }
+    CM_DEV static void store_nat(u32 (&x)[V][4], u32 *Y, int lim, int logn2, const MxCtx &cx) {
+        const int b = MxMap<P::words(0), V>::base();
+        const u32 off = ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+        const u32 row = 1u << (logn2 + P::logs(0));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = (int)(off + r * row);
+            MxQuad v;
+#pragma unroll
+            for (int s = 0; s < V; ++s) v.v[s] = mx_canon(x[s][r], cx);
+            if (e + V <= lim) {
+                *(MxQuad *)(Y + e) = v;
+            } else {
+#pragma unroll
+                for (int s = 0; s < V; ++s)
+                    if (e + s < lim) Y[e + s] = v.v[s];
+            }
+        }
+    }
+    // digit-reversed rows
+    CM_DEV static u32 rev_offset(int logn2) {
+        const int b = MxMap<LOGC, V>::base();
+        return ((u32)(b >> LOGC) << logn2) + (b & (C - 1));
+    }
+    CM_DEV static void load_rev(u32 (&x)[V][4], const u32 *X, int logn2) {
+        const u32 *q = X + rev_offset(logn2);
+#pragma unroll
+        for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
+            const uint4 v = *(const uint4 *)q;
+            x[0][r] = v.x; x[1][r] = v.y; x[2][r] = v.z; x[3][r] = v.w;
+        }
+    }
+    CM_DEV static void store_rev(const u32 (&x)[V][4], u32 *Y, int logn2) {
+        u32 *q = Y + rev_offset(logn2);
+#pragma unroll
+        for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2)
+            *(uint4 *)q = make_uint4(x[0][r], x[1][r], x[2][r], x[3][r]);
+    }
+};
 
 // Words of a row tile: at least the 256 V words of a wave.
 template <int LOGL, int V>

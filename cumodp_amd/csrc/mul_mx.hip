@@ -269,6 +269,51 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_col_inv_mx(MxCols S, int logn2
         Y[(int64_t)1 << (LOGL + logn2)] = 1u;
 }
 
+// Both passes for arrays of many tiles: one workgroup per CU takes every
+// gridDim.x-th tile, in two LDS buffers, so a tile costs one barrier (a wave that
+// stores tile t + 2 has passed tile t + 1's barrier, which every wave reaches
+// after its loads of tile t).
+template <int LOGL, int LOGC, bool INV>
+__global__ __launch_bounds__((1 << (LOGL + LOGC)) / 16) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_cols_loop(MxCols s0, MxCols s1, int cnt0, int ntiles, int logn2, MxCtx cx) {
+    using K = MxCols4<LOGL, LOGC>;
+    __shared__ __align__(16) u32 lds[2][mx_col_lds<LOGL, LOGC>()], mats[K::kMats];
+    const int lx = logn2 - LOGC;    // log2 of the tiles of an array
+    K k;
+    k.begin(INV, mats, cx);
+    u32 x[4][4], next[4][4];
+    auto load = [&](u32 (&y)[4][4], int t) {
+        const int a0 = t >> lx, c0 = (t & ((1 << lx) - 1)) << LOGC;
+        const MxCols &S = a0 < cnt0 ? s0 : s1;
+        const int64_t a = a0 < cnt0 ? a0 : a0 - cnt0;
+        const u32 *X = S.in + a * S.in_stride + c0;
+        if constexpr (INV) K::load_rev(y, X, logn2);
+        else K::load_nat(y, X, S.in + a * S.in_stride, (int)(S.in_len - c0), logn2);
+    };
+    int t = mx_xcd(blockIdx.x, gridDim.x);
+    if (t < ntiles) load(next, t);
+    for (int b = 0; t < ntiles; t += gridDim.x, b ^= 1) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[s][r] = next[s][r];
+        if (t + (int)gridDim.x < ntiles) load(next, t + gridDim.x);
+        mx_fence<4>();
+        const int a0 = t >> lx, c0 = (t & ((1 << lx) - 1)) << LOGC;
+        const MxCols &S = a0 < cnt0 ? s0 : s1;
+        const int64_t a = a0 < cnt0 ? a0 : a0 - cnt0;
+        u32 *Y = S.out + a * S.out_stride + c0;
+        if constexpr (INV) {
+            k.template inverse<K::P::NR - 1>(x, lds[b], cx);
+            K::store_nat(x, Y, (int)(S.out_len - c0), logn2, cx);
+        } else {
+            K::clear_nat(x, (int)(S.in_len - c0), logn2);
+            k.template forward<0>(x, lds[b], cx);
+            K::store_rev(x, Y, logn2);
+        }
+    }
+}
+
 // Row pass (mx_row) over all rows of the arrays of F, in place.
 template <int LOGL, int V>
 __global__ __launch_bounds__((1 << mx_row_logw<LOGL, V>()) / (4 * V))
@@ -284,12 +329,34 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_row_mx(u32 *F, const u32 *__re
     mx_row<LOGL, V>(lds, F + t0, G + tg, (int)(blockIdx.x << (LOGW - LOGL)), k1, o, cx);
 }
 
+// Tiles of 16384 words that run as one workgroup per CU, two to eight for each
+// (the inverse, of one array, half as many).  Back to back, 2^22, 2^23 and 2^24
+// points: 50.0, 94.0 and 197.1 us with a workgroup per tile, 47.5, 88.8 and 193.3
+// us so (of new operands, 204 and 189 us at 2^24: repeated calls lower the
+// clock); at 2^25, beyond the last-level cache, 466 us without it and 475 with.
+// Operands whose last quad of words is not whole take a workgroup per tile.
+constexpr int64_t kLoopMin = 512, kLoopMax = 2048;
+
 template <int LOGL, int LOGC, int V>
 static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int cnt0, int cnt1,
                          int k2, const MxCtx &cx, hipStream_t s) {
     constexpr int T = (1 << (LOGL + LOGC)) / (4 * V);
     ProfScope ps(inverse ? kProfColInv : kProfColFwd, s);
     const dim3 g(1u << (k2 - LOGC), cnt0 + cnt1);
+    if constexpr (V == 4 && LOGL + LOGC == 14 && LOGL >= 9) {
+        const int64_t tiles = (int64_t)g.x * g.y;
+        const bool edges = s0.out_from || s0.out_xor || s0.monic || s0.neg;
+        const bool whole = inverse || (s0.in_len % 4 == 0 && s1.in_len % 4 == 0);
+        if (tiles >= kLoopMin && tiles <= (inverse ? kLoopMax / 2 : kLoopMax) && !edges && whole) {
+            if (inverse)
+                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, true>), dim3(256), dim3(T), 0, s, s0, s1,
+                                   cnt0, (int)tiles, k2, cx);
+            else
+                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, false>), dim3(256), dim3(T), 0, s, s0,
+                                   s1, cnt0, (int)tiles, k2, cx);
+            return hipGetLastError();
+        }
+    }
     if (inverse && (s0.out_from || s0.out_xor || s0.monic || s0.neg))
         hipLaunchKernelGGL((k_col_inv_mx<LOGL, LOGC, V, true>), g, dim3(T), 0, s, s0, k2, cx);
     else if (inverse)

@@ -284,3 +284,27 @@ def test_list_products_in_pieces(cm, orc, p):
         for i in range(n):
             w = want[i % len(items)]
             assert (got[arr[i].h_off:arr[i].h_off + len(w)] == w).all(), (i, shapes[i % len(items)])
+
+
+@pytest.mark.parametrize("p", [P1, P2])
+def test_columns_of_many_tiles(cm, p):
+    """From 512 column tiles on, one workgroup per CU takes several tiles if the
+    operands end on a whole quad of words: the same products as with tiles of
+    half the width, which run one workgroup per tile."""
+    L = cm.lib()
+    rng = np.random.default_rng(p + 5)
+    for e, shapes in ((22, ((0, 0, 0), (4, 4, 0), (-4, 8, 3), (2, 2, 0), (0, 1, 1))),
+                      (23, ((0, 0, 0), (1, 0, 5))), (24, ((0, -8, 0), (0, 0, 1)))):
+        for da, db, cut in shapes:
+            lf, lg = (5 << (e - 3)) - da, (3 << (e - 3)) - db - (da == db == 0)
+            lf, lg = (lf, lg & ~3) if da % 4 == 0 and db % 4 == 0 else (lf, lg)
+            F, G = (rng.integers(0, p, n, dtype=np.int32) for n in (lf, lg))
+            nout = lf + lg - 1 - cut
+            old = L.cumodp_tune_get_col_tile()
+            got = _mul(cm, F, G, p, nout)
+            try:
+                assert L.cumodp_tune_set_col_tile(8192) == 0
+                want = _mul(cm, F, G, p, nout)
+            finally:
+                L.cumodp_tune_set_col_tile(old)
+            assert (got == want).all(), (e, lf, lg, nout)
