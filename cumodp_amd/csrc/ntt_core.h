@@ -12,11 +12,10 @@
 // Forward transforms are decimation in frequency (natural order in,
 // bit-reversed order out); inverse transforms are the exact stage-by-stage
 // inverse (decimation in time, bit-reversed in, natural out) with inverse
-// twiddles.  The multiply path therefore never permutes data: the pointwise
-// product is taken in bit-reversed order.  Stand-alone transforms that must
-// return the natural-order DFT Y_j = sum_i X_i w^(ij) (the output of the
-// reference's Stockham kernels, src/stockham.cu:40-46 and :413-453) read
-// the tile back through a bit reversal.
+// twiddles.  A multiply therefore never permutes data: the pointwise product is
+// taken in bit-reversed order.  The column transforms of the bivariate DFT read
+// the tile back through a bit reversal.  (The framework's other transforms run
+// on the matrix cores, ntt_mx.h.)
 //
 // DIF stage s (0-based) pairs positions q and q + d, d = L >> (s+1), inside
 // blocks of 2d words, and maps (x, y) -> (x + y, (x - y) * w_{2d}^(q mod d)).
@@ -91,9 +90,7 @@ CM_DEV u32 cm_canon(u32 a, MD md) {
 }
 
 // Twiddle w = tab[base + mm + lane] of a level table (base and mm uniform,
-// lane per thread; lane == 0 when the index is uniform).  Plain loads: a raw
-// buffer form (uniform part as the scalar offset) measured slower here,
-// 80 against 75 us on the forward column pass of the 2^24 multiply.
+// lane per thread; lane == 0 when the index is uniform).
 template <bool UNIFORM>
 CM_DEV u32 cm_twiddle(const u32 *tab, int base_mm, int lane) {
     if constexpr (UNIFORM) return tab[base_mm];
@@ -169,14 +166,11 @@ struct Tile {
     // the three bits above each 64-word block into the low six
     // (x ^ 9 ((x >> 6) & 7)): every round's wave access and the linear load
     // and store phases then hit 64 distinct banks (at worst two per bank on a
-    // 32-bank LDS), with no padding; the row pass's bank-conflict cycles drop
-    // eightfold.
+    // 32-bank LDS), with no padding.
     // Column tiles of 4 or more columns pad every 64-word block by K = 8 words
     // (4 for four columns): x + K (x >> 6).  A wave's 64 lanes then hit 64
     // distinct banks in every round (the last round's lanes stride 64 words,
-    // one block apart, and land K banks apart), a four-word group stays
-    // contiguous and 16-byte aligned for the 128-bit load and store phases,
-    // and each thread's elements of a round sit at constant offsets from its
+    // one block apart, and land K banks apart), and each thread's elements of a round sit at constant offsets from its
     // first (the XOR swizzle removes the conflicts too, but its address
     // arithmetic does not fold into LDS instruction offsets and pushes the
     // column kernels past 64 VGPRs).  Other tiles keep one pad word per 16.
@@ -189,9 +183,6 @@ struct Tile {
         else if constexpr (BLKPAD != 0) return x + BLKPAD * (x >> 6);
         else return cm_pad(x);
     }
-    // four consecutive words x .. x+3 (x a multiple of 4) are contiguous and
-    // 16-byte aligned in LDS
-    static constexpr bool QUAD = BLKPAD != 0;
     static constexpr int T = T_;                   // threads per workgroup
     static constexpr int NR = (LOGL_ + 3) / 4;     // rounds
     static constexpr int rsz(int j) { return LOGL_ / NR + (j < LOGL_ % NR ? 1 : 0); }
@@ -209,34 +200,6 @@ struct Tile {
         else { c = g >> (LOGL_ - R); gi = g & ((1 << (LOGL_ - R)) - 1); }
     }
 };
-
-// Words idx .. idx+3 of a tile (idx a multiple of 4): one 128-bit LDS access
-// when the layout keeps them together (the LDS array is 16-byte aligned).
-template <class TL>
-CM_DEV void cm_lds_put4(u32 *lds, int idx, uint4 v) {
-    if constexpr (TL::QUAD) {
-        *(uint4 *)(lds + TL::phys(idx)) = v;
-    } else {
-        lds[TL::phys(idx)] = v.x;
-        lds[TL::phys(idx + 1)] = v.y;
-        lds[TL::phys(idx + 2)] = v.z;
-        lds[TL::phys(idx + 3)] = v.w;
-    }
-}
-
-template <class TL>
-CM_DEV uint4 cm_lds_get4(const u32 *lds, int idx) {
-    if constexpr (TL::QUAD) {
-        return *(const uint4 *)(lds + TL::phys(idx));
-    } else {
-        uint4 v;
-        v.x = lds[TL::phys(idx)];
-        v.y = lds[TL::phys(idx + 1)];
-        v.z = lds[TL::phys(idx + 2)];
-        v.w = lds[TL::phys(idx + 3)];
-        return v;
-    }
-}
 
 // R DIF stages (S0 .. S0+R-1 of an L = 2^LOGL transform) on NV register
 // groups that share their positions (and so their twiddles).  TOPZERO: the
@@ -332,24 +295,15 @@ struct Round {
 #pragma unroll
             for (int m = 0; m < (1 << R); ++m) lds[a][g.a(m)] = v[a][m];
     }
-    // full forward round on NV tiles, LDS -> LDS; TOPZERO (first round
-    // only): the upper half of every vector is zero and is not read
-    template <int NV, bool TOPZERO = false, class MD>
+    // full forward round on NV tiles, LDS -> LDS
+    template <int NV, class MD>
     static CM_DEV void dif(u32 *const (&lds)[NV], const u32 *lv, MD md) {
-        static_assert(!TOPZERO || S0 == 0, "zero upper half only in the first round");
 #pragma unroll
         for (int q = 0; q < GPT; ++q) {
             G g(threadIdx.x + q * TL::T);
             u32 v[NV][1 << R];
-            if (TOPZERO) {
-#pragma unroll
-                for (int a = 0; a < NV; ++a)
-#pragma unroll
-                    for (int m = 0; m < (1 << (R - 1)); ++m) v[a][m] = lds[a][g.a(m)];
-            } else {
-                load<NV>(lds, g, v);
-            }
-            cm_dif_stages<TL::LOGL, R, S0, DLOG, NV, TOPZERO>(v, g.gi_lo, lv, md);
+            load<NV>(lds, g, v);
+            cm_dif_stages<TL::LOGL, R, S0, DLOG, NV>(v, g.gi_lo, lv, md);
             store<NV>(lds, g, v);
         }
     }
@@ -392,12 +346,6 @@ template <class TL, class MD>
 CM_DEV void cm_tile_dif(u32 *lds, const u32 *lv, MD md) {
     u32 *const t[1] = {lds};
     cm_dif_rounds<TL, 0, TL::NR, 1>(t, lv, md);
-}
-
-template <class TL, class MD>
-CM_DEV void cm_tile_dit(u32 *lds, const u32 *lvi, MD md) {
-    u32 *const t[1] = {lds};
-    cm_dit_rounds<TL, TL::NR - 1, 0, 1>(t, lvi, md);
 }
 
 // Multiply of two tiles A (first operand, becomes the product) and B:
