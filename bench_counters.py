@@ -99,8 +99,10 @@ def traffic(args):
            "fetch_scale": fs, "write_scale": ws,
            "copy_calibration": {"bytes": COPY_BYTES, "fetch_kib": fk, "write_kib": wk},
            "commands": args.cmd or [], "kernels": {}}
-    for key in ("k_col_fwd", "k_row_mul", "k_col_inv"):
-        names = [k for k in fetch if k.startswith(key)]
+    # the kernels behind the three timer names, with rows of 2^13 words
+    for key, pre, end in (("k_col_fwd", "k_cols_loop<", "false>"),
+                          ("k_row_mul", "k_row_mx<", ">"), ("k_col_inv", "k_cols_loop<", "true>")):
+        names = [k for k in fetch if k.startswith(pre) and k.endswith(end)]
         if not names:
             continue
         k = names[0]

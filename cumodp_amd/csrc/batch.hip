@@ -166,8 +166,9 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 //     kernel recombines them after the launch;
 //   * plain: 2048 consecutive outputs of one schoolbook product (8 waves of
 //     256 outputs, each wave on its own, the arithmetic of k_plain_mul).
-// Bound by vector issue (59.9 M wave instructions of 6.9 cycles on 1024 SIMDs,
-// most of them 32-bit multiplies).  4096 pairs of degrees 32 .. 16384: 197 us per
+// Bound by issue and the chains inside a wave: 59.9 M vector and 3.8 M matrix
+// instructions take 58% and 15% of the SIMDs' cycles with four waves on each,
+// and the CUs are busy 83% of the time.  4096 pairs of degrees 32 .. 16384: 197 us per
 // call against 226 us with 1024 threads and 16384-word tiles, one workgroup per
 // CU, 2^15 points as two halves; a product of up to 12288 words as 8192 + 4096
 // points takes 5 us of that.  2^24 points in all of 2^13-point products take 96

@@ -38,7 +38,8 @@ int64_t tree_level_offset(int k, int i) {
 // Bound by the chain of LDS loads and multiply-adds of a thread: 256 one after
 // the other if a word has one thread.  The levels above 64 words split each sum
 // over kTreeParts threads; up to 64 words a node stays within a wave, which
-// needs no barrier.
+// needs no barrier.  Whole tree of 2^16 points: 84.6 us with one thread per
+// word, 78.8 us so.
 constexpr int kTreeFuse = 8;
 constexpr int kTreeParts = 4;
 
