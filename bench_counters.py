@@ -53,6 +53,7 @@ def counters(d):
 
 def short(kernel):
     """Kernel name without its argument list (template arguments kept)."""
+    kernel = kernel.replace("(anonymous namespace)::", "")
     depth, end = 0, len(kernel)
     for i, c in enumerate(kernel):
         if c == "<":
