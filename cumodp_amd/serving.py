@@ -10,8 +10,13 @@ result buffer.
 
 Design:
   * Two slots, each with its own HIP stream and device buffers. While one
-    batch computes, the next one uploads and launches on the other slot.
-    Both streams have the default priority.
+    batch computes, the next one uploads and launches on the other slot;
+    a third holds the batch whose products are copied back. All streams have
+    the default priority.
+  * One copy back at a time, queued when the batch ahead has left. Copies
+    that share the link end together, and the slots then stay in step, with
+    the link idle while they compute: 20,000 requests at once took 0.231 s
+    so, 0.180 s with the copies one at a time, 0.154 s with the third slot.
   * FIFO admission. A batch is a contiguous range of request ids, so its
     inputs and outputs are contiguous in the packed pinned host buffers:
     one host-to-device copy in and one device-to-host copy out per batch.
@@ -179,7 +184,8 @@ class ZmulServer:
     seconds of estimated GPU work (max_batch_s None: no time cap)."""
 
     def __init__(self, slots=2, slot_bytes=1 << 30, max_batch_s=None, age_factor=0.0):
-        self.slots = [_Slot() for _ in range(slots)]
+        # one more for the batch whose products are copied back
+        self.slots = [_Slot() for _ in range(slots + 1)]
         self.slot_bytes = int(slot_bytes)
         self.max_batch_s = max_batch_s
         self.age_factor = age_factor
@@ -273,10 +279,16 @@ class ZmulServer:
         _check("cumodp_two_convolution_list_dev", L.cumodp_two_convolution_list_dev(
             items.ctypes.data_as(C.POINTER(ZmulItem)), n, C.c_void_p(slot.din),
             C.c_void_p(slot.din), C.c_void_p(slot.dout), st))
-        _check("cumodp_memcpy_d2h_async", L.cumodp_memcpy_d2h_async(
-            C.c_void_p(Q.OUT.ptr + 8 * out0), C.c_void_p(slot.dout), 8 * (out1 - out0), st))
         slot.range = (i0, i1)
         slot.units = self._batch_units(Q, i0, i1)
+
+    def _collect(self, slot, Q):
+        """Queue the copy of a launched batch's products back to the host."""
+        i0, i1 = slot.range
+        out0, out1 = int(Q.out_off[i0]), int(Q.out_off[i1])
+        _check("cumodp_memcpy_d2h_async", lib().cumodp_memcpy_d2h_async(
+            C.c_void_p(Q.OUT.ptr + 8 * out0), C.c_void_p(slot.dout), 8 * (out1 - out0),
+            C.c_void_p(slot.stream)))
 
     def run(self, Q, arrivals):
         """Serve requests 0..Q.n-1 arriving at `arrivals` (seconds from the
@@ -313,6 +325,8 @@ class ZmulServer:
                 last_done = t
                 s.range = None
                 free.append(s)
+                if inflight:
+                    self._collect(inflight[0], Q)
             arrived = int(np.searchsorted(arrivals, now, side="right"))
             if head < arrived and free:
                 self._age = now - arrivals[head]
@@ -322,6 +336,8 @@ class ZmulServer:
                 self._launch(s, Q, head, j)
                 batches.append(j - head)
                 inflight.append(s)
+                if len(inflight) == 1:
+                    self._collect(s, Q)
                 head = j
                 continue
             if not inflight and head < N and head >= arrived:
