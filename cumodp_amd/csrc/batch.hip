@@ -897,7 +897,9 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     u32 *big_s = nullptr;
     if (nbig > 0 && ntasks < 4 * device_cus() && !stream_capturing(s)) {
         big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig * 4 * kPW), s);
-        if (!big_s) return hipErrorOutOfMemory;
+        if (!big_s) (void)hipGetLastError();   // whole products need no scratch
+    }
+    if (big_s) {
         ntasks -= nbig;
         for (int64_t i = 0; i < count; ++i)
             if (!is_plain(descs[i]) && (descs[i].logn == kPLog + 1 || descs[i].logn == kBigLog))

@@ -412,7 +412,7 @@ hipError_t launch_fast_evaluation(const u32 *F_in, const u32 *pts, int k, u32 p,
                                n >> L0, plain_mod(p), inv_at(L0));
         e = hipGetLastError();
     }
-    if (e == hipSuccess && k - 1 > L0) {
+    if (e == hipSuccess && k - 1 > istart) {
         LevelOffsets lo{};
         for (int l = 0; l <= k && l < 32; ++l) lo.off[l] = tree_level_offset(k, l);
         hipLaunchKernelGGL(k_rev_nodes, dim3(eblocks(n), k - 1 - L0), dim3(256), 0, s, tree, lo,

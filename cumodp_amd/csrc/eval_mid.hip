@@ -257,7 +257,7 @@ __global__ __launch_bounds__(4 << kMidBase) void k_mid_descend(const u32 *__rest
 // The product at the root is on 2^(k+1) points, which the modulus and the
 // largest transform have to allow.  2^9 points: 39.8 us against 81.2 us by the
 // remainder tree, 2^13: 142 against 343 us; at 2^8, one node of k_mid_descend, the
-// remainder tree is a few launches (33.5 us).
+// remainder tree is a few launches (31.1 us).
 bool evaluate_transposed_takes(int k, const Family *fam) {
     return k > kMidBase && k + 1 <= std::min(fam->K, kMaxLog);
 }
