@@ -185,17 +185,25 @@ constexpr int kPW = 1 << kPLog;              // words per product tile
 constexpr int kPlainTaskOut = kPT / 64 * 256;   // outputs of a plain task
 constexpr int kPlainJT = 512;                // B coefficients per pass of a plain task
 
-enum : int32_t { kTaskTile = 0, kTaskBig = 1, kTaskPlain = 2 };
+enum : uint32_t { kTaskTile = 0, kTaskBig = 1, kTaskPlain = 2 };
 
+// Eight bytes, since a call uploads its tasks and descriptors and an upload
+// above 16 KiB takes about 12 us longer: 300 products of 2^13 points take 31.6 us
+// so and 45.4 us with tasks of 16 bytes.
 struct ListTask {
-    int32_t kind;
     int32_t first;   // tile: first descriptor; else the descriptor
-    int32_t count;   // tile: products; big: pieces, kShort, or the product's slot in the
-                     // scratch; plain: first output of the task
-    int32_t logn;    // tile: transform size; big: -1 for all pieces, or which
+    uint32_t what;   // bits 0-1: kind; bits 2-6, sub: tile: transform size; big: kBigAll,
+                     // kBigShort, or which piece goes to the scratch; the rest, count: tile:
+                     // products; big, all: pieces; plain: outputs before the task, in
+                     // kPlainTaskOut
 };
 
-constexpr int32_t kShort = -1;   // ListTask::count of a product of up to 3/2 kPW words
+static ListTask list_task(uint32_t kind, int64_t first, uint32_t sub, int64_t count) {
+    return ListTask{(int32_t)first, kind | sub << 2 | (uint32_t)count << 7};
+}
+
+constexpr uint32_t kBigAll = 4;     // every piece of a product, one after the other
+constexpr uint32_t kBigShort = 5;   // a product of up to 3/2 kPW words
 
 // Pieces modulo x^kPW - omega that a product of `words` words needs.
 static int big_pieces(int words) { return (words + kPW - 1) / kPW; }
@@ -547,7 +555,7 @@ CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDes
 __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_list_persistent(
     const u32 *__restrict__ F, const u32 *__restrict__ G, u32 *__restrict__ H,
     const MulDesc *__restrict__ descs, const ListTask *__restrict__ tasks, int ntasks,
-    int *__restrict__ counter, u32 *__restrict__ big_s, const u32 *__restrict__ lv,
+    int *__restrict__ counter, u32 *__restrict__ big_s, int big0, const u32 *__restrict__ lv,
     const u32 *__restrict__ lvi, MxCtx cx, PlainMod pm) {
     __shared__ __align__(16) u32 lds[2 * mx_lds_words(kPW)];
     __shared__ int s_next;
@@ -557,23 +565,26 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const int ti = __builtin_amdgcn_readfirstlane(s_next);
     if (ti >= ntasks) return;   // one workgroup per task: never taken
     const ListTask t = tasks[ti];
-    if (t.kind == kTaskPlain) {
-        task_plain(lds, F, G, H, descs + t.first, t.count, pm);
-    } else if (t.kind == kTaskBig) {
-        if (t.count == kShort) {
+    const uint32_t kind = t.what & 3, sub = t.what >> 2 & 31;
+    const int count = (int)(t.what >> 7);
+    if (kind == kTaskPlain) {
+        task_plain(lds, F, G, H, descs + t.first, count * kPlainTaskOut, pm);
+    } else if (kind == kTaskBig) {
+        if (sub == kBigShort) {
             task_big_short(lds, F, G, H, descs + t.first, lv, lvi, cx);
             return;
         }
-        const bool all = t.logn < 0;
-        task_big(lds, F, G, H, descs + t.first, all ? 0 : t.logn, all ? t.count : t.logn + 1,
-                 all ? nullptr : big_s + ((int64_t)t.count * 4 + t.logn) * kPW, lv, lvi, cx);
+        const bool all = sub == kBigAll;
+        const int q = (int)sub;
+        task_big(lds, F, G, H, descs + t.first, all ? 0 : q, all ? count : q + 1,
+                 all ? nullptr : big_s + ((int64_t)(t.first - big0) * 4 + q) * kPW, lv, lvi, cx);
     } else {
         const MulDesc *d = descs + t.first;
 #define CM_PMIX(K)                                       \
     case K:                                              \
-        task_tile<K>(lds, F, G, H, d, t.count, cx);      \
+        task_tile<K>(lds, F, G, H, d, count, cx);        \
         break;
-        switch (t.logn) {
+        switch (sub) {
             CM_PMIX(4) CM_PMIX(5) CM_PMIX(6) CM_PMIX(7) CM_PMIX(8) CM_PMIX(9) CM_PMIX(10)
             CM_PMIX(11) CM_PMIX(12) CM_PMIX(13)
         default: break;
@@ -939,14 +950,14 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
                 const int lb = std::min(d.lf, d.lg);
                 for (int c0 = 0; c0 < d.lh; c0 += kPlainTaskOut) {
                     const int outs = std::min(kPlainTaskOut, d.lh - c0);
-                    emit(ListTask{kTaskPlain, (int32_t)i, c0, 0}, (double)outs * lb / 8.0);
+                    emit(list_task(kTaskPlain, i, 0, c0 / kPlainTaskOut), (double)outs * lb / 8.0);
                 }
             }
             for (int e2 = 4; e2 <= kPLog; ++e2) {
                 const int per = kPW >> e2;
                 for (int64_t i = off[e2]; i < off[e2 + 1]; i += per) {
                     const int cnt = (int)std::min<int64_t>(per, off[e2 + 1] - i);
-                    emit(ListTask{kTaskTile, (int32_t)i, cnt, e2},
+                    emit(list_task(kTaskTile, i, (uint32_t)e2, cnt),
                          3.0 * e2 * (double)cnt * (1 << (e2 - 1)));
                 }
             }
@@ -955,11 +966,11 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
                 const double piece = 3.0 * kPLog * (1 << (kPLog - 1));
                 if (!big_s) {
                     const bool sh = sorted[i].lf + sorted[i].lg - 1 <= kPW / 2 * 3;
-                    emit(ListTask{kTaskBig, (int32_t)i, sh ? kShort : np, -1},
+                    emit(list_task(kTaskBig, i, sh ? kBigShort : kBigAll, np),
                          (sh ? 1.5 : np) * piece);
                 }
                 for (int q = 0; big_s && q < np; ++q)
-                    emit(ListTask{kTaskBig, (int32_t)i, (int32_t)(i - off[kPLog + 1]), q}, piece);
+                    emit(list_task(kTaskBig, i, (uint32_t)q, 0), piece);
             }
         };
         int64_t nb[64] = {0};
@@ -981,8 +992,8 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
         ProfScope ps(kProfListPersistent, s);
         const dim3 grid((unsigned)ntasks);
         hipLaunchKernelGGL(k_list_persistent, grid, dim3(kPT), 0, s, F, G, H, d_descs, d_tasks,
-                           (int)ntasks, d_counter, big_s, fam->lv, fam->lvi, mx_ctx(fam),
-                           plain_mod(fam->p));
+                           (int)ntasks, d_counter, big_s, (int)off[kPLog + 1], fam->lv, fam->lvi,
+                           mx_ctx(fam), plain_mod(fam->p));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
