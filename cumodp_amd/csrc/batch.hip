@@ -155,15 +155,18 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 // One launch for every product of a list call up to 2^15 points, schoolbook
 // and NTT alike: one workgroup of 512 threads and 68 KiB of LDS per task, so
 // that two run on a CU and one's loads and stores go on under the other's
-// transforms.  Each workgroup takes its task from a list in descending order of
-// estimated cost through an atomic counter, so the tasks start largest first
-// whatever order the hardware dispatches workgroups in:
-//   * tile: 8192 words of products of one size 2^logn <= 2^13 (8192 >> logn
-//     products), multiplied in LDS;
+// transforms, or of 1024 threads and 136 KiB (list_log).  Each workgroup takes
+// its task from a list in descending order of estimated cost through an atomic
+// counter, so the tasks start largest first whatever order the hardware
+// dispatches workgroups in (figures for 512 threads, W = 8192 words; twice that
+// for 1024):
+//   * tile: W words of products of one size 2^logn <= W (W >> logn products),
+//     multiplied in LDS;
 //   * big: a product of 2^14 or 2^15 points, modulo 2 to 4 factors x^8192 -
 //     omega one after the other (omega = 1, -1, i, -i; 3 reach 24576 words), or
-//     one of them when the list has too few tasks for the chip; then a short
-//     kernel recombines them after the launch;
+//     one of them when whole products would be too long for the chip; then a
+//     short kernel recombines them after the launch.  With 1024 threads: one of
+//     the two halves of a 2^15-point product, modulo x^16384 - 1 and + 1;
 //   * plain: 2048 consecutive outputs of one schoolbook product (8 waves of
 //     256 outputs, each wave on its own, the arithmetic of k_plain_mul).
 // Bound by issue and the chains inside a wave: 59.9 M vector and 3.8 M matrix
@@ -179,10 +182,15 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 // workgroups was measured slower: inlined into the loop, the task bodies'
 // thread-index arithmetic is hoisted out of it and spills, and called out of
 // line they take their uniform pointers in vector registers.)
-constexpr int kPT = 512;                     // threads of the persistent workgroup
-constexpr int kPLog = 13;
-constexpr int kPW = 1 << kPLog;              // words per product tile
-constexpr int kPlainTaskOut = kPT / 64 * 256;   // outputs of a plain task
+// All of this on W = 2^LOG words, LOG = 13 or 14 (list_log chooses).
+template <int LOG>
+struct ListGeo {
+    static constexpr int W = 1 << LOG;               // words per product tile
+    static constexpr int T = W / 16;                 // threads
+    static constexpr int PlainOut = T / 64 * 256;    // outputs of a plain task
+    static constexpr int Pieces = LOG == 13 ? 4 : 2; // of the largest product
+};
+constexpr int kBigLog = 15;                  // largest product of the launch
 constexpr int kPlainJT = 512;                // B coefficients per pass of a plain task
 
 enum : uint32_t { kTaskTile = 0, kTaskBig = 1, kTaskPlain = 2 };
@@ -195,7 +203,7 @@ struct ListTask {
     uint32_t what;   // bits 0-1: kind; bits 2-6, sub: tile: transform size; big: kBigAll,
                      // kBigShort, or which piece goes to the scratch; the rest, count: tile:
                      // products; big, all: pieces; plain: outputs before the task, in
-                     // kPlainTaskOut
+                     // PlainOut
 };
 
 static ListTask list_task(uint32_t kind, int64_t first, uint32_t sub, int64_t count) {
@@ -203,20 +211,22 @@ static ListTask list_task(uint32_t kind, int64_t first, uint32_t sub, int64_t co
 }
 
 constexpr uint32_t kBigAll = 4;     // every piece of a product, one after the other
-constexpr uint32_t kBigShort = 5;   // a product of up to 3/2 kPW words
+constexpr uint32_t kBigShort = 5;   // a product of up to 3/2 W words
 
-// Pieces modulo x^kPW - omega that a product of `words` words needs.
-static int big_pieces(int words) { return (words + kPW - 1) / kPW; }
+// Pieces modulo x^W - omega that a product of `words` words needs.
+template <int LOG>
+CM_HD int big_pieces(int words) { return (words + ListGeo<LOG>::W - 1) >> LOG; }
 
-// x[0] <- (canonical, natural order) the product d modulo x^kPW - omega, omega =
-// 1, -1, i, -i for q = 0 .. 3 (i = w_4): the operands' chunks of kPW words are
-// folded by powers of omega, twisted by psi^j (psi^kPW = omega: w_2M, w_4M or
-// its inverse, M = kPW; entries of the level tables) and untwisted after the
+// x[0] <- (canonical, natural order) the product d modulo x^W - omega, omega =
+// 1, -1, i, -i for q = 0 .. 3 (i = w_4): the operands' chunks of W words are
+// folded by powers of omega, twisted by psi^j (psi^W = omega: w_2M, w_4M or
+// its inverse, M = W; entries of the level tables) and untwisted after the
 // cyclic product.
+template <int LOG>
 CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u32 *G,
                       const MulDesc &d, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
-    constexpr int V = 4, M = kPW;
-    using Map = MxMap<kPLog - 4, V>;
+    constexpr int V = 4, M = ListGeo<LOG>::W;
+    using Map = MxMap<LOG - 4, V>;
     const int i0 = Map::base();
     const u32 p = cx.p;
     const int lev = q == 1 ? M - 1 : 2 * M - 1;
@@ -237,7 +247,7 @@ CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u3
                 return v;
             };
             MxQuad a = chunk(0), b = chunk(1);
-            if (len > 2 * M) {
+            if (ListGeo<LOG>::Pieces > 2 && len > 2 * M) {
                 const MxQuad c = chunk(2), e = chunk(3);
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
@@ -245,7 +255,7 @@ CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u3
                     b.v[s] = cm_add(b.v[s], q < 2 ? e.v[s] : cm_sub(0u, e.v[s], p), p);
                 }
             }
-            if (q < 2) {
+            if (ListGeo<LOG>::Pieces == 2 || q < 2) {
 #pragma unroll
                 for (int s = 0; s < 4; ++s) y[s][r] = a.v[s] + (q ? p - b.v[s] : b.v[s]);
             } else {   // omega psi^j = psi^(j + M)
@@ -270,8 +280,8 @@ CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u3
     operand(x[1], G + d.g, d.lg);
     MxMat m;
     u32 tw[V][4];
-    mx_forward_begin<kPLog, 0, V>(m, tw, cx);
-    mx_tile_multiply<kPLog, V>(x, lds, lds + mx_lds_words(kPW), cx, m, tw);
+    mx_forward_begin<LOG, 0, V>(m, tw, cx);
+    mx_tile_multiply<LOG, V>(x, lds, lds + mx_lds_words(M), cx, m, tw);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if (q == 0) {
@@ -285,8 +295,8 @@ CM_DEV void big_piece(int q, u32 (&x)[2][4][4], u32 *lds, const u32 *F, const u3
     }
 }
 
-// The chunks h[c] (h = sum_c h[c] x^(c kPW)) from its residues a[q] modulo
-// x^kPW - omega_q, np = 2, 3 or 4 of them (h[3] = 0 for 3).
+// The chunks h[c] (h = sum_c h[c] x^(c W)) from its residues a[q] modulo
+// x^W - omega_q, np = 2, 3 or 4 of them (h[3] = 0 for 3).
 CM_DEV void big_recombine(u32 (&a)[4], int np, u32 w4, u32 w4i, const MxCtx &cx) {
     const u32 p = cx.p;
     auto half = [&](u32 v) { return (v + (v & 1 ? p : 0u)) >> 1; };
@@ -311,19 +321,20 @@ CM_DEV void big_recombine(u32 (&a)[4], int np, u32 w4, u32 w4i, const MxCtx &cx)
 }
 
 // Pieces q0 .. q1 - 1 of one product.  With S, a piece goes there; else all but
-// the last wait in the output (which has more than (q1 - 1) kPW words), each
+// the last wait in the output (which has more than (q1 - 1) W words), each
 // word where this lane put it, and the last recombines them.
 CM_DEV void task_big(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp, int q0,
                      int q1, u32 *S, const u32 *lv, const u32 *lvi, const MxCtx &cx) {
-    using Map = MxMap<kPLog - 4, 4>;
+    constexpr int LOG = 13, W = 1 << LOG;
+    using Map = MxMap<LOG - 4, 4>;
     const MulDesc d = *dp;
     u32 x[2][4][4];
     u32 *h = H + d.h;
     const int i0 = Map::base();
     for (int q = q0;; ++q) {
-        big_piece(q, x, lds, F, G, d, lv, lvi, cx);
+        big_piece<LOG>(q, x, lds, F, G, d, lv, lvi, cx);
         if (q == q1 - 1 && !S) break;
-        u32 *out = S ? S : h + q * kPW;
+        u32 *out = S ? S : h + q * W;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             *(MxQuad *)(out + i0 + Map::off(0, r)) =
@@ -338,7 +349,7 @@ CM_DEV void task_big(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc
         MxQuad c[3] = {};
 #pragma unroll
         for (int q = 0; q < 3; ++q)
-            if (q < q1 - 1) c[q] = *(const MxQuad *)(h + q * kPW + i);
+            if (q < q1 - 1) c[q] = *(const MxQuad *)(h + q * W + i);
         MxQuad o[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -351,7 +362,7 @@ CM_DEV void task_big(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if (q >= q1) break;
-            const int k = q * kPW + i;
+            const int k = q * W + i;
             if (k + 4 <= d.lh) {
                 *(MxQuad *)(h + k) = o[q];
             } else {
@@ -363,20 +374,33 @@ CM_DEV void task_big(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc
     }
 }
 
-// A product of kPW < words <= 3/2 kPW, with M = kPW / 2: A = H mod x^(2M) - 1 = (H0
+// Half Q of a 2^15-point product, modulo x^W - 1 or x^W + 1 (W = 2^14), to S.
+template <int Q>
+CM_DEV void task_half(u32 *lds, const u32 *F, const u32 *G, const MulDesc *dp, u32 *S,
+                      const u32 *lv, const u32 *lvi, const MxCtx &cx) {
+    using Map = MxMap<14 - 4, 4>;
+    u32 x[2][4][4];
+    big_piece<14>(Q, x, lds, F, G, *dp, lv, lvi, cx);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        *(MxQuad *)(S + Map::base() + Map::off(0, r)) =
+            MxQuad{{x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]}};
+}
+
+// A product of W < words <= 3/2 W (W = 2^13), with M = W / 2: A = H mod x^(2M) - 1 = (H0
 // + H2) + H1 x^M, then B = H mod x^M - i = H0 + i H1 - H2 on M points, which
 // leaves H2 = (A_lo + i A_hi - B) / 2.  A waits in the output.
 CM_DEV void task_big_short(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *dp,
                            const u32 *lv, const u32 *lvi, const MxCtx &cx) {
-    constexpr int V = 2, L = kPLog - 1, M = 1 << L;
+    constexpr int LOG = 13, V = 2, L = LOG - 1, M = 1 << L;
     using Map = MxMap<L - 4, V>;
     const MulDesc d = *dp;
     const u32 p = cx.p;
     u32 *h = H + d.h;
     {
-        using Map4 = MxMap<kPLog - 4, 4>;
+        using Map4 = MxMap<LOG - 4, 4>;
         u32 x[2][4][4];
-        big_piece(0, x, lds, F, G, d, lv, lvi, cx);
+        big_piece<LOG>(0, x, lds, F, G, d, lv, lvi, cx);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             *(MxQuad *)(h + Map4::base() + Map4::off(0, r)) =
@@ -386,7 +410,7 @@ CM_DEV void task_big_short(u32 *lds, const u32 *F, const u32 *G, u32 *H, const M
     u32 x[2][V][4], tw[V][4];
     MxMat m;
     const int i0 = Map::base();
-    const u32 *const wf = lv + kPW - 1, *const wi = lvi + kPW - 1;   // psi^j, psi = w_4M
+    const u32 *const wf = lv + 2 * M - 1, *const wi = lvi + 2 * M - 1;   // psi^j, psi = w_4M
     auto operand = [&](u32 (&y)[V][4], const u32 *q, int len) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -417,27 +441,29 @@ CM_DEV void task_big_short(u32 *lds, const u32 *F, const u32 *G, u32 *H, const M
         }
 }
 
-// The pieces of the products descs[0 .. count) (slot j at S + 4 j kPW) put
+// The pieces of the products descs[0 .. count) (slot j at S + j Pieces W) put
 // together.
+template <int LOG>
 __global__ void k_big_combine(u32 *__restrict__ H, const MulDesc *__restrict__ descs,
                               const u32 *__restrict__ S, const u32 *__restrict__ lv,
                               const u32 *__restrict__ lvi, MxCtx cx) {
     const MulDesc d = descs[blockIdx.y];
-    const u32 *Sp = S + (int64_t)blockIdx.y * (4 * kPW);
-    const int np = (d.lf + d.lg - 1 + kPW - 1) / kPW;
+    constexpr int W = ListGeo<LOG>::W, NP = ListGeo<LOG>::Pieces;
+    const u32 *Sp = S + (int64_t)blockIdx.y * (NP * W);
+    const int np = big_pieces<LOG>(d.lf + d.lg - 1);
     const u32 w4 = lv[2], w4i = lvi[2];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kPW; i += gridDim.x * blockDim.x) {
-        u32 a[4];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < W; i += gridDim.x * blockDim.x) {
+        u32 a[4] = {};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a[q] = q < np ? Sp[q * kPW + i] : 0u;
-        big_recombine(a, np, w4, w4i, cx);
+        for (int q = 0; q < NP; ++q) a[q] = q < np ? Sp[q * W + i] : 0u;
+        big_recombine(a, NP == 2 ? 2 : np, w4, w4i, cx);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (q < np && q * kPW + i < d.lh) H[d.h + q * kPW + i] = a[q];
+        for (int q = 0; q < NP; ++q)
+            if (q < np && q * W + i < d.lh) H[d.h + q * W + i] = a[q];
     }
 }
 
-// Outputs c0 .. c0 + kPlainTaskOut - 1 of the schoolbook product d: wave w computes the
+// Outputs c0 .. c0 + PlainOut - 1 of the schoolbook product d: wave w computes the
 // 256 outputs from c0 + 256 w on its own (its own LDS region, no workgroup
 // barrier; a wave past the end of the product leaves at once), lane t four of
 // them, with the arithmetic of k_plain_mul.  LDS operations of one wavefront
@@ -517,8 +543,8 @@ CM_DEV void task_plain(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDe
     }
 }
 
-// One tile of products of 2^K points (kPW >> K of them).
-template <int K>
+// One tile of products of 2^K points (W >> K of them).
+template <int K, int LOG>
 CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDesc *d, int cnt,
                       const MxCtx &cx) {
     constexpr int V = 4;
@@ -541,7 +567,7 @@ CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDes
         q = G + e.g;
         len = e.lg;
     });
-    mx_tile_multiply<K, V>(x, lds, lds + mx_lds_words(kPW), cx, m, tw);
+    mx_tile_multiply<K, V>(x, lds, lds + mx_lds_words(ListGeo<LOG>::W), cx, m, tw);
     mx_store_rows<K, V>(
         x[0],
         [&](int s, u32 *&q, int &len) {
@@ -552,13 +578,17 @@ CM_DEV void task_tile(u32 *lds, const u32 *F, const u32 *G, u32 *H, const MulDes
         cx);
 }
 
-__global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_list_persistent(
+template <int LOG>
+__global__ __launch_bounds__(ListGeo<LOG>::T)
+__attribute__((amdgpu_waves_per_eu(4, 8))) void k_list_persistent(
     const u32 *__restrict__ F, const u32 *__restrict__ G, u32 *__restrict__ H,
     const MulDesc *__restrict__ descs, const ListTask *__restrict__ tasks, int ntasks,
     int *__restrict__ counter, u32 *__restrict__ big_s, int big0, const u32 *__restrict__ lv,
     const u32 *__restrict__ lvi, MxCtx cx, PlainMod pm) {
-    __shared__ __align__(16) u32 lds[2 * mx_lds_words(kPW)];
+    using Geo = ListGeo<LOG>;
+    __shared__ __align__(16) u32 lds[2 * mx_lds_words(Geo::W)];
     __shared__ int s_next;
+    static_assert(sizeof(lds) / 4 >= Geo::T / 64 * kPlainWaveWords, "schoolbook tasks");
     if (threadIdx.x == 0) s_next = atomicAdd(counter, 1);
     __syncthreads();
     // uniform: the task and its descriptor load through the scalar unit
@@ -568,25 +598,32 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     const uint32_t kind = t.what & 3, sub = t.what >> 2 & 31;
     const int count = (int)(t.what >> 7);
     if (kind == kTaskPlain) {
-        task_plain(lds, F, G, H, descs + t.first, count * kPlainTaskOut, pm);
+        task_plain(lds, F, G, H, descs + t.first, count * Geo::PlainOut, pm);
     } else if (kind == kTaskBig) {
-        if (sub == kBigShort) {
-            task_big_short(lds, F, G, H, descs + t.first, lv, lvi, cx);
-            return;
+        const MulDesc *d = descs + t.first;
+        u32 *S = big_s + ((int64_t)(t.first - big0) * Geo::Pieces + sub) * Geo::W;
+        if constexpr (LOG == 14) {
+            // the omega as a constant: as a variable it spills 47 registers
+            if (sub == 0) task_half<0>(lds, F, G, d, S, lv, lvi, cx);
+            else task_half<1>(lds, F, G, d, S, lv, lvi, cx);
+        } else if (sub == kBigShort) {
+            task_big_short(lds, F, G, H, d, lv, lvi, cx);
+        } else {
+            const bool all = sub == kBigAll;
+            const int q = (int)sub;
+            task_big(lds, F, G, H, d, all ? 0 : q, all ? count : q + 1, all ? nullptr : S, lv, lvi,
+                     cx);
         }
-        const bool all = sub == kBigAll;
-        const int q = (int)sub;
-        task_big(lds, F, G, H, descs + t.first, all ? 0 : q, all ? count : q + 1,
-                 all ? nullptr : big_s + ((int64_t)(t.first - big0) * 4 + q) * kPW, lv, lvi, cx);
     } else {
         const MulDesc *d = descs + t.first;
 #define CM_PMIX(K)                                       \
     case K:                                              \
-        task_tile<K>(lds, F, G, H, d, count, cx);        \
+        if constexpr (K <= LOG)                          \
+            task_tile<K, LOG>(lds, F, G, H, d, count, cx); \
         break;
         switch (sub) {
             CM_PMIX(4) CM_PMIX(5) CM_PMIX(6) CM_PMIX(7) CM_PMIX(8) CM_PMIX(9) CM_PMIX(10)
-            CM_PMIX(11) CM_PMIX(12) CM_PMIX(13)
+            CM_PMIX(11) CM_PMIX(12) CM_PMIX(13) CM_PMIX(14)
         default: break;
         }
 #undef CM_PMIX
@@ -848,8 +885,7 @@ static hipError_t run_four_step_classes(const MulDesc *sorted, int64_t count,
     return hipSuccess;
 }
 
-// CUs of the current device: the persistent grid holds one workgroup per CU
-// (its LDS allows no more).
+// CUs of the current device.
 static int device_cus() {
     static int cached[64];
     int dev = 0;
@@ -874,47 +910,74 @@ static int cost_bucket(double x) {
     return b > 63 ? 63 : b;
 }
 
-static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, const u32 *F,
-                                         const u32 *G, u32 *H, const Family *fam, hipStream_t s) {
-    if (count > INT32_MAX / 4) return hipErrorInvalidValue;
-    constexpr int kBigLog = 15;
-    const int cut = g_plain_cutoff;
-    auto is_plain = [&](const MulDesc &d) { return cut > 0 && std::min(d.lf, d.lg) <= cut; };
-    // descriptor order: the schoolbook products, then the transform sizes
-    // ascending (class 0: schoolbook, class e: 2^e points)
-    int64_t ncls[33] = {0};
-    int64_t nplain_tasks = 0;
-    for (int64_t i = 0; i < count; ++i) {
-        const MulDesc &d = descs[i];
-        if (is_plain(d)) {
-            ++ncls[0];
-            nplain_tasks += (d.lh + kPlainTaskOut - 1) / kPlainTaskOut;
-        } else {
-            ++ncls[d.logn];
-        }
-    }
+static bool is_plain(const MulDesc &d) {
+    return g_plain_cutoff > 0 && std::min(d.lf, d.lg) <= g_plain_cutoff;
+}
+
+// tiles of 2^log words that the classes 2^4 .. 2^log fill
+static int64_t list_tiles(const int64_t (&ncls)[33], int log) {
+    int64_t n = 0;
+    for (int e = 4; e <= log; ++e) n += (ncls[e] + (1 << (log - e)) - 1) >> (log - e);
+    return n;
+}
+
+// Tasks of 2^13 words with 512 threads, two to a CU, or of 2^14 words with 1024,
+// one to a CU.  A 2^14-point product is two pieces of the small tasks (each reads
+// the operands, and a pass recombines them) and one large task, so the large
+// ones win where they fill the chip once and the small ones would fill it
+// more than half (150 products of 2^14 points: 32 us as large tasks, 44 as
+// small ones, 35 as radix-2 butterflies of 1024 threads), and where 2^14-point
+// products hold half the words and the small tasks either run in pieces or
+// have whole products of 2^15 points, four pieces long, at the end (400
+// products of 2^14 points: 71 us and 84; 700 with 116 of 2^15 and as many words
+// of 2^13 and 2^11: 174 and 196).  The other lists take small tasks (4096 pairs
+// of degrees 32 .. 16384: 187 us).  Measured over 220 mixes of sizes.  pieces:
+// small tasks of the 2^15-point products.
+static int list_log(const int64_t (&ncls)[33], int64_t pieces) {
+    const int64_t tiles = list_tiles(ncls, 13), n14 = ncls[14], n15 = ncls[15];
+    const int64_t large = list_tiles(ncls, 14) + 2 * n15, cus = device_cus();
+    if (large <= cus) return tiles + 2 * n14 + pieces > cus ? 14 : 13;
+    const bool half = 2 * n14 >= tiles + 4 * n15;
+    return half && large <= 8 * cus && (tiles + n14 + n15 < 4 * cus || n15 > 0) ? 14 : 13;
+}
+
+template <int LOG>
+static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const int64_t (&ncls)[33],
+                                    int64_t pieces, const u32 *F, const u32 *G, u32 *H,
+                                    const Family *fam, hipStream_t s) {
+    using Geo = ListGeo<LOG>;
     int64_t off[34];
     off[0] = 0;
     for (int c = 0; c < 33; ++c) off[c + 1] = off[c] + ncls[c];
-    int64_t ntile = 0;
-    for (int e = 4; e <= kPLog; ++e) ntile += (ncls[e] + (kPW >> e) - 1) / (kPW >> e);
-    const int64_t nbig = ncls[kPLog + 1] + ncls[kBigLog];
-    int64_t ntasks = nplain_tasks + ntile + nbig;
-    // Below four tasks per CU (two rounds of workgroups) a long task leaves the
+    int64_t nbig = 0, ntasks = list_tiles(ncls, LOG);
+    for (int e = LOG + 1; e <= kBigLog; ++e) nbig += ncls[e];
+    ntasks += nbig;
+    for (int64_t i = 0; ncls[0] && i < count; ++i)
+        if (is_plain(descs[i])) ntasks += (descs[i].lh + Geo::PlainOut - 1) / Geo::PlainOut;
+    // Small tasks: below four per CU (two rounds of workgroups), or with products of
+    // 2^15 points below 3 1/2 rounds of pieces, a whole product would leave the
     // chip waiting at the end, so every piece is a task, at the price of a
     // recombining pass over scratch (whose allocation a capture does without).
-    // 40 pairs of degrees 32 .. 16384: 26.5 us against 35.3 as 2^14-word
-    // workgroups, 1000 pairs: 82 us so and 105 with whole products.
+    // 40 pairs of degrees 32 .. 16384: 26 us, 56 with whole products; 42 products
+    // of 2^15 points, 256 of 2^14 and as many words of sizes below: 107 us and 135.
+    // Large tasks always take a 2^15-point product as two.
+    const int64_t cus = device_cus();
+    const bool split = LOG == 14 ||
+                       (!stream_capturing(s) &&
+                        (ntasks < 4 * cus ||
+                         (pieces > 0 && list_tiles(ncls, 13) + 2 * ncls[14] + pieces < 7 * cus)));
     u32 *big_s = nullptr;
-    if (nbig > 0 && ntasks < 4 * device_cus() && !stream_capturing(s)) {
-        big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig * 4 * kPW), s);
+    if (nbig > 0 && split) {
+        big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig * Geo::Pieces * Geo::W), s);
         if (!big_s) (void)hipGetLastError();   // whole products need no scratch
     }
+    if (LOG == 14 && nbig > 0 && !big_s)
+        return list_persistent_t<13>(descs, count, ncls, pieces, F, G, H, fam, s);
     if (big_s) {
         ntasks -= nbig;
         for (int64_t i = 0; i < count; ++i)
-            if (!is_plain(descs[i]) && (descs[i].logn == kPLog + 1 || descs[i].logn == kBigLog))
-                ntasks += big_pieces(descs[i].lf + descs[i].lg - 1);
+            if (!is_plain(descs[i]) && descs[i].logn > LOG && descs[i].logn <= kBigLog)
+                ntasks += big_pieces<LOG>(descs[i].lf + descs[i].lg - 1);
     }
     if (ntasks > INT32_MAX) return hipErrorInvalidValue;
 
@@ -948,24 +1011,24 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
             for (int64_t i = off[0]; i < off[1]; ++i) {
                 const MulDesc &d = sorted[i];
                 const int lb = std::min(d.lf, d.lg);
-                for (int c0 = 0; c0 < d.lh; c0 += kPlainTaskOut) {
-                    const int outs = std::min(kPlainTaskOut, d.lh - c0);
-                    emit(list_task(kTaskPlain, i, 0, c0 / kPlainTaskOut), (double)outs * lb / 8.0);
+                for (int c0 = 0; c0 < d.lh; c0 += Geo::PlainOut) {
+                    const int outs = std::min(Geo::PlainOut, d.lh - c0);
+                    emit(list_task(kTaskPlain, i, 0, c0 / Geo::PlainOut), (double)outs * lb / 8.0);
                 }
             }
-            for (int e2 = 4; e2 <= kPLog; ++e2) {
-                const int per = kPW >> e2;
+            for (int e2 = 4; e2 <= LOG; ++e2) {
+                const int per = Geo::W >> e2;
                 for (int64_t i = off[e2]; i < off[e2 + 1]; i += per) {
                     const int cnt = (int)std::min<int64_t>(per, off[e2 + 1] - i);
                     emit(list_task(kTaskTile, i, (uint32_t)e2, cnt),
                          3.0 * e2 * (double)cnt * (1 << (e2 - 1)));
                 }
             }
-            for (int64_t i = off[kPLog + 1]; i < off[kBigLog + 1]; ++i) {
-                const int np = big_pieces(sorted[i].lf + sorted[i].lg - 1);
-                const double piece = 3.0 * kPLog * (1 << (kPLog - 1));
+            for (int64_t i = off[LOG + 1]; i < off[kBigLog + 1]; ++i) {
+                const int np = big_pieces<LOG>(sorted[i].lf + sorted[i].lg - 1);
+                const double piece = 3.0 * LOG * (1 << (LOG - 1));
                 if (!big_s) {
-                    const bool sh = sorted[i].lf + sorted[i].lg - 1 <= kPW / 2 * 3;
+                    const bool sh = sorted[i].lf + sorted[i].lg - 1 <= Geo::W / 2 * 3;
                     emit(list_task(kTaskBig, i, sh ? kBigShort : kBigAll, np),
                          (sh ? 1.5 : np) * piece);
                 }
@@ -991,22 +1054,38 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
     if (ntasks > 0) {
         ProfScope ps(kProfListPersistent, s);
         const dim3 grid((unsigned)ntasks);
-        hipLaunchKernelGGL(k_list_persistent, grid, dim3(kPT), 0, s, F, G, H, d_descs, d_tasks,
-                           (int)ntasks, d_counter, big_s, (int)off[kPLog + 1], fam->lv, fam->lvi,
-                           mx_ctx(fam), plain_mod(fam->p));
+        hipLaunchKernelGGL(k_list_persistent<LOG>, grid, dim3(Geo::T), 0, s, F, G, H, d_descs,
+                           d_tasks, (int)ntasks, d_counter, big_s, (int)off[LOG + 1], fam->lv,
+                           fam->lvi, mx_ctx(fam), plain_mod(fam->p));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (big_s) {
         ProfScope ps(kProfListPersistent, s);
-        hipLaunchKernelGGL(k_big_combine, dim3(kPW / 1024, (unsigned)nbig), dim3(1024), 0, s, H,
-                           d_descs + off[kPLog + 1], big_s, fam->lv, fam->lvi, mx_ctx(fam));
+        hipLaunchKernelGGL(k_big_combine<LOG>, dim3(Geo::W / 1024, (unsigned)nbig), dim3(1024), 0, s,
+                           H, d_descs + off[LOG + 1], big_s, fam->lv, fam->lvi, mx_ctx(fam));
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     // 2^16 points and more: batched four-step multiplies
     return run_four_step_classes(tail.data(), (int64_t)tail.size(), d_descs + off[kBigLog + 1], F,
                                  G, H, fam, s);
+}
+
+static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, const u32 *F,
+                                         const u32 *G, u32 *H, const Family *fam, hipStream_t s) {
+    if (count > INT32_MAX / 4) return hipErrorInvalidValue;
+    // descriptor order: the schoolbook products, then the transform sizes
+    // ascending (class 0: schoolbook, class e: 2^e points)
+    int64_t ncls[33] = {0}, pieces = 0;
+    for (int64_t i = 0; i < count; ++i) {
+        const MulDesc &d = descs[i];
+        const int c = is_plain(d) ? 0 : d.logn;
+        ++ncls[c];
+        if (c == kBigLog) pieces += big_pieces<13>(d.lf + d.lg - 1);
+    }
+    const auto run = list_log(ncls, pieces) == 14 ? list_persistent_t<14> : list_persistent_t<13>;
+    return run(descs, count, ncls, pieces, F, G, H, fam, s);
 }
 
 }  // namespace cm
