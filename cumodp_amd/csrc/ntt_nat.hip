@@ -79,6 +79,13 @@ CM_DEV int nat_index(int u, int e16) {
 }
 
 // Rows of 2^LOGL words, 2^(LOGW-LOGL) per workgroup, in place.
+//
+// Many rows are bound by memory.  A lane's words lie 2^(LOGL-4) words apart, and
+// so do its outputs: pieces of 4 to 16 bytes for rows up to 2^7 words (STAGE),
+// whose tile, one wave's 256 V words, therefore goes through LDS in both
+// directions and through memory in quads of consecutive lanes.  2^25 words as
+// rows of 2^4, 2^5, 2^6 and 2^7: 44.5, 47.6, 47.7 and 47.6 us; straight from and to the
+// registers 92, 127, 101 and 100 us.
 template <int LOGL, int LOGW, int V>
 __global__ __launch_bounds__((1 << LOGW) / (4 * V))
 __attribute__((amdgpu_waves_per_eu(4, 8))) void k_ntt_mx(u32 *__restrict__ X, int64_t m, MxCtx cx) {
@@ -91,12 +98,56 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_ntt_mx(u32 *__restrict__ X, in
     const int row0 = Map::base() >> LOGL;
     MxMat mat = mx_load_mat(cx, kMxFwd + (P::NF == 0 ? P::T : 0));
     u32 x[V][4];
-    mx_load_rows<LOGL, V>(x, [&](int s, const u32 *&q, int &len) {
-        const int64_t row = r0 + row0 + (Map::off(s, 0) >> LOGL);
-        q = X + (row << LOGL);
-        len = row < m ? 1 << LOGL : 0;
-    });
-    if constexpr (P::NR == 1) {
+    constexpr bool STAGE = LOGL <= 7 && V == 4;
+    using Flat = MxMap<0, V>;       // quads in the order of the lanes
+    if constexpr (STAGE) {
+        static_assert((1 << LOGW) == 256 * V, "a tile is one wave's words");
+#pragma unroll
+        for (int s = 0; s < V; ++s) {
+            const int i = Flat::base() + Flat::off(s, 0);
+            MxQuad v{};
+            if (r0 + (i >> LOGL) < m) v = *(const MxQuad *)(X + (r0 << LOGL) + i);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[s][r] = v.v[r];
+        }
+        if constexpr (P::NR > 1) {
+            Flat::store(lds, x);
+            mx_sync<0, V>();
+            Map::load(lds, x);
+        }
+    } else {
+        mx_load_rows<LOGL, V>(x, [&](int s, const u32 *&q, int &len) {
+            const int64_t row = r0 + row0 + (Map::off(s, 0) >> LOGL);
+            q = X + (row << LOGL);
+            len = row < m ? 1 << LOGL : 0;
+        });
+    }
+    if constexpr (STAGE) {
+        if constexpr (P::NR > 1) nat_rounds<LOGL, LOGW, V, false, 0>(x, lds, cx, mat);
+        mx_dft<V>(x, mat, cx);
+        if constexpr (P::NR > 1) {
+            const int n = threadIdx.x & 15, g = (threadIdx.x >> 4) & 3;
+            mx_sync<0, V>();
+#pragma unroll
+            for (int s = 0; s < V; ++s)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int id = V * n + s;
+                    lds[mx_phys_d(((id >> LU) << LOGL) +
+                                  nat_index<LOGL>(id & ((1 << LU) - 1), 4 * g + r))] = x[s][r];
+                }
+            mx_sync<0, V>();
+            Flat::load(lds, x);
+        }
+#pragma unroll
+        for (int s = 0; s < V; ++s) {
+            const int i = Flat::base() + Flat::off(s, 0);
+            if (r0 + (i >> LOGL) < m)
+                *(MxQuad *)(X + (r0 << LOGL) + i) =
+                    MxQuad{{mx_canon(x[s][0], cx), mx_canon(x[s][1], cx), mx_canon(x[s][2], cx),
+                            mx_canon(x[s][3], cx)}};
+        }
+    } else if constexpr (P::NR == 1) {
         mx_dft<V>(x, mat, cx);
         mx_store_rows<LOGL, V>(
             x,
