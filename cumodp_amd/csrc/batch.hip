@@ -931,11 +931,15 @@ static int64_t list_tiles(const int64_t (&ncls)[33], int log) {
 // have whole products of 2^15 points, four pieces long, at the end (400
 // products of 2^14 points: 71 us and 84; 700 with 116 of 2^15 and as many words
 // of 2^13 and 2^11: 174 and 196).  The other lists take small tasks (4096 pairs
-// of degrees 32 .. 16384: 187 us).  Measured over 220 mixes of sizes.  pieces:
-// small tasks of the 2^15-point products.
+// of degrees 32 .. 16384: 187 us).  Measured over 220 mixes of sizes.  Schoolbook
+// products alone take large tasks, of which there are half as many (16 products
+// of 20 by 50000 coefficients: 13.0 us, 15.0 as small ones).  pieces: small tasks
+// of the 2^15-point products.
 static int list_log(const int64_t (&ncls)[33], int64_t pieces) {
     const int64_t tiles = list_tiles(ncls, 13), n14 = ncls[14], n15 = ncls[15];
-    const int64_t large = list_tiles(ncls, 14) + 2 * n15, cus = device_cus();
+    const int64_t large = list_tiles(ncls, 14) + 2 * n15;
+    if (large == 0) return 14;
+    const int64_t cus = device_cus();
     if (large <= cus) return tiles + 2 * n14 + pieces > cus ? 14 : 13;
     const bool half = 2 * n14 >= tiles + 4 * n15;
     return half && large <= 8 * cus && (tiles + n14 + n15 < 4 * cus || n15 > 0) ? 14 : 13;
@@ -961,13 +965,14 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const i
     // 40 pairs of degrees 32 .. 16384: 26 us, 56 with whole products; 42 products
     // of 2^15 points, 256 of 2^14 and as many words of sizes below: 107 us and 135.
     // Large tasks always take a 2^15-point product as two.
-    const int64_t cus = device_cus();
-    const bool split = LOG == 14 ||
-                       (!stream_capturing(s) &&
-                        (ntasks < 4 * cus ||
-                         (pieces > 0 && list_tiles(ncls, 13) + 2 * ncls[14] + pieces < 7 * cus)));
+    auto split = [&] {
+        if (LOG == 14 || stream_capturing(s)) return LOG == 14;
+        const int64_t cus = device_cus();
+        return ntasks < 4 * cus ||
+               (pieces > 0 && list_tiles(ncls, 13) + 2 * ncls[14] + pieces < 7 * cus);
+    };
     u32 *big_s = nullptr;
-    if (nbig > 0 && split) {
+    if (nbig > 0 && split()) {
         big_s = (u32 *)workspace(20, sizeof(u32) * (size_t)(nbig * Geo::Pieces * Geo::W), s);
         if (!big_s) (void)hipGetLastError();   // whole products need no scratch
     }
