@@ -3,8 +3,8 @@
 There are four tunables:
 
   * The four-step split of a 2^k-point transform (k > 13): rows of 2^k2
-    words, with k2 in {12, 13, 14}, and columns of 2^(k-k2) words.
-    `cumodp_tune_set_split`.
+    words, with k2 in {12, 13, 14} or the library's own value of that size,
+    and columns of 2^(k-k2) words. `cumodp_tune_set_split`.
   * The tile of the list multiply's mixed-size kernel: 2048, 4096 or 8192
     words per workgroup, which sets how many small products share a
     workgroup and how many waves run per CU. `cumodp_tune_set_list_tile`.
@@ -56,7 +56,13 @@ def _median_time(fn, reps, min_s=2e-3):
 
 
 def split_candidates(k):
-    return [k2 for k2 in (12, 13, 14) if 1 <= k - k2 <= 13]
+    """The row lengths that the library takes for 2^k points (its own among
+    them); the present one stays set."""
+    L = lib()
+    keep = L.cumodp_tune_get_split(k)
+    c = [k2 for k2 in range(4, 15) if L.cumodp_tune_set_split(k, k2) == 0]
+    _check("cumodp_tune_set_split", L.cumodp_tune_set_split(k, keep))
+    return c
 
 
 def tune_split(ks=range(14, 25), reps=5, p=P2, log=None):

@@ -816,7 +816,9 @@ cumodp_err cumodp_graph_destroy(void *graph) {
 
 int cumodp_tune_get_split(int k) {
     if (k <= kMaxLdsLog || k > kMaxLog) return 0;
-    return nominal_split(k);
+    int k1, k2;
+    four_step_split(k, k1, k2);
+    return k2;
 }
 
 cumodp_err cumodp_tune_set_list_tile(int words) {

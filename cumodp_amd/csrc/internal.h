@@ -13,7 +13,6 @@
 namespace cm {
 
 constexpr int kMaxLdsLog = 13;     // largest multiply done inside one workgroup
-constexpr int kMaxRowLog = 14;     // largest four-step row
 constexpr int kMaxLevelLog = 15;   // largest level of the twiddle tables (in-LDS 2^15 products)
 constexpr int kMaxLog = 26;        // largest transform supported (2^13 x 2^13)
 constexpr int kNoAllocMaxLog = 22; // largest transform of the non-allocating multiply
@@ -65,10 +64,9 @@ const Outer *outer_for_split(const Family *f, int k, int k1, int k2);
 const Family *family_default_cached(u32 p);
 const Outer *outer_cached(const Family *f, int k);
 
-// four-step split of a transform of size 2^k (k > kMaxLdsLog): columns of 2^k1
-// words (4 <= k1 <= 12), rows of 2^k2.  nominal_split: the row length 12, 13 or
-// 14 that cumodp_tune_set_split or CUMODP_SPLIT_<k>=<k2> names.
-int nominal_split(int k);
+// four-step split of a transform of size 2^k (kMaxLdsLog < k <= kMaxLog):
+// columns of 2^k1 words, rows of 2^k2, as cumodp_tune_set_split or
+// CUMODP_SPLIT_<k>=<k2> names them, else the library's own
 void four_step_split(int k, int &k1, int &k2);
 bool set_four_step_split(int k, int k2);
 

@@ -38,10 +38,10 @@ constexpr int mx_col_lds() {
 // X and Y point at the tile's first column; rows are 2^logn2 words apart.
 template <int LOGL, int LOGC, int V>
 CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const MxCtx &cx) {
-    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
+    constexpr int C = 1 << LOGC;
+    static_assert((C >= V || (C == 2 && V == 4)) && LOGL >= 4 && (C << LOGL) >= 256 * V,
                   "a wave's 256 V words lie inside the tile");
     using P = MxPlan<LOGL, LOGC>;
-    constexpr int C = 1 << LOGC;
     MxMat m;
     u32 x[1][V][4], tw[V][4];
     mx_forward_begin<LOGL, LOGC, V>(m, tw, cx);
@@ -52,6 +52,15 @@ CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int e = (int)(off + r * row);
+            if constexpr (C < V) {
+                // two columns of two rows
+#pragma unroll
+                for (int s = 0; s < V; ++s) {
+                    const int i = e + ((s >> LOGC) << logn2) + (s & (C - 1));
+                    x[0][s][r] = i < lim ? X[i] : 0u;
+                }
+                continue;
+            }
             if (V == 4 && e + V <= lim) {
                 const MxQuad v = *(const MxQuad *)(X + e);
 #pragma unroll
@@ -68,7 +77,11 @@ CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const
     u32 *q = Y + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
 #pragma unroll
     for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
-        if constexpr (V == 4) {
+        if constexpr (C < V) {
+            // two columns of rows r and r + 16
+            *(uint2 *)q = make_uint2(x[0][0][r], x[0][1][r]);
+            *(uint2 *)(q + ((size_t)16 << logn2)) = make_uint2(x[0][2][r], x[0][3][r]);
+        } else if constexpr (V == 4) {
             *(uint4 *)q = make_uint4(x[0][0][r], x[0][1][r], x[0][2][r], x[0][3][r]);
         } else {
 #pragma unroll
@@ -84,10 +97,10 @@ CM_DEV void mx_col_fwd(u32 *lds, const u32 *X, int lim, u32 *Y, int logn2, const
 template <int LOGL, int LOGC, int V, bool EDGES>
 CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fix, bool neg,
                        int logn2, const MxCtx &cx) {
-    static_assert((1 << LOGC) >= V && LOGL >= 4 && (1 << (LOGL + LOGC)) >= 256 * V,
+    constexpr int C = 1 << LOGC;
+    static_assert((C >= V || (C == 2 && V == 4)) && LOGL >= 4 && (C << LOGL) >= 256 * V,
                   "a wave's 256 V words lie inside the tile");
     using P = MxPlan<LOGL, LOGC>;
-    constexpr int C = 1 << LOGC;
     u32 x[V][4], tw[V][4];
     MxMat m = mx_load_mat(cx, kMxInv + P::T);
     {
@@ -95,7 +108,10 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fi
         const u32 *q = X + (((u32)(b >> LOGC) << logn2) + (b & (C - 1)));
 #pragma unroll
         for (int r = 0; r < 4; ++r, q += (size_t)1 << logn2) {
-            if constexpr (V == 4) {
+            if constexpr (C < V) {
+                const uint2 v = *(const uint2 *)q, w = *(const uint2 *)(q + ((size_t)16 << logn2));
+                x[0][r] = v.x; x[1][r] = v.y; x[2][r] = w.x; x[3][r] = w.y;
+            } else if constexpr (V == 4) {
                 const uint4 v = *(const uint4 *)q;
                 x[0][r] = v.x; x[1][r] = v.y; x[2][r] = v.z; x[3][r] = v.w;
             } else {
@@ -111,13 +127,14 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fi
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int e = (int)(off + r * row);
+        auto at = [&](int s) { return C < V ? e + ((s >> LOGC) << logn2) + (s & (C - 1)) : e + s; };
 #pragma unroll
         for (int s = 0; s < V; ++s) {
             x[s][r] = mx_canon(x[s][r], cx);
-            if (EDGES && e + s == fix) x[s][r] = cm_sub(x[s][r], 1u, cx.p);
+            if (EDGES && at(s) == fix) x[s][r] = cm_sub(x[s][r], 1u, cx.p);
             if (EDGES && neg) x[s][r] = cm_sub(0u, x[s][r], cx.p);
         }
-        if constexpr (V == 4) {
+        if constexpr (V == 4 && C >= V) {
             if ((!EDGES || e >= from) && e + V <= lim) {
                 *(MxQuad *)(Y + e) = MxQuad{{x[0][r], x[1][r], x[2][r], x[3][r]}};
                 continue;
@@ -125,7 +142,7 @@ CM_DEV void mx_col_inv(u32 *lds, const u32 *X, u32 *Y, int from, int lim, int fi
         }
 #pragma unroll
         for (int s = 0; s < V; ++s)
-            if ((!EDGES || e + s >= from) && e + s < lim) Y[e + s] = x[s][r];
+            if ((!EDGES || at(s) >= from) && at(s) < lim) Y[at(s)] = x[s][r];
     }
 }
 

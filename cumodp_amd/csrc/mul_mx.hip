@@ -3,6 +3,7 @@
 
 #include "internal.h"
 #include "mul_mx.h"
+#include "ntt_core.h"
 
 namespace cm {
 
@@ -343,7 +344,7 @@ static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int c
     constexpr int T = (1 << (LOGL + LOGC)) / (4 * V);
     ProfScope ps(inverse ? kProfColInv : kProfColFwd, s);
     const dim3 g(1u << (k2 - LOGC), cnt0 + cnt1);
-    if constexpr (V == 4 && LOGL + LOGC == 14 && LOGL >= 9) {
+    if constexpr (V == 4 && LOGL + LOGC == 14 && LOGL >= 9 && LOGC >= 2) {
         const int64_t tiles = (int64_t)g.x * g.y;
         const bool edges = s0.out_from || s0.out_xor || s0.monic || s0.neg;
         const bool whole = inverse || (s0.in_len % 4 == 0 && s1.in_len % 4 == 0);
@@ -418,7 +419,12 @@ static hipError_t launch_cols(int k1, bool inverse, const MxCols &s0, const MxCo
     }
     case 12: {
         constexpr int K = 12;
+        if (g_col_words == 8192) CM_COL(1, 2);
         CM_COL(2, 4);
+    }
+    case 13: {
+        constexpr int K = 13;
+        CM_COL(1, 4);
     }
     }
 #undef CM_COLB
@@ -431,6 +437,76 @@ hipError_t launch_cols_out(int k1, const u32 *X, u32 *Y, int64_t n, int cnt, int
                            const MxCtx &cx, hipStream_t s) {
     const MxCols c{X, Y, n, n, n, n};
     return launch_cols(k1, false, c, c, cnt, 0, k2, n * cnt <= kMxSmallWords, cx, s);
+}
+
+// Columns of 2, 4 and 8 words, which only named splits have: a thread takes a
+// column, as radix-2 butterflies in registers (a radix-16 step would be mostly
+// zeros).  A wave's loads and stores are 64 words of a row.  Both directions are
+// decimation in frequency with the root's or the inverse root's levels; position
+// r holds frequency r.  Input words are any 32 bits.
+template <int LOGL, bool INV>
+__global__ __launch_bounds__(256) void k_col_short(MxCols s0, MxCols s1, int cnt0, int logn2,
+                                                   const u32 *__restrict__ lv, Mod md, u32 r1,
+                                                   u32 sc) {
+    constexpr int L = 1 << LOGL;
+    const int y = blockIdx.y;
+    const MxCols &S = y < cnt0 ? s0 : s1;
+    const int64_t a = y < cnt0 ? y : y - cnt0;
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const u32 *X = S.in + a * S.in_stride;
+    u32 *Y = S.out + (INV ? a ^ S.out_xor : a) * S.out_stride;
+    u32 v[1][L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+        const int64_t e = ((int64_t)i << logn2) + c;
+        v[0][i] = e < S.in_len ? X[e] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < L; ++i) v[0][i] = cm_mul_tw(v[0][i], r1, md.p, md.np);
+    cm_dif_stages<LOGL, LOGL, 0, 0, 1>(v, 0, lv, md);
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+        const int64_t e = ((int64_t)i << logn2) + c;
+        u32 w = v[0][cm_brev((u32)i, LOGL)];
+        if (!INV) {
+            Y[e] = w;
+            continue;
+        }
+        w = cm_mul_tw(w, sc, md.p, md.np);
+        if (S.monic && e == 0) w = cm_sub(w, 1u, md.p);
+        if (S.neg) w = cm_sub(0u, w, md.p);
+        if (e >= S.out_from && e < S.out_len) Y[e] = w;
+    }
+    if (INV && S.monic && c == 0) Y[(int64_t)1 << (LOGL + logn2)] = 1u;
+}
+
+template <int LOGL>
+static hipError_t cols_short_t(bool inverse, const MxCols &s0, const MxCols &s1, int cnt0,
+                               int cnt1, int k2, const Family *fam, hipStream_t s) {
+    const Mod md{fam->p, fam->np};
+    const dim3 g(1u << (k2 - 8), cnt0 + cnt1);
+    const u32 r1 = cm_host_r1(fam->p),
+              sc = cm_host_mont(cm_host_inv((1u << LOGL) % fam->p, fam->p), fam->p);
+    ProfScope ps(inverse ? kProfColInv : kProfColFwd, s);
+    if (inverse)
+        hipLaunchKernelGGL((k_col_short<LOGL, true>), g, dim3(256), 0, s, s0, s1, cnt0, k2,
+                           fam->lvi, md, r1, sc);
+    else
+        hipLaunchKernelGGL((k_col_short<LOGL, false>), g, dim3(256), 0, s, s0, s1, cnt0, k2,
+                           fam->lv, md, r1, sc);
+    return hipGetLastError();
+}
+
+// The columns of any split that cumodp_tune_set_split takes.
+static hipError_t launch_cols_any(int k1, bool inverse, const MxCols &s0, const MxCols &s1,
+                                  int cnt0, int cnt1, int k2, bool small, const Family *fam,
+                                  hipStream_t s) {
+    switch (k1) {
+    case 1: return cols_short_t<1>(inverse, s0, s1, cnt0, cnt1, k2, fam, s);
+    case 2: return cols_short_t<2>(inverse, s0, s1, cnt0, cnt1, k2, fam, s);
+    case 3: return cols_short_t<3>(inverse, s0, s1, cnt0, cnt1, k2, fam, s);
+    }
+    return launch_cols(k1, inverse, s0, s1, cnt0, cnt1, k2, small, mx_ctx(fam), s);
 }
 
 template <int LOGL, int V>
@@ -472,15 +548,14 @@ hipError_t launch_mul_four_step_with(const FourStepIO &io, const Family *fam, co
     const int64_t n = (int64_t)1 << o->k;
     const MxCols sf{io.f_in, io.f_ws, io.in_stride, io.f_len, n, n};
     const MxCols sg{io.g_in, io.g_ws, io.g_stride < 0 ? io.in_stride : io.g_stride, io.g_len, n, n};
-    const MxCtx cx = mx_ctx(fam);
     const bool small = n * io.cnt <= kMxSmallWords;
     hipError_t e =
-        launch_cols(o->k1, false, sf, sg, io.cnt, io.cnt >> io.g_shift, o->k2, small, cx, s);
+        launch_cols_any(o->k1, false, sf, sg, io.cnt, io.cnt >> io.g_shift, o->k2, small, fam, s);
     if (e == hipSuccess) e = launch_rows(io, o, fam, s);
     if (e != hipSuccess) return e;
     const MxCols sh{io.f_ws, io.h_out, n, n, io.out_stride, io.h_len,
                     io.out_from, io.out_xor, io.monic, io.neg};
-    return launch_cols(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, cx, s);
+    return launch_cols_any(o->k1, true, sh, sh, io.cnt, 0, o->k2, small, fam, s);
 }
 
 hipError_t launch_mul_four_step(int k, const FourStepIO &io, const Family *fam, hipStream_t s) {

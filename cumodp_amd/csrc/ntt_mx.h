@@ -269,6 +269,14 @@ CM_DEV void mx_load_tw(u32 (&tw)[V][4], const u32 *tab) {
 #pragma unroll
             for (int s = 0; s < V; ++s) tw[s][r] = w;
         }
+    } else if constexpr (LOGC == 1 && V == 4) {
+        // two positions of two columns
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint2 w = *(const uint2 *)(q + (r << LOGS));
+            tw[0][r] = tw[1][r] = w.x;
+            tw[2][r] = tw[3][r] = w.y;
+        }
     } else if constexpr (V == 4 && LOGS >= 2) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -438,6 +446,13 @@ CM_DEV int mx_freq(int r, int logl) {
     int k = 0, shift = 0;
     for (; logl >= 4; logl -= 4, shift += 4) k |= ((r >> (logl - 4)) & 15) << shift;
     return k | ((r & ((1 << logl) - 1)) << shift);
+}
+
+// Position that holds frequency f (inverse of mx_freq).
+CM_DEV int mx_pos(int f, int logl) {
+    int r = 0;
+    for (; logl >= 4; logl -= 4, f >>= 4) r |= (f & 15) << (logl - 4);
+    return r | f;
 }
 
 // four consecutive words at a 4-byte aligned address

@@ -19,13 +19,6 @@
 
 namespace cm {
 
-// Position that holds frequency f (inverse of mx_freq).
-CM_DEV int mx_pos(int f, int logl) {
-    int r = 0;
-    for (; logl >= 4; logl -= 4, f >>= 4) r |= (f & 15) << (logl - 4);
-    return r | f;
-}
-
 // Rounds J .. NR-2 of a row tile and the exchange into the last round, whose
 // words are left in x: set s of lane (n, g) holds elements 4g .. 4g+3 of vector
 // id = 16 V wave + V n + s.  ROWS: id = u 2^LOGR + row, else row L/16 + u,

@@ -27,8 +27,7 @@ namespace {
 std::mutex g_plan_mutex;
 std::map<std::tuple<u32, u32, int>, Family *> g_families;
 std::map<std::tuple<const Family *, int, int>, Outer *> g_outer;
-int g_split[kMaxLog + 1];   // chosen k2 per k (0: default)
-int default_split(int k) { return k >= 25 ? 14 : (k >= 21 ? 13 : 12); }
+int g_split[kMaxLog + 1];   // named k2 per k (0: none)
 std::map<u32, const Family *> g_default;
 
 u32 *upload(const std::vector<u32> &h) {
@@ -194,41 +193,40 @@ const Family *family_default_cached(u32 p) {
     return it != g_default.end() ? it->second : nullptr;
 }
 
-// The row length 2^k2 that cumodp_tune_set_split or the environment names;
-// 12 (k <= 20), 13 (k <= 24) or 14 when nothing does.
-int nominal_split(int k) {
-    int c = (k >= 0 && k <= kMaxLog) ? g_split[k] : 0;
-    if (!c) {
-        char name[32];
-        snprintf(name, sizeof(name), "CUMODP_SPLIT_%d", k);
-        const char *e = getenv(name);
-        if (e) c = atoi(e);
-    }
-    if (c < 12 || c > 14 || k - c < 1 || k - c > kMaxLdsLog) c = default_split(k);
-    return c;
+// The library's own columns: short enough that both passes fill the chip
+// (measured over every split of 2^14 .. 2^24).
+static int own_split(int k) {
+    static const int k1[kMaxLog - kMaxLdsLog] = {6, 6, 6, 7, 8, 8, 8, 8, 10, 10, 11, 11, 12};
+    return k - k1[k - kMaxLdsLog - 1];
 }
 
-// The nominal value stands for the library's own choice: columns short enough
-// that both passes fill the chip (measured over every split of 2^14 .. 2^24).
-// Columns have 2^4 .. 2^12 words.  2^13 points (a few products of a tree level)
-// have no choice.
+// Row lengths that a caller may name: 2^12 to 2^14 with columns up to 2^13, and the
+// library's own.
+static bool named_split(int k, int k2) {
+    if (k <= kMaxLdsLog || k > kMaxLog) return false;
+    return k2 == own_split(k) || (k2 >= 12 && k2 <= 14 && k - k2 >= 1 && k - k2 <= kMaxLdsLog);
+}
+
+// 2^13 points (a few products of a tree level) have no choice.
 void four_step_split(int k, int &k1, int &k2) {
     if (k <= kMaxLdsLog) {
         k1 = 5;
         k2 = k - k1;
         return;
     }
-    static const int own[kMaxLog - kMaxLdsLog] = {6, 6, 6, 7, 8, 8, 8, 8, 10, 10, 11, 11, 12};
-    const int c = nominal_split(k);
-    k1 = c == default_split(k) ? own[k - kMaxLdsLog - 1] : k - c;
-    k1 = k1 < 4 ? 4 : (k1 > 12 ? 12 : k1);
-    k2 = k - k1;
+    k2 = g_split[k];
+    if (!k2) {
+        char name[32];
+        snprintf(name, sizeof(name), "CUMODP_SPLIT_%d", k);
+        const char *e = getenv(name);
+        if (e) k2 = atoi(e);
+    }
+    if (!named_split(k, k2)) k2 = own_split(k);
+    k1 = k - k2;
 }
 
 bool set_four_step_split(int k, int k2) {
-    if (k <= kMaxLdsLog || k > kMaxLog || k2 < 12 || k2 > 14 || k - k2 < 1 ||
-        k - k2 > kMaxLdsLog)
-        return false;
+    if (!named_split(k, k2)) return false;
     std::lock_guard<std::mutex> lk(g_plan_mutex);
     g_split[k] = k2;
     return true;

@@ -198,11 +198,10 @@ CUMODP_API cumodp_err cumodp_fast_evaluation(const sfixn *F, const sfixn *points
                                              sfixn *values);
 /* ---- tuning: four-step split ----------------------------------------------
  * Transforms of 2^k points above 2^13 run as 2^(k-k2) columns x 2^k2 rows;
- * this chooses k2 (12, 13 or 14) for one k.  The value that get returns when
- * nothing was set (12 up to 2^20, 13 up to 2^24, 14 above) stands for the
- * library's own split of that size; columns keep 2^4 .. 2^12 words whatever
- * is named.  The tuner (cumodp_amd/autotune.py) measures the candidates and
- * records its choice. */
+ * this chooses k2 (12, 13 or 14 with columns of 2 to 2^13 words, or the
+ * library's own value for that size, which get returns when nothing was set: 8
+ * to 14) for one k.  The tuner (cumodp_amd/autotune.py) measures the candidates
+ * and records its choice. */
 CUMODP_API cumodp_err cumodp_tune_set_split(int k, int k2);
 /* the current split k2 of 2^k-point transforms (0 when k needs none) */
 CUMODP_API int cumodp_tune_get_split(int k);
@@ -230,9 +229,9 @@ CUMODP_API int cumodp_tune_get_list_persistent(void);
  * transform work for the narrower products) */
 CUMODP_API cumodp_err cumodp_tune_set_zmul_merge(int merge);
 CUMODP_API int cumodp_tune_get_zmul_merge(void);
-/* words per workgroup tile of the four-step multiply's column passes above
- * 2^20 words, for columns of 2^9 to 2^11 words: 16384 (the default; 1024
- * threads) or 8192 (512 threads, more workgroups) */
+/* words per workgroup tile of the four-step passes over columns of 2^9 to 2^12
+ * words, above 2^20 words in all: 16384 (the default; 1024 threads) or 8192
+ * (half the columns, more workgroups) */
 CUMODP_API cumodp_err cumodp_tune_set_col_tile(int words);
 CUMODP_API int cumodp_tune_get_col_tile(void);
 

@@ -37,3 +37,112 @@ def test_many_short_rows(cm, orc, k, p):
     for off, m in enumerate((base, base + 1, base + per - 1, base + per + 1)):
         check = sorted({0, 1, per - 1, per, m // 2, m - 2, m - 1})
         _rows(cm, orc, m, k, p, off, check, 100 * k + off)
+
+
+class _Splits:
+    """Named row lengths {k: k2} for a while."""
+
+    def __init__(self, cm, named):
+        self.L, self.named = cm.lib(), named
+
+    def __enter__(self):
+        self.keep = {k: self.L.cumodp_tune_get_split(k) for k in self.named}
+        for k, k2 in self.named.items():
+            assert self.L.cumodp_tune_set_split(k, k2) == 0, (k, k2)
+            assert self.L.cumodp_tune_get_split(k) == k2
+
+    def __exit__(self, *exc):
+        for k, k2 in self.keep.items():
+            assert self.L.cumodp_tune_set_split(k, k2) == 0
+            assert self.L.cumodp_tune_get_split(k) == k2
+
+
+@pytest.mark.parametrize("k2", [12, 13, 14])
+def test_a_named_split_is_the_one_that_runs(cm, k2):
+    """The tables of a split are built by its first product, and the
+    non-allocating multiply refuses a split without tables."""
+    k, n = 18, 1 << 18
+    rng = np.random.default_rng(k2)
+    F, G = (cm.DeviceArray.from_host(rng.integers(0, P1, n // 2, dtype=np.int32)) for _ in "FG")
+    H = cm.DeviceArray(n - 1)
+    def mul(**kw):
+        cm.fftmul_uni_dev(n - 2, H, n // 2 - 1, F, n // 2 - 1, G, P1, **kw)
+        return H.download()
+    want = mul()
+    assert (mul(noalloc=True) == want).all()
+    assert cm.lib().cumodp_tune_get_split(k) not in (12, 13, 14)
+    with _Splits(cm, {k: k2}):
+        with pytest.raises(cm.CumodpError):
+            mul(noalloc=True)
+        assert (mul() == want).all()
+        assert (mul(noalloc=True) == want).all()
+
+
+def test_splits_refused(cm):
+    L = cm.lib()
+    for k, k2 in ((13, 12), (14, 11), (14, 14), (17, 9), (20, 11), (26, 12), (27, 14), (22, 15)):
+        keep = L.cumodp_tune_get_split(k)
+        assert L.cumodp_tune_set_split(k, k2) == cm.CUMODP_ASSUMPTION_ERROR, (k, k2)
+        assert L.cumodp_tune_get_split(k) == keep
+
+
+@pytest.mark.parametrize("k,k2", [(24, 12), (25, 12), (25, 13), (26, 13)])
+def test_longest_columns(cm, k, k2):
+    """Columns of 2^12 and 2^13 words in both tiles, against the library's own split
+    and the product's values at 1, -1 and the square roots of -1."""
+    L, p, n = cm.lib(), P2, 1 << k
+    rng = np.random.default_rng(k)
+    F, G = (rng.integers(0, p, m, dtype=np.int32) for m in (n // 2 - 3, n // 2 + 1))
+    dF, dG, dH = cm.DeviceArray.from_host(F), cm.DeviceArray.from_host(G), cm.DeviceArray(n - 3)
+
+    def mul():
+        cm.fftmul_uni_dev(n - 4, dH, len(F) - 1, dF, len(G) - 1, dG, p)
+        return dH.download()
+
+    def at(X):
+        """values at the fourth roots of unity"""
+        s = [int(X[j::4].astype(np.int64).sum()) for j in range(4)]
+        return [sum(v * pow(w, j, p) for j, v in enumerate(s)) % p
+                for w in (pow(31, (p - 1) // 4 * t, p) for t in range(4))]
+
+    want = mul()
+    assert [a * b % p for a, b in zip(at(F), at(G))] == at(want)
+    try:
+        with _Splits(cm, {k: k2}):
+            for tile in (16384, 8192):
+                assert L.cumodp_tune_set_col_tile(tile) == 0
+                assert (mul() == want).all(), (k, k2, tile)
+    finally:
+        assert L.cumodp_tune_set_col_tile(16384) == 0
+
+
+@pytest.mark.parametrize("named", [{14: 13, 15: 13, 16: 13, 17: 14}, {14: 12, 15: 12, 16: 14, 17: 12},
+                                   {14: 13, 15: 14, 16: 12, 17: 13}])
+@pytest.mark.parametrize("p", [P1, P2])
+def test_trees_and_lists_on_named_splits(cm, orc, p, named):
+    """Monic nodes, middle products (with coefficients of any 32 bits) and batched
+    products over columns of 2 to 32 words: the words of the library's own
+    splits."""
+    rng = np.random.default_rng(9)
+    k = 16
+    pts = rng.integers(0, p, 1 << k, dtype=np.int32)
+    pts[:2] = 0, p - 1
+    F = rng.integers(0, 1 << 32, 1 << k, dtype=np.uint64).astype(np.uint32).view(np.int32)
+    f = [rng.integers(0, p, m, dtype=np.int32) for m in (30000, 40000, 70001, 33000)]
+    items, nf, ng, nh = cm.make_items([len(x) - 1 for x in f], [len(x) - 2 for x in f])
+    dF = cm.DeviceArray.from_host(np.concatenate(f))
+    dG = cm.DeviceArray.from_host(np.concatenate([x[::-1][1:] for x in f]))
+
+    def run():
+        H = cm.DeviceArray.from_host(np.full(nh, -1, np.int32))
+        cm.list_fftmul_dev(items, dF, dG, H, p)
+        tree = cm.subproduct_tree(pts, p)
+        return [H.download(), cm.fast_evaluation(F, pts, p)] + [np.concatenate(t) for t in tree]
+
+    want = run()
+    it = items[2]
+    assert (want[0][it.h_off:it.h_off + it.df + it.dg + 1] ==
+            orc.ntt_polymul(f[2], f[2][::-1][1:].copy(), p)).all()
+    with _Splits(cm, named):
+        for a, b in zip(run(), want):
+            assert (a == b).all()
