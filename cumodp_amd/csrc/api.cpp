@@ -1109,9 +1109,13 @@ void stockham_poly_mul_dev(sfixn n, sfixn e, sfixn *F, sfixn *G, sfixn p) {
             he = launch_mul_lds_one(e, (const u32 *)F, (const u32 *)G, (u32 *)F, nullptr, 1, d,
                                     fam, 0);
         } else if (fam) {
-            FourStepIO io{(const u32 *)F, (const u32 *)G, n, n, 0, (u32 *)F, (u32 *)G, (u32 *)F,
-                          n, 0, 1};
-            he = launch_mul_four_step(e, io, fam, 0);
+            // in place where the passes' 16-byte accesses may work on F and G
+            const bool aligned = (((uintptr_t)F | (uintptr_t)G) & 15) == 0;
+            const size_t bytes = sizeof(u32) * (size_t)n;
+            u32 *wf = aligned ? (u32 *)F : (u32 *)workspace(0, bytes, 0);
+            u32 *wg = aligned ? (u32 *)G : (u32 *)workspace(1, bytes, 0);
+            FourStepIO io{(const u32 *)F, (const u32 *)G, n, n, 0, wf, wg, (u32 *)F, n, 0, 1};
+            if (wf && wg) he = launch_mul_four_step(e, io, fam, 0);
         }
         if (he == hipSuccess) he = hipStreamSynchronize(0);
         if (he != hipSuccess) ce = fail(CUMODP_FFT_ERROR, "multiply", he);

@@ -146,3 +146,21 @@ def test_trees_and_lists_on_named_splits(cm, orc, p, named):
     with _Splits(cm, named):
         for a, b in zip(run(), want):
             assert (a == b).all()
+
+
+@pytest.mark.parametrize("e", [13, 14, 17, 21])
+def test_cyclic_product_at_any_word(cm, orc, e):
+    """stockham_poly_mul_dev on operands at every word of a 16-byte block."""
+    p, n = P1, 1 << e
+    rng = np.random.default_rng(e)
+    F, G = (rng.integers(0, p, n, dtype=np.int32) for _ in "FG")
+    full = np.append(orc.ntt_polymul(F, G, p), 0).astype(np.int64)
+    want = ((full[:n] + full[n:]) % p).astype(np.int32)
+    for a, b in ((0, 0), (1, 0), (0, 2), (3, 3)):
+        dF = cm.DeviceArray.from_host(np.concatenate([np.full(a, 5, np.int32), F, [6] * 4]).astype(np.int32))
+        dG = cm.DeviceArray.from_host(np.concatenate([np.full(b, 5, np.int32), G, [6] * 4]).astype(np.int32))
+        cm.cxx("stockham_poly_mul_dev")(n, e, dF.addr(a), dG.addr(b), p)
+        got, other = dF.download(), dG.download()
+        assert (got[a:a + n] == want).all(), (e, a, b)
+        assert (got[:a] == 5).all() and (got[a + n:] == 6).all(), (e, a, b)
+        assert (other[:b] == 5).all() and (other[b + n:] == 6).all(), (e, a, b)
