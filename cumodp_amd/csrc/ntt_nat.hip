@@ -279,12 +279,8 @@ template <int LOGL, int LOGR, int V>
 static hipError_t row_nat_t(const u32 *Y, u32 *X, int cnt, int k1, const MxOuter &o,
                             const MxCtx &cx, hipStream_t s) {
     ProfScope ps(kProfRowOut, s);
-    for (int a = 0; a < cnt; a += 65535) {
-        const int64_t at = (int64_t)a << (k1 + LOGL);
-        hipLaunchKernelGGL((k_row_nat<LOGL, LOGR, V>),
-                           dim3(1u << (k1 - LOGR), std::min(cnt - a, 65535)),
-                           dim3((1 << (LOGL + LOGR)) / (4 * V)), 0, s, Y + at, X + at, k1, o, cx);
-    }
+    hipLaunchKernelGGL((k_row_nat<LOGL, LOGR, V>), dim3(1u << (k1 - LOGR), cnt),
+                       dim3((1 << (LOGL + LOGR)) / (4 * V)), 0, s, Y, X, k1, o, cx);
     return hipGetLastError();
 }
 
@@ -299,6 +295,11 @@ static void ntt_split(int k, int &k1, int &k2) {
 hipError_t launch_ntt_four_step(int k, u32 *X, u32 *Y, int cnt, bool inverse, const Family *fam,
                                 hipStream_t s) {
     if (k <= kMaxLdsLog || k > kMaxLog || k > fam->K) return hipErrorInvalidValue;
+    // both passes take their arrays in grid.y
+    for (; cnt > 65535; cnt -= 65535, X += (int64_t)65535 << k, Y += (int64_t)65535 << k) {
+        const hipError_t e = launch_ntt_four_step(k, X, Y, 65535, inverse, fam, s);
+        if (e != hipSuccess) return e;
+    }
     int k1, k2;
     ntt_split(k, k1, k2);
     const Outer *o = outer_for_split(fam, k, k1, k2);

@@ -164,3 +164,21 @@ def test_cyclic_product_at_any_word(cm, orc, e):
         assert (got[a:a + n] == want).all(), (e, a, b)
         assert (got[:a] == 5).all() and (got[a + n:] == 6).all(), (e, a, b)
         assert (other[:b] == 5).all() and (other[b + n:] == 6).all(), (e, a, b)
+
+
+def test_more_rows_than_a_grid_holds(cm, orc):
+    """65540 rows of 2^14 words: both passes are launched in parts."""
+    k, m, p = 14, 65540, P1
+    n, w = 1 << k, _root(k, P1)
+    d = cm.DeviceArray(m * n)
+    cm.cxx("reset_vector_dev")(m * n, d.addr())
+    rng = np.random.default_rng(14)
+    rows = {r: rng.integers(0, p, n, dtype=np.int32) for r in (0, 1, 65534, 65535, 65536, m - 1)}
+    for r, x in rows.items():
+        d.upload(x, r * n)
+    cm.cxx("list_stockham_dev_w")(d.addr(), m, k, w, p)
+    for r, x in rows.items():
+        assert (d.download(n, r * n) == orc.stockham(x, w, p)).all(), r
+    for r in (2, 65533, 65537):
+        assert (d.download(n, r * n) == 0).all(), r
+    d.free()
