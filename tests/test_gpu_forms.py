@@ -3,6 +3,8 @@ each against the CPU oracle (exact residues and integers)."""
 import numpy as np
 import pytest
 
+from cumodp_amd.serving import out_words
+
 pytestmark = pytest.mark.gpu
 
 P1, P2 = 469762049, 2013265921
@@ -182,3 +184,116 @@ def test_more_rows_than_a_grid_holds(cm, orc):
     for r in (2, 65533, 65537):
         assert (d.download(n, r * n) == 0).all(), r
     d.free()
+
+
+@pytest.mark.parametrize("m,k", [(9, 17), (5, 18), (3, 19), (3, 20), (2, 21), (2, 22), (70, 14), (40, 15),
+                                 (17, 16), (300, 14)])
+@pytest.mark.parametrize("p", [P1, P2])
+def test_rows_of_two_passes(cm, orc, m, k, p):
+    """Several rows above 2^13 words, more than 2^20 words in all: row tiles of 8
+    and 16 frequencies; with the inverse root and 1/2^k, back again."""
+    n, w = 1 << k, _root(k, p)
+    _rows(cm, orc, m, k, p, 1, sorted({0, m // 2, m - 1}), 10 * k + m)
+    X = np.random.default_rng(k).integers(0, p, m * n, dtype=np.int32)
+    d = cm.DeviceArray.from_host(X)
+    f = cm.cxx("list_stockham_dev_w")
+    f(d.addr(), m, k, w, p)
+    f(d.addr(), m, k, pow(w, p - 2, p), p)
+    back = d.download().astype(np.int64) * pow(n, p - 2, p) % p
+    assert (back == X).all()
+
+
+@pytest.mark.parametrize("persistent,count,logn", [(1, 70, 16), (1, 35, 17), (1, 20, 18), (1, 9, 19),
+                                                   (0, 100, 14), (0, 300, 14), (0, 150, 15),
+                                                   (0, 40, 15)])
+@pytest.mark.parametrize("p", [P1, P2])
+def test_batched_four_step_products(cm, orc, persistent, count, logn, p):
+    """Lists of one four-step size above 2^20 and above 2^22 words: two and four
+    sets per lane in rows of 2^8 to 2^11 words."""
+    rng = np.random.default_rng(count)
+    n, df, dg = 1 << logn, [], []
+    for _ in range(count):
+        s = int(rng.integers(n // 2 + 1, n + 1))
+        x = int(rng.integers(s // 4, s // 2))
+        df.append(x)
+        dg.append(s - 1 - x)
+    items, nf, ng, nh = cm.make_items(df, dg)
+    F, G = (rng.integers(0, p, m, dtype=np.int32) for m in (nf, ng))
+    H = cm.DeviceArray.from_host(np.full(nh, -1, np.int32))
+    L = cm.lib()
+    keep = L.cumodp_tune_get_list_persistent()
+    try:
+        assert L.cumodp_tune_set_list_persistent(persistent) == 0
+        cm.list_fftmul_dev(items, cm.DeviceArray.from_host(F), cm.DeviceArray.from_host(G), H, p)
+        got = H.download()
+    finally:
+        assert L.cumodp_tune_set_list_persistent(keep) == 0
+    for i in sorted({0, 1, count // 2, count - 1}):
+        it = items[i]
+        f, g = F[it.f_off:it.f_off + it.df + 1], G[it.g_off:it.g_off + it.dg + 1]
+        assert (got[it.h_off:it.h_off + it.df + it.dg + 1] == orc.ntt_polymul(f, g, p)).all(), i
+
+
+def _zpair(rng, s, nb, bits):
+    """Operands of s + 1 coefficients in all, the extremes of the width among them."""
+    lim = (1 << (bits - 1)) - 1 if bits == 64 else (1 << bits) - 1
+    a, b = (rng.integers(-lim, lim, n, dtype=np.int64, endpoint=True) for n in (s + 1 - nb, nb))
+    a[0] = a[-1] = b[0] = -lim
+    return a, b
+
+
+def test_integer_batch_of_long_rows(cm, orc):
+    """One batch with rows of 2^17 to 2^21 points (and short ones): four-step passes
+    of several column and row lengths in one list, and the rows above 2^20 after
+    it.  One operand is short, since the check is schoolbook."""
+    rng = np.random.default_rng(21)
+    A, items, at, out = [], [], 0, 0
+    for e in (17, 21, 19, 20, 18, 5, 13, 17, 20):
+        for bits in (16, 34, 64) if e < 20 else (34,):
+            s = (1 << e) - int(rng.integers(0, 3))
+            a, b = _zpair(rng, s, int(rng.integers(5, 24)), bits)
+            if len(items) % 2:
+                a, b = b, a
+            wc = out_words(bits, len(a), len(b))
+            items.append((at, at + len(a), out, len(a), len(b), 1, 1, wc, bits))
+            A += [a, b]
+            at += len(a) + len(b)
+            out += (len(a) + len(b) - 1) * wc
+    arr = (cm.ZmulItem * len(items))(*[cm.ZmulItem(*t) for t in items])
+    D = cm.DeviceArray.from_host(np.concatenate(A).view(np.uint64), np.uint64)
+    H = cm.DeviceArray.from_host(np.full(out, 0x5A5A5A5A5A5A5A5A, np.uint64), np.uint64)
+    assert cm.lib().cumodp_two_convolution_list_dev(arr, len(items), D.addr(), D.addr(), H.addr(),
+                                                    None) == 0
+    got = H.download()
+    for i, t in enumerate(items):
+        na, nb, wc = t[3], t[4], t[7]
+        want = orc.zmul_i64(A[2 * i], A[2 * i + 1])[:, :wc]
+        assert (got[t[2]:t[2] + (na + nb - 1) * wc].reshape(-1, wc) == want).all(), t
+
+
+@pytest.mark.parametrize("e,bits", [(18, 16), (19, 34), (19, 64), (20, 34), (21, 34), (21, 64)])
+def test_long_integer_products(cm, orc, e, bits):
+    rng = np.random.default_rng(e)
+    a, b = _zpair(rng, (1 << e) - 1, 19, bits)
+    wc = out_words(bits, len(a), len(b))
+    dA, dB = (cm.DeviceArray.from_host(x.view(np.uint64), np.uint64) for x in (a, b))
+    H = cm.DeviceArray((len(a) + len(b) - 1) * wc, np.uint64)
+    assert cm.lib().cumodp_two_convolution_poly_mul_dev(
+        dA.addr(), len(a), 1, dB.addr(), len(b), 1, H.addr(), wc, bits, None) == 0
+    assert (H.download().reshape(-1, wc) == orc.zmul_i64(a, b)[:, :wc]).all()
+
+
+@pytest.mark.parametrize("e,p", [(22, P1), (22, P2), (23, P2)])
+def test_column_loop(cm, orc, e, p):
+    """512 column tiles and more, operands of whole quads and unlike lengths, the
+    product whole and cut inside a quad."""
+    rng = np.random.default_rng(e)
+    lf, lg = (5 << (e - 3)) - 12, (3 << (e - 3)) - 8
+    F, G = (rng.integers(0, p, m, dtype=np.int32) for m in (lf, lg))
+    want = orc.ntt_polymul(F, G, p)
+    dF, dG = cm.DeviceArray.from_host(F), cm.DeviceArray.from_host(G)
+    for nout in (lf + lg - 1, lf + 1):
+        H = cm.DeviceArray.from_host(np.full(lf + lg + 3, -1, np.int32))
+        cm.fftmul_uni_dev(nout - 1, H, lf - 1, dF, lg - 1, dG, p)
+        got = H.download()
+        assert (got[:nout] == want[:nout]).all() and (got[nout:] == -1).all(), nout
