@@ -613,7 +613,7 @@ def bench_serving(cm, cpu, nreq=20000, max_batch_ms=1.5, age_factor=0.5):
     Q = serving.make_requests(w)
     log(f"bench: serving: {Q.n} requests generated in {time.perf_counter() - t0:.1f} s, "
         f"{Q.total_coeffs} output coefficients")
-    srv = serving.ZmulServer(slots=2, slot_bytes=1 << 30, age_factor=age_factor)
+    srv = serving.ZmulServer(slots=3, slot_bytes=1 << 30, age_factor=age_factor)
     runs = []
     try:
         srv.run(Q, np.zeros(Q.n))   # warm-up pass (plans, twiddles, buffers)
@@ -746,7 +746,7 @@ def counter_calls(cm, line, ncalls):
     elif line == "serving":
         from cumodp_amd import serving
         Q = serving.make_requests(cm.workload5())
-        srv = serving.ZmulServer(slots=2, slot_bytes=1 << 30)   # the capacity run: no time cap
+        srv = serving.ZmulServer(slots=3, slot_bytes=1 << 30)   # the capacity run: no time cap
         run = lambda: srv.run(Q, np.zeros(Q.n))
     else:
         raise SystemExit(f"no counter form for line {line}")

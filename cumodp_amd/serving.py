@@ -9,14 +9,19 @@ sequence of batched launches. Results are copied back into the caller's
 result buffer.
 
 Design:
-  * Two slots, each with its own HIP stream and device buffers. While one
-    batch computes, the next one uploads and launches on the other slot;
-    a third holds the batch whose products are copied back. All streams have
-    the default priority.
-  * One copy back at a time, queued when the batch ahead has left. Copies
-    that share the link end together, and the slots then stay in step, with
-    the link idle while they compute: 20,000 requests at once took 0.231 s
-    so, 0.180 s with the copies one at a time, 0.154 s with the third slot.
+  * `slots` slots, each with its own HIP stream and device buffers, all
+    streams of the default priority: while one batch's products are copied
+    back, others upload and compute. Copies that share the link end together,
+    and two slots would stay in step, with the link idle while both compute:
+    20,000 requests at once took 0.223 s so.
+  * With two slots (the default) one batch therefore computes at a time: the
+    next one is launched when its products are ready, their copy back having
+    been queued first. 20,000 requests at once: 0.137 s once the buffers have
+    their sizes; at 85,000 requests a second half of them are back in 0.5 ms
+    and 99% in 1.0 ms (1.3 and 2.4 to 4.8 with two batches in step).
+  * With three and more the copies back go one at a time instead, each queued
+    when the batch ahead has left, and a free slot launches at once. Three
+    slots: 0.123 s, 0.9 and 2.0 ms.
   * FIFO admission. A batch is a contiguous range of request ids, so its
     inputs and outputs are contiguous in the packed pinned host buffers:
     one host-to-device copy in and one device-to-host copy out per batch.
@@ -148,6 +153,7 @@ class _Slot:
         self.din = self.dout = None
         self.cap_in = self.cap_out = 0
         self.range = None            # (i0, i1) in flight
+        self.collected = False       # its copy back is queued
         self.units = 0.0             # its work count
         self.t_launch = 0.0          # when it was launched (seconds into the run)
 
@@ -178,14 +184,13 @@ class _Slot:
 
 
 class ZmulServer:
-    """Continuous batching over `slots` streams; a batch holds at most
+    """Continuous batching over `slots` streams; each holds one batch, of at most
     `slot_bytes` of inputs, outputs and estimated transform scratch, and at
     most max(`max_batch_s`, `age_factor` x the oldest waiting request's age)
     seconds of estimated GPU work (max_batch_s None: no time cap)."""
 
     def __init__(self, slots=2, slot_bytes=1 << 30, max_batch_s=None, age_factor=0.0):
-        # one more for the batch whose products are copied back
-        self.slots = [_Slot() for _ in range(slots + 1)]
+        self.slots = [_Slot() for _ in range(slots)]
         self.slot_bytes = int(slot_bytes)
         self.max_batch_s = max_batch_s
         self.age_factor = age_factor
@@ -280,6 +285,7 @@ class ZmulServer:
             items.ctypes.data_as(C.POINTER(ZmulItem)), n, C.c_void_p(slot.din),
             C.c_void_p(slot.din), C.c_void_p(slot.dout), st))
         slot.range = (i0, i1)
+        slot.collected = False
         slot.units = self._batch_units(Q, i0, i1)
 
     def _collect(self, slot, Q):
@@ -289,16 +295,25 @@ class ZmulServer:
         _check("cumodp_memcpy_d2h_async", lib().cumodp_memcpy_d2h_async(
             C.c_void_p(Q.OUT.ptr + 8 * out0), C.c_void_p(slot.dout), 8 * (out1 - out0),
             C.c_void_p(slot.stream)))
+        slot.collected = True
+
+    @staticmethod
+    def _ready(slot):
+        """True when everything queued on the slot's stream has run."""
+        q = lib().cumodp_stream_query(C.c_void_p(slot.stream))
+        if q < 0:
+            raise CumodpError("cumodp_stream_query", 0x999)
+        return q > 0
 
     def run(self, Q, arrivals):
         """Serve requests 0..Q.n-1 arriving at `arrivals` (seconds from the
         start, non-decreasing).  Returns (done, stats): done[r] is the time
         (seconds from the start) at which product r was back in host memory."""
-        L = lib()
         N = Q.n
         arrivals = np.asarray(arrivals, np.float64)
         done = np.full(N, np.nan)
         inflight = collections.deque()
+        serial = len(self.slots) <= 2    # one batch computes at a time
         free = list(self.slots)
         head = 0
         batches = []
@@ -308,12 +323,7 @@ class ZmulServer:
         while retired < N:
             now = time.perf_counter() - t0
             # retire finished batches in launch order
-            while inflight:
-                q = L.cumodp_stream_query(C.c_void_p(inflight[0].stream))
-                if q < 0:
-                    raise CumodpError("cumodp_stream_query", 0x999)
-                if q == 0:
-                    break
+            while inflight and inflight[0].collected and self._ready(inflight[0]):
                 s = inflight.popleft()
                 t = time.perf_counter() - t0
                 i0, i1 = s.range
@@ -325,10 +335,15 @@ class ZmulServer:
                 last_done = t
                 s.range = None
                 free.append(s)
-                if inflight:
-                    self._collect(inflight[0], Q)
+            # the copy back of the newest batch once it has computed, or of the
+            # oldest one behind its kernels
+            if inflight:
+                s = inflight[-1 if serial else 0]
+                if not s.collected and (not serial or self._ready(s)):
+                    self._collect(s, Q)
             arrived = int(np.searchsorted(arrivals, now, side="right"))
-            if head < arrived and free:
+            if head < arrived and free and not (serial and inflight and
+                                                not inflight[-1].collected):
                 self._age = now - arrivals[head]
                 j = self._fit(Q, head, arrived)
                 s = free.pop(0)
@@ -336,8 +351,6 @@ class ZmulServer:
                 self._launch(s, Q, head, j)
                 batches.append(j - head)
                 inflight.append(s)
-                if len(inflight) == 1:
-                    self._collect(s, Q)
                 head = j
                 continue
             if not inflight and head < N and head >= arrived:
