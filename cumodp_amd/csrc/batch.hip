@@ -910,9 +910,31 @@ static int cost_bucket(double x) {
     return b > 63 ? 63 : b;
 }
 
-static bool is_plain(const MulDesc &d) {
-    return g_plain_cutoff > 0 && std::min(d.lf, d.lg) <= g_plain_cutoff;
-}
+// What the products of a list call are.  Their classes come in no order, so the
+// passes have no branch on them (20000 pairs of degrees 16 .. 300: 227 us per call
+// with three passes that do, 155 us so).
+struct ListCount {
+    int64_t cls[33];              // products by class: 0 schoolbook, e 2^e points
+    int64_t plain = 0;            // small tasks of the schoolbook products
+    int64_t pieces = 0;           // small tasks of the 2^15-point products
+    int cut;                      // class 0: a side of at most cut words
+
+    int of(const MulDesc &d) const { return std::min(d.lf, d.lg) <= cut ? 0 : d.logn; }
+    // a product's tasks of `words` words if it is of class c
+    int64_t tasks(const MulDesc &d, int c, int words) const {
+        return (uint32_t)(d.lh + words - 1) / (uint32_t)words & -(uint32_t)(of(d) == c);
+    }
+    ListCount(const MulDesc *descs, int64_t count) : cut(g_plain_cutoff) {
+        uint32_t n[2][33] = {};   // neighbours count apart
+        for (int64_t i = 0; i < count; ++i) {
+            ++n[i & 1][of(descs[i])];
+            plain += tasks(descs[i], 0, ListGeo<13>::PlainOut);
+        }
+        for (int c = 0; c < 33; ++c) cls[c] = (int64_t)n[0][c] + n[1][c];
+        for (int64_t i = 0; cls[kBigLog] && i < count; ++i)
+            pieces += tasks(descs[i], kBigLog, ListGeo<13>::W);
+    }
+};
 
 // tiles of 2^log words that the classes 2^4 .. 2^log fill
 static int64_t list_tiles(const int64_t (&ncls)[33], int log) {
@@ -932,32 +954,37 @@ static int64_t list_tiles(const int64_t (&ncls)[33], int log) {
 // products of 2^14 points: 71 us and 84; 700 with 116 of 2^15 and as many words
 // of 2^13 and 2^11: 174 and 196).  The other lists take small tasks (4096 pairs
 // of degrees 32 .. 16384: 187 us).  Measured over 220 mixes of sizes.  Schoolbook
-// products alone take large tasks, of which there are half as many (16 products
-// of 20 by 50000 coefficients: 13.0 us, 15.0 as small ones).  pieces: small tasks
-// of the 2^15-point products.
-static int list_log(const int64_t (&ncls)[33], int64_t pieces) {
+// products alone take large tasks, which are fewer (16 products of 20 by 50000
+// coefficients: 13.0 us, 15.0 as small ones); many of up to 3/2 small tasks, which
+// leave most waves of a large one idle, keep their list to small tasks (the kernel
+// of 20000 pairs of degrees 16 .. 300: 119 us, 138 with large ones).
+static int list_log(const ListCount &n) {
+    const int64_t (&ncls)[33] = n.cls, pieces = n.pieces;
     const int64_t tiles = list_tiles(ncls, 13), n14 = ncls[14], n15 = ncls[15];
     const int64_t large = list_tiles(ncls, 14) + 2 * n15;
-    if (large == 0) return 14;
+    const bool shorts = 2 * n.plain < 3 * ncls[0];
+    if (large == 0) return shorts ? 13 : 14;
     const int64_t cus = device_cus();
+    if (shorts && n.plain > cus) return 13;
     if (large <= cus) return tiles + 2 * n14 + pieces > cus ? 14 : 13;
     const bool half = 2 * n14 >= tiles + 4 * n15;
     return half && large <= 8 * cus && (tiles + n14 + n15 < 4 * cus || n15 > 0) ? 14 : 13;
 }
 
 template <int LOG>
-static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const int64_t (&ncls)[33],
-                                    int64_t pieces, const u32 *F, const u32 *G, u32 *H,
-                                    const Family *fam, hipStream_t s) {
+static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const ListCount &nl,
+                                    const u32 *F, const u32 *G, u32 *H, const Family *fam,
+                                    hipStream_t s) {
     using Geo = ListGeo<LOG>;
+    const int64_t (&ncls)[33] = nl.cls;
     int64_t off[34];
     off[0] = 0;
     for (int c = 0; c < 33; ++c) off[c + 1] = off[c] + ncls[c];
     int64_t nbig = 0, ntasks = list_tiles(ncls, LOG);
     for (int e = LOG + 1; e <= kBigLog; ++e) nbig += ncls[e];
-    ntasks += nbig;
-    for (int64_t i = 0; ncls[0] && i < count; ++i)
-        if (is_plain(descs[i])) ntasks += (descs[i].lh + Geo::PlainOut - 1) / Geo::PlainOut;
+    ntasks += nbig + (LOG == 13 ? nl.plain : 0);
+    for (int64_t i = 0; LOG == 14 && ncls[0] && i < count; ++i)
+        ntasks += nl.tasks(descs[i], 0, Geo::PlainOut);
     // Small tasks: below four per CU (two rounds of workgroups), or with products of
     // 2^15 points below 3 1/2 rounds of pieces, a whole product would leave the
     // chip waiting at the end, so every piece is a task, at the price of a
@@ -969,7 +996,8 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const i
         if (LOG == 14 || stream_capturing(s)) return LOG == 14;
         const int64_t cus = device_cus();
         return ntasks < 4 * cus ||
-               (pieces > 0 && list_tiles(ncls, 13) + 2 * ncls[14] + pieces < 7 * cus);
+               (ncls[kBigLog] > 0 &&
+                list_tiles(ncls, 13) + 2 * ncls[14] + nl.pieces < 7 * cus);
     };
     u32 *big_s = nullptr;
     if (nbig > 0 && split()) {
@@ -977,13 +1005,8 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const i
         if (!big_s) (void)hipGetLastError();   // whole products need no scratch
     }
     if (LOG == 14 && nbig > 0 && !big_s)
-        return list_persistent_t<13>(descs, count, ncls, pieces, F, G, H, fam, s);
-    if (big_s) {
-        ntasks -= nbig;
-        for (int64_t i = 0; i < count; ++i)
-            if (!is_plain(descs[i]) && descs[i].logn > LOG && descs[i].logn <= kBigLog)
-                ntasks += big_pieces<LOG>(descs[i].lf + descs[i].lg - 1);
-    }
+        return list_persistent_t<13>(descs, count, nl, F, G, H, fam, s);
+    if (big_s) ntasks += (LOG == 13 ? 2 * ncls[14] + nl.pieces : 2 * nbig) - nbig;
     if (ntasks > INT32_MAX) return hipErrorInvalidValue;
 
     // blob: the task counter (16 bytes), the sorted descriptors, the tasks;
@@ -1001,13 +1024,11 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const i
         int64_t pos[33];
         for (int c = 0; c < 33; ++c) pos[c] = off[c];
         for (int64_t i = 0; i < count; ++i) {
-            MulDesc q = descs[i];
-            if (is_plain(q)) {
-                q.logn = q.lg > q.lf ? 1 : 0;   // sweep the shorter operand
-                sorted[pos[0]++] = q;
-            } else {
-                sorted[pos[q.logn]++] = q;
-            }
+            const MulDesc &d = descs[i];
+            const int c = nl.of(d);
+            MulDesc &q = sorted[pos[c]++];
+            q = d;
+            q.logn = c ? c : (int)(d.lg > d.lf);   // schoolbook: sweep the shorter operand
         }
         // the tasks with their costs (butterflies; a schoolbook term costs
         // about an eighth of one), ordered by descending power-of-two cost
@@ -1081,16 +1102,10 @@ static hipError_t launch_list_persistent(const MulDesc *descs, int64_t count, co
                                          const u32 *G, u32 *H, const Family *fam, hipStream_t s) {
     if (count > INT32_MAX / 4) return hipErrorInvalidValue;
     // descriptor order: the schoolbook products, then the transform sizes
-    // ascending (class 0: schoolbook, class e: 2^e points)
-    int64_t ncls[33] = {0}, pieces = 0;
-    for (int64_t i = 0; i < count; ++i) {
-        const MulDesc &d = descs[i];
-        const int c = is_plain(d) ? 0 : d.logn;
-        ++ncls[c];
-        if (c == kBigLog) pieces += big_pieces<13>(d.lf + d.lg - 1);
-    }
-    const auto run = list_log(ncls, pieces) == 14 ? list_persistent_t<14> : list_persistent_t<13>;
-    return run(descs, count, ncls, pieces, F, G, H, fam, s);
+    // ascending
+    const ListCount n(descs, count);
+    const auto run = list_log(n) == 14 ? list_persistent_t<14> : list_persistent_t<13>;
+    return run(descs, count, n, F, G, H, fam, s);
 }
 
 }  // namespace cm
