@@ -3,7 +3,7 @@
 // The reference rebuilds its twiddle table W[j] = w^j on every call
 // (get_powers_binary, src/fft_aux.cu:87-132, one 4 KB host copy plus e-10
 // doubling launches) and cudaMallocs every temporary.  Here each root family
-// is built once per process, on the host, with Shoup companions, and kept in
+// is built once per process, on the host, in Montgomery form, and kept in
 // device memory; scratch space grows and is reused.
 #include <cstdio>
 #include <cstdlib>
@@ -40,15 +40,18 @@ u32 *upload(const std::vector<u32> &h) {
     return d;
 }
 
-// powers r^0 .. r^(cnt-1) in Montgomery form
-std::vector<u32> power_table(u32 r, size_t cnt, u32 p) {
-    std::vector<u32> t(cnt);
-    u64 x = cm_host_mont(1, p);
-    for (size_t j = 0; j < cnt; ++j) {
-        t[j] = (u32)x;
-        x = x * r % p;
+// r^0 .. r^(2^log - 1) in Montgomery form, by doubling: t[h + j] = r^h t[j], so no
+// entry waits for its neighbour.  The first 2^12-point product modulo a new prime
+// takes 0.24 ms with the tables built this way, 0.82 with chains of 64-bit
+// remainders; the first product of 2^22 points 1.20 against 2.75 ms.
+void power_table(u32 *t, u32 r, int log, u32 p) {
+    t[0] = cm_host_mont(1, p);
+    u32 w = r;   // r^h
+    for (size_t h = 1; h < (size_t)1 << log; h *= 2) {
+        const u32 wq = cm_host_shoup_q(w, p);
+        for (size_t j = 0; j < h; ++j) t[h + j] = cm_shoup(t[j], w, wq, p);
+        w = cm_host_mul(w, w, p);
     }
-    return t;
 }
 
 // One byte matrix of ntt_mx.h: output k of 16 adjacent elements is
@@ -59,23 +62,31 @@ std::vector<u32> power_table(u32 r, size_t cnt, u32 p) {
 void mx_matrix(int8_t *out, u32 w, int t, u32 scale, u32 p) {
     const int m = t ? 1 << t : 16;
     u32 *init = (u32 *)(out + 4 * 64 * 16);
-    const u32 f = cm_host_mul(scale, cm_host_r1(p), p);
+    // the 16 digits, byte 4 b + a, of the entries at exponents (d mod m)(k mod m)
+    u32 entry[226];
+    int8_t digits[226][16];
+    u32 e = cm_host_mul(scale, cm_host_r1(p), p);
+    for (int x = 0; x <= (m - 1) * (m - 1); ++x, e = cm_host_mul(e, w, p)) {
+        entry[x] = e;
+        u32 y = e;
+        for (int a = 0; a < 4; ++a, y = cm_host_mul(y, 256u, p)) {
+            int64_t v = y > p / 2 ? (int64_t)y - p : (int64_t)y;
+            for (int b = 0; b < 4; ++b) {
+                const int8_t digit = (int8_t)(v & 255);
+                v = (v - digit) / 256;
+                digits[x][4 * b + a] = digit;
+            }
+        }
+    }
     u32 sum[16];
     for (int k = 0; k < 16; ++k) {
         u64 acc = 0;
-        for (int d = 0; d < 16; ++d) {
-            const u32 e = d / m == k / m ? cm_host_mul(cm_host_pow(w, (u64)(d % m) * (k % m), p), f, p) : 0u;
-            acc += e;
-            for (int a = 0; a < 4; ++a) {
-                const u32 y = cm_host_mul(e, (u32)(((u64)1 << (8 * a)) % p), p);
-                int64_t v = y > p / 2 ? (int64_t)y - p : (int64_t)y;
-                for (int b = 0; b < 4; ++b) {
-                    const int8_t digit = (int8_t)(v & 255);
-                    v = (v - digit) / 256;
-                    // lane (output k, group d / 4), byte 4 (d mod 4) + a
-                    out[(b * 64 + (d / 4) * 16 + k) * 16 + 4 * (d % 4) + a] = digit;
-                }
-            }
+        for (int d = k / m * m; d < k / m * m + m; ++d) {
+            const int x = (d % m) * (k % m);
+            acc += entry[x];
+            // lane (output k, group d / 4), bytes 4 (d mod 4) .. + 3; other blocks stay 0
+            for (int b = 0; b < 4; ++b)
+                memcpy(out + (b * 64 + (d / 4) * 16 + k) * 16 + 4 * (d % 4), digits[x] + 4 * b, 4);
         }
         sum[k] = (u32)(acc % p);
     }
@@ -90,8 +101,9 @@ void mx_matrix(int8_t *out, u32 w, int t, u32 scale, u32 p) {
         }
 }
 
-// matrices and twiddles of the matrix-core transforms
-bool make_mx(Family *f) {
+// matrices and twiddles of the matrix-core transforms; pw[dir]: the powers of the
+// root of order 2^LT and of its inverse.  Every level's twiddles are among them.
+bool make_mx(Family *f, const std::vector<u32> *pw) {
     const u32 p = f->p;
     std::vector<u32> mats((size_t)kMxMats * kMxMatWords * 4, 0u);
     auto mat = [&](int which) { return (int8_t *)(mats.data() + (size_t)which * kMxMatWords * 4); };
@@ -110,18 +122,9 @@ bool make_mx(Family *f) {
     for (int dir = 0; dir < 2; ++dir) {
         std::vector<u32> tab((size_t)2 << f->LT, 0u);
         for (int j = 5; j <= f->LT; ++j) {
-            const size_t M = (size_t)1 << j, S = M / 16;
-            u32 w = cm_host_pow(f->wN, (u64)1 << (f->K - j), p);
-            if (dir) w = cm_host_inv(w, p);
-            u32 wk = 1;   // w^k
-            for (size_t k = 0; k < 16; ++k) {
-                u64 x = cm_host_mont(1, p);
-                for (size_t v = 0; v < S; ++v) {
-                    tab[M + k * S + v] = (u32)x;
-                    x = x * wk % p;
-                }
-                wk = cm_host_mul(wk, w, p);
-            }
+            const size_t M = (size_t)1 << j, S = M / 16, step = (size_t)1 << (f->LT - j);
+            for (size_t k = 0; k < 16; ++k)
+                for (size_t v = 0; v < S; ++v) tab[M + k * S + v] = pw[dir][k * v * step];
         }
         (dir ? f->mx_ti : f->mx_tf) = upload(tab);
     }
@@ -136,21 +139,24 @@ Family *make_family(u32 p, u32 wN, int K) {
     f->K = K;
     f->wN = wN;
     f->LT = K < kMaxLevelLog ? K : kMaxLevelLog;
-    // level tables: level M = 2^j (j = 1 .. LT) at offset 2^(j-1) - 1
-    std::vector<u32> lv, lvi;
-    for (int j = 1; j <= f->LT; ++j) {
-        u32 wm = cm_host_pow(wN, (u64)1 << (K - j), p);   // order 2^j
-        std::vector<u32> a = power_table(wm, (size_t)1 << (j - 1), p);
-        std::vector<u32> b = power_table(cm_host_inv(wm, p), (size_t)1 << (j - 1), p);
-        lv.insert(lv.end(), a.begin(), a.end());
-        lvi.insert(lvi.end(), b.begin(), b.end());
+    // level tables: level M = 2^j (j = 1 .. LT) at offset 2^(j-1) - 1, each a part of
+    // the largest level's powers
+    std::vector<u32> pw[2];
+    for (int dir = 0; dir < 2; ++dir) {
+        const u32 w = cm_host_pow(wN, (u64)1 << (K - f->LT), p);   // order 2^LT
+        pw[dir].resize((size_t)1 << f->LT);
+        power_table(pw[dir].data(), dir ? cm_host_inv(w, p) : w, f->LT, p);
+        std::vector<u32> lv;
+        lv.reserve((size_t)1 << f->LT);
+        for (int j = 1; j <= f->LT; ++j)
+            for (size_t q = 0; q < (size_t)1 << (j - 1); ++q)
+                lv.push_back(pw[dir][q << (f->LT - j)]);
+        if (lv.empty()) lv.push_back(cm_host_mont(1, p));
+        (dir ? f->lvi : f->lv) = upload(lv);
     }
-    if (lv.empty()) { lv.push_back(cm_host_mont(1, p)); lvi.push_back(cm_host_mont(1, p)); }
-    f->lv = upload(lv);
-    f->lvi = upload(lvi);
     f->mx_mat = nullptr;
     f->mx_tf = f->mx_ti = nullptr;
-    if (!f->lv || !f->lvi || (K >= 4 && !make_mx(f))) {
+    if (!f->lv || !f->lvi || (K >= 4 && !make_mx(f, pw))) {
         delete f;
         return nullptr;
     }
@@ -254,21 +260,14 @@ const Outer *outer_for_split(const Family *f, int k, int k1, int k2) {
     // row-pass tables
     const size_t n1 = (size_t)1 << k1, T = ((size_t)1 << k2) / 16;
     for (int dir = 0; dir < 2; ++dir) {
-        const u32 w = dir ? wni : wn;
+        const u32 w = dir ? wni : wn, wT = cm_host_pow(w, T, p);
         std::vector<u32> rb(n1 * T), rc(n1 * 16);
+        u32 wr = 1, wrT = 1;   // w^r, w^(r T)
         for (size_t r = 0; r < n1; ++r) {
-            const u32 wr = cm_host_pow(w, r, p);                 // w^k1
-            u64 x = cm_host_mont(1, p);
-            for (size_t t = 0; t < T; ++t) {
-                rb[r * T + t] = (u32)x;
-                x = x * wr % p;
-            }
-            const u32 wrT = cm_host_pow(wr, T, p);              // w^(k1 T)
-            x = cm_host_mont(1, p);
-            for (size_t m = 0; m < 16; ++m) {
-                rc[r * 16 + m] = (u32)x;
-                x = x * wrT % p;
-            }
+            power_table(&rb[r * T], wr, k2 - 4, p);
+            power_table(&rc[r * 16], wrT, 4, p);
+            wr = cm_host_mul(wr, w, p);
+            wrT = cm_host_mul(wrT, wT, p);
         }
         (dir ? o->rb_i : o->rb_f) = upload(rb);
         (dir ? o->rc_i : o->rc_f) = upload(rc);
