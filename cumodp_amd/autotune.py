@@ -1,6 +1,6 @@
 """Measured choice of the library's run-time tunables on the current GPU.
 
-There are four tunables:
+There are five tunables:
 
   * The four-step split of a 2^k-point transform (k > 13): rows of 2^k2
     words, with k2 in {12, 13, 14} or the library's own value of that size,

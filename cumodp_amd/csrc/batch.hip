@@ -4,14 +4,18 @@
 // (src/list_stockham.cu:595-630) transforms m rows of one length, and the
 // unbuilt draft src/.list_fft_poly_mul.cu:15-53 multiplies equal-length
 // pairs.  Here products are binned by transform size 2^e:
+//   * e <= 15, and every schoolbook product: one launch of tasks in LDS
+//     (k_list_persistent);
+//   * e >= 16: per size, the inputs are gathered into zero-padded slabs,
+//     multiplied by the batched four-step kernels and scattered back.
+// A tuned choice, the per-class form (g_list_persistent = false), takes instead
 //   * 2^e <= W (W = 2048, 4096 or 8192 words, a tuned choice): one fused
 //     launch for every such product.  Each workgroup takes a W-word tile
 //     holding W / 2^e products of one size and runs the whole multiply in
 //     LDS; the tile's size selects the code path at run time, so one launch
 //     covers all sizes;
 //   * 2^e <= 2^13 above W: one launch of the 8192-point workgroup multiply;
-//   * e >= 14: per size, the inputs are gathered into zero-padded slabs,
-//     multiplied by the batched four-step kernels and scattered back.
+//   * e >= 14: as above (many products of 2^14 points in LDS).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -171,7 +175,7 @@ __global__ void k_scatter(u32 *__restrict__ H, const u32 *__restrict__ slab, int
 //     256 outputs, each wave on its own, the arithmetic of k_plain_mul).
 // Bound by issue and the chains inside a wave: 59.9 M vector and 3.8 M matrix
 // instructions take 58% and 15% of the SIMDs' cycles with four waves on each,
-// and the CUs are busy 83% of the time.  4096 pairs of degrees 32 .. 16384: 197 us per
+// and the CUs are busy 83% of the time.  4096 pairs of degrees 32 .. 16384: 187 us per
 // call against 226 us with 1024 threads and 16384-word tiles, one workgroup per
 // CU, 2^15 points as two halves; a product of up to 12288 words as 8192 + 4096
 // points takes 5 us of that.  2^24 points in all of 2^13-point products take 96
@@ -661,9 +665,9 @@ int list_tile_words() { return kMixWordsOf[g_mix_variant]; }
 // the schoolbook kernel (plain.hip) in list multiplies: there the la * lb
 // products cost less than three transforms of 2^ceil(log2(la + lb - 1))
 // points.  0 sends everything to the NTT.  The tuner sets it.  Measured on
-// the 4096 uneven pairs: 32 in the one-launch form (its transform tasks run
-// at about two thirds of the VALU peak, its schoolbook tasks well below:
-// 0.29 ms per call against 0.34 ms at 256), 256 in the per-class form.
+// the 4096 uneven pairs: 32 in the one-launch form (0.204 ms per call with a wait
+// after each few, 0.207 at 0, 0.229 at 64 and 0.274 at 256), 256 in the
+// per-class form.
 int g_plain_cutoff = 32;
 
 bool set_list_plain_cutoff(int c) {

@@ -1,4 +1,5 @@
-// mul_mx.hip -- whole multiplies in one workgroup on the matrix cores.
+// mul_mx.hip -- multiplies on the matrix cores: whole products of up to 2^13 points
+// in one workgroup, and the column and row passes of the four-step ones above.
 #include <algorithm>
 
 #include "internal.h"
@@ -172,7 +173,7 @@ hipError_t launch_tree_level(int i, const u32 *prev, u32 *cur, int64_t nodes, co
 #define CM_CASE(K)                                                                        \
     case K:                                                                               \
         return mul_mx_t<K, kMonic>(prev, prev + (h + 1), cur, nullptr, (int)nodes, sd, fam, s);
-        CM_CASE(8) CM_CASE(9) CM_CASE(10) CM_CASE(11) CM_CASE(12) CM_CASE(13)
+        CM_CASE(9) CM_CASE(10) CM_CASE(11) CM_CASE(12) CM_CASE(13)
 #undef CM_CASE
     }
     // four-step straight from and into the tree, in chunks whose two slabs
@@ -330,13 +331,15 @@ __attribute__((amdgpu_waves_per_eu(4, 8))) void k_row_mx(u32 *F, const u32 *__re
     mx_row<LOGL, V>(lds, F + t0, G + tg, (int)(blockIdx.x << (LOGW - LOGL)), k1, o, cx);
 }
 
-// Tiles of 16384 words that run as one workgroup per CU, two to eight for each
-// (the inverse, of one array, half as many).  Back to back, 2^22, 2^23 and 2^24
-// points: 50.0, 94.0 and 197.1 us with a workgroup per tile, 47.5, 88.8 and 193.3
-// us so (of new operands, 204 and 189 us at 2^24: repeated calls lower the
-// clock); at 2^25, beyond the last-level cache, 466 us without it and 475 with.
+// Tiles of 16384 words that run as kLoopWgs workgroups, one per CU: two to eight
+// tiles for each, the inverse (of one array) two to four, so products of 2^22
+// points loop the forward pass only.  Back to back, 2^22, 2^23 and 2^24 points:
+// 53.1, 101.1 and 203.1 us on one pair of operands and 51.5, 106.0 and 213.3 on six
+// in turn with a workgroup per tile; 50.9, 95.2, 194.1 and 48.9, 97.9, 207.6 us so;
+// at 2^25, beyond the last-level cache, 466 us without it and 475 with.
 // Operands whose last quad of words is not whole take a workgroup per tile.
 constexpr int64_t kLoopMin = 512, kLoopMax = 2048;
+constexpr unsigned kLoopWgs = 256;   // CUs of the whole device; any number is correct
 
 template <int LOGL, int LOGC, int V>
 static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int cnt0, int cnt1,
@@ -350,11 +353,11 @@ static hipError_t cols_t(bool inverse, const MxCols &s0, const MxCols &s1, int c
         const bool whole = inverse || (s0.in_len % 4 == 0 && s1.in_len % 4 == 0);
         if (tiles >= kLoopMin && tiles <= (inverse ? kLoopMax / 2 : kLoopMax) && !edges && whole) {
             if (inverse)
-                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, true>), dim3(256), dim3(T), 0, s, s0, s1,
-                                   cnt0, (int)tiles, k2, cx);
+                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, true>), dim3(kLoopWgs), dim3(T), 0, s,
+                                   s0, s1, cnt0, (int)tiles, k2, cx);
             else
-                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, false>), dim3(256), dim3(T), 0, s, s0,
-                                   s1, cnt0, (int)tiles, k2, cx);
+                hipLaunchKernelGGL((k_cols_loop<LOGL, LOGC, false>), dim3(kLoopWgs), dim3(T), 0, s,
+                                   s0, s1, cnt0, (int)tiles, k2, cx);
             return hipGetLastError();
         }
     }

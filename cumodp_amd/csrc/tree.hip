@@ -11,8 +11,8 @@
 // Level i is one batch of products on 2^i points of the whole monic nodes of
 // level i-1 (leading 1 included): the product's x^(2^i) wraps onto its constant
 // term, which the store takes back while it writes the leading 1, so a level
-// is one launch up to 2^13 points and three above, with no pass that adds the
-// leading terms.  (The reference multiplies without the leading terms and adds
+// is one launch up to 2^12 points and three above (of 2^13 points three for 2 to
+// 32 nodes and one otherwise), with no pass that adds the leading terms.  (The reference multiplies without the leading terms and adds
 // x^h (a + b) afterwards, :601-650.)  Levels 0 .. 8 are built before that in
 // one launch, a 256-point subtree per workgroup (k_tree_bottom).
 #include "accum.h"

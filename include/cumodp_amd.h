@@ -62,11 +62,10 @@ CUMODP_API cumodp_err cumodp_fftmul_uni_dev_noalloc(sfixn dh, sfixn *Hd, sfixn d
  * One call multiplies `count` independent pairs mod p.  Item i reads
  * F[f_off .. f_off+df], G[g_off .. g_off+dg] and writes H[h_off ..
  * h_off+df+dg] (df+dg+1 words).  Output ranges must not overlap each other
- * or any input.  Products are binned by transform size; sizes up to 2^13 run
- * many products per workgroup in one launch per size class, larger ones as
- * batched four-step transforms.  Replaces a loop of stockham_poly_mul_dev
- * calls; the reference's list path (src/list_stockham.cu:595-630) only
- * transforms rows of one length. */
+ * or any input.  Products are binned by transform size; sizes up to 2^15 run
+ * in one launch, larger ones as batched four-step transforms per size.
+ * Replaces a loop of stockham_poly_mul_dev calls; the reference's list path
+ * (src/list_stockham.cu:595-630) only transforms rows of one length. */
 typedef struct {
     int64_t f_off, g_off, h_off;
     int32_t df, dg;
