@@ -914,29 +914,33 @@ static int cost_bucket(double x) {
     return b > 63 ? 63 : b;
 }
 
-// What the products of a list call are.  Their classes come in no order, so the
-// passes have no branch on them (20000 pairs of degrees 16 .. 300: 227 us per call
-// with three passes that do, 155 us so).
+// What the products of a list call are, in one pass over them: a pass of its own
+// for each figure mispredicts its branches again (20000 pairs of degrees 16 .. 300:
+// 227 us per call with three such passes, 156 us so).
 struct ListCount {
-    int64_t cls[33];              // products by class: 0 schoolbook, e 2^e points
-    int64_t plain = 0;            // small tasks of the schoolbook products
-    int64_t pieces = 0;           // small tasks of the 2^15-point products
-    int cut;                      // class 0: a side of at most cut words
+    int64_t cls[33] = {0};   // products by class: 0 schoolbook, e 2^e points
+    int64_t plain = 0;       // small tasks of the schoolbook products
+    int64_t pieces = 0;      // small tasks of the 2^15-point products
+    int cut;                 // class 0: a side of at most cut words
 
-    int of(const MulDesc &d) const { return std::min(d.lf, d.lg) <= cut ? 0 : d.logn; }
-    // a product's tasks of `words` words if it is of class c
-    int64_t tasks(const MulDesc &d, int c, int words) const {
-        return (uint32_t)(d.lh + words - 1) / (uint32_t)words & -(uint32_t)(of(d) == c);
+    bool is_plain(const MulDesc &d) const { return std::min(d.lf, d.lg) <= cut; }
+    static int64_t tasks(const MulDesc &d, int words) {
+        return (uint32_t)(d.lh + words - 1) / (uint32_t)words;
     }
     ListCount(const MulDesc *descs, int64_t count) : cut(g_plain_cutoff) {
-        uint32_t n[2][33] = {};   // neighbours count apart
+        int64_t pl = 0, pc = 0;
         for (int64_t i = 0; i < count; ++i) {
-            ++n[i & 1][of(descs[i])];
-            plain += tasks(descs[i], 0, ListGeo<13>::PlainOut);
+            const MulDesc &d = descs[i];
+            if (is_plain(d)) {
+                ++cls[0];
+                pl += tasks(d, ListGeo<13>::PlainOut);
+            } else {
+                ++cls[d.logn];
+                pc += tasks(d, ListGeo<13>::W) & -(int64_t)(d.logn == kBigLog);
+            }
         }
-        for (int c = 0; c < 33; ++c) cls[c] = (int64_t)n[0][c] + n[1][c];
-        for (int64_t i = 0; cls[kBigLog] && i < count; ++i)
-            pieces += tasks(descs[i], kBigLog, ListGeo<13>::W);
+        plain = pl;
+        pieces = pc;
     }
 };
 
@@ -988,7 +992,7 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const L
     for (int e = LOG + 1; e <= kBigLog; ++e) nbig += ncls[e];
     ntasks += nbig + (LOG == 13 ? nl.plain : 0);
     for (int64_t i = 0; LOG == 14 && ncls[0] && i < count; ++i)
-        ntasks += nl.tasks(descs[i], 0, Geo::PlainOut);
+        if (nl.is_plain(descs[i])) ntasks += nl.tasks(descs[i], Geo::PlainOut);
     // Small tasks: below four per CU (two rounds of workgroups), or with products of
     // 2^15 points below 3 1/2 rounds of pieces, a whole product would leave the
     // chip waiting at the end, so every piece is a task, at the price of a
@@ -1017,7 +1021,8 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const L
     // written straight into the pinned staging buffer
     const size_t desc_off = 16;
     const size_t task_off = desc_off + sizeof(MulDesc) * (size_t)count;
-    const size_t bytes = task_off + sizeof(ListTask) * (size_t)ntasks;
+    // whole 16-byte words, or the copy takes about 1 us longer
+    const size_t bytes = (task_off + sizeof(ListTask) * (size_t)ntasks + 15) & ~(size_t)15;
     std::vector<MulDesc> tail;   // host copy of the four-step classes' descriptors
     char *dblob = (char *)workspace(7, bytes, s);
     if (!dblob) return hipErrorOutOfMemory;
@@ -1028,11 +1033,13 @@ static hipError_t list_persistent_t(const MulDesc *descs, int64_t count, const L
         int64_t pos[33];
         for (int c = 0; c < 33; ++c) pos[c] = off[c];
         for (int64_t i = 0; i < count; ++i) {
-            const MulDesc &d = descs[i];
-            const int c = nl.of(d);
-            MulDesc &q = sorted[pos[c]++];
-            q = d;
-            q.logn = c ? c : (int)(d.lg > d.lf);   // schoolbook: sweep the shorter operand
+            MulDesc q = descs[i];
+            if (nl.is_plain(q)) {
+                q.logn = q.lg > q.lf ? 1 : 0;   // sweep the shorter operand
+                sorted[pos[0]++] = q;
+            } else {
+                sorted[pos[q.logn]++] = q;
+            }
         }
         // the tasks with their costs (butterflies; a schoolbook term costs
         // about an eighth of one), ordered by descending power-of-two cost
